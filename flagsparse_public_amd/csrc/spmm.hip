@@ -2,13 +2,22 @@
 //
 // A group of G lanes owns one row and a tile of G*VW dense columns; each lane
 // owns VW consecutive columns and gathers them from the B row of every entry
-// with one vector load (VW * element size bytes, e.g. 16 B for fp32 x4), so a
-// group reads one contiguous B-row segment per entry.  U entries are kept in
+// with one vector load (16 bytes: fp32 x4, fp64 x2, 16-bit x8, complex64 x2), so
+// a group reads one contiguous B-row segment per entry.  U entries are kept in
 // flight per lane.  Rows longer than short_max are cut into chunks reduced by
 // whole wavefronts (64/G groups interleave over the chunk's entries and are
 // combined with xor exchanges); a row spanning several chunks stores one
 // partial row per chunk, and spmm_fixup_kernel (a second, small launch) sums
 // them in chunk order.
+//
+// Bound (B beyond L2): the 128-byte lines of the gathered B rows, which the
+// Infinity Cache delivers at about 7 TB/s whatever the element type: 250,000
+// rows with 5M random entries take 181 us for 256-byte B rows both in bf16
+// (N = 128) and fp32 (N = 64).  16-bit values were bound by the lane instead:
+// one 2-byte element per lane and load, one row per wavefront, 374 us for
+// bf16 N = 128, 190 us for N = 64 (now 97 us); odd widths by scalar loads:
+// fp32 N = 33 191 -> 167 us, bf16 N = 47 194 -> 138 us (a 94-byte row touches
+// 1.7 lines on average).
 //
 // Replaces the reference's ALG1 row x column-tile kernel (spmm_csr.py:92-134,
 // 525-599) and the bucketed opt / alg2 kernels (spmm_csr.py:602-919,
@@ -80,96 +89,141 @@ template <int G, typename A> __device__ __forceinline__ void cross_group_reduce(
   if constexpr (G <= 32) { A o = xor_x<32>(a); a.merge(o); }
 }
 
+// VW consecutive stored values of type V as loaded: 32-bit words (one 16-bit
+// value in the low half for a single 2-byte element).  The vector types carry
+// only the element's own alignment, so a lane's segment may start at any
+// element of B or C (odd leading dimensions, offset bases, the shifted tail
+// window below); gfx950 serves a misaligned global dwordx4 in hardware and the
+// compiler emits the same instruction as for an aligned one.
+template <typename V, int VW> struct RawVec {
+  static constexpr int kBytes = (int)sizeof(V) * VW;
+  static constexpr int kWords = kBytes < 4 ? 1 : kBytes / 4;
+  uint32_t w[kWords];
+};
+// alignment of a vector access: the stored element's scalar
+template <typename V> constexpr int kElemAlign = alignof(V) < sizeof(V) ? (int)alignof(V) : (int)sizeof(V);
+
+template <int W, int AL> struct WordVec;
+template <> struct WordVec<1, 2> { typedef uint32_t type __attribute__((aligned(2))); };
+template <> struct WordVec<2, 2> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(2))); };
+template <> struct WordVec<4, 2> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); };
+template <> struct WordVec<1, 4> { typedef uint32_t type __attribute__((aligned(4))); };
+template <> struct WordVec<2, 4> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct WordVec<4, 4> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct WordVec<2, 8> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct WordVec<4, 8> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(8))); };
+
+template <typename V, int VW>
+__device__ __forceinline__ void load_raw(RawVec<V, VW>& r, const V* __restrict__ p, int64_t off) {
+  using R = RawVec<V, VW>;
+  if constexpr (R::kBytes < 4) {
+    r.w[0] = *reinterpret_cast<const uint16_t*>(p + off);
+  } else {
+    using T = typename WordVec<R::kWords, kElemAlign<V>>::type;
+    const T v = *reinterpret_cast<const T*>(p + off);
+    __builtin_memcpy(r.w, &v, R::kBytes);
+  }
+}
+
+template <typename V, int VW, typename C>
+__device__ __forceinline__ void unpack_raw(C (&out)[VW], const RawVec<V, VW>& r) {
+  V v[VW];
+  __builtin_memcpy(v, r.w, sizeof(V) * VW);
+#pragma unroll
+  for (int k = 0; k < VW; ++k) out[k] = load_as<C>(v, k);
+}
+
 // Load VW consecutive stored values starting at element `off` as compute type.
 template <typename C, int VW, typename S>
 __device__ __forceinline__ void load_vec(C (&out)[VW], const S* __restrict__ p, int64_t off) {
-  if constexpr (std::is_same<S, float>::value && VW == 4) {
-    const float4 v = *reinterpret_cast<const float4*>(p + off);
-    out[0] = (C)v.x; out[1] = (C)v.y; out[2] = (C)v.z; out[3] = (C)v.w;
-  } else if constexpr (std::is_same<S, float>::value && VW == 2) {
-    const float2 v = *reinterpret_cast<const float2*>(p + off);
-    out[0] = (C)v.x; out[1] = (C)v.y;
-  } else if constexpr (std::is_same<S, double>::value && VW == 2) {
-    const double2 v = *reinterpret_cast<const double2*>(p + off);
-    out[0] = (C)v.x; out[1] = (C)v.y;
-  } else {
+  RawVec<S, VW> r;
+  load_raw(r, p, off);
+  unpack_raw(out, r);
+}
+
+// B rows of a masked batch, raw: r[u] = B[col[u] * ldb + n0 .. + VW) for the u
+// whose bit is set in `ok` (others zero).
+template <int VW, int U, typename V>
+__device__ __forceinline__ void gather_masked(RawVec<V, VW> (&r)[U], const V* __restrict__ B,
+                                              int64_t ldb, const int64_t (&col)[U], int64_t n0,
+                                              unsigned ok) {
 #pragma unroll
-    for (int k = 0; k < VW; ++k) out[k] = load_as<C>(p, off + k);
+  for (int u = 0; u < U; ++u) {
+    if ((ok >> u) & 1u) {
+      load_raw(r[u], B, col[u] * ldb + n0);
+    } else {
+#pragma unroll
+      for (int w = 0; w < RawVec<V, VW>::kWords; ++w) r[u].w[w] = 0u;
+    }
   }
 }
 
-// B rows of a masked batch: b[u] = B[col[u] * ldb + n0 .. + VW) for the u
-// whose bit is set in `ok` (others zero).  When the compute type differs from
-// the stored one (fp32 B accumulated in fp64), the rows are loaded raw and kept
-// opaque (empty asm) until every load of the batch is issued, then widened: a
-// widening placed inside a masked load's branch brings a wait for that load
-// with it and serialises the batch.
-template <int VW, int U, typename C, typename V>
-__device__ __forceinline__ void gather_masked(C (&b)[U][VW], const V* __restrict__ B, int64_t ldb,
-                                              const int64_t (&col)[U], int64_t n0, unsigned ok) {
-  if constexpr (std::is_same<C, V>::value || !std::is_arithmetic<V>::value) {
+// Widening of a gathered row.  When the compute type differs from the stored
+// one (fp32 B accumulated in fp64, 16-bit values, complex), the words stay
+// opaque (empty asm) until every load of the batch is issued: a widening placed
+// inside a masked load's branch brings a wait for that load with it and
+// serialises the batch.
+template <typename V, int VW, typename C>
+__device__ __forceinline__ void widen_row(C (&b)[VW], RawVec<V, VW>& r) {
+  if constexpr (!std::is_same<C, V>::value) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if ((ok >> u) & 1u) {
-        load_vec<C, VW>(b[u], B, col[u] * ldb + n0);
-      } else {
-#pragma unroll
-        for (int k = 0; k < VW; ++k) b[u][k] = zero<C>();
-      }
-    }
-  } else {
-    V r[U][VW];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if ((ok >> u) & 1u) {
-        load_vec<V, VW>(r[u], B, col[u] * ldb + n0);
-      } else {
-#pragma unroll
-        for (int k = 0; k < VW; ++k) r[u][k] = V(0);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int k = 0; k < VW; ++k) {
-        asm volatile("" : "+v"(r[u][k]));
-        b[u][k] = (C)r[u][k];
-      }
+    for (int w = 0; w < RawVec<V, VW>::kWords; ++w) asm volatile("" : "+v"(r.w[w]));
   }
+  unpack_raw(b, r);
 }
 
-// C[off .. off + VW) = alpha * acc + beta * C (C read only when beta is
-// nonzero): write_out's arithmetic, with one vector load / store where
-// load_vec has a vector form (the launch keeps C aligned whenever VW > 1) and
-// the row's lane group is at least 32 lanes wide.  Measured on the 1M-row
-// banded matrix: vector stores took N = 128 (32 lanes) from 798 to 776 us,
-// but were ~2 us slower than VW scalar stores at N = 32 / 64 (8 / 16 lanes).
+// The lane's column window: columns n0 .. n0 + VW - 1 of which the last
+// VW - skip are its own.  A row's last lane shifts its window back so that it
+// ends at the last column (n_dense >= VW always holds): every load stays
+// inside the row with no scalar tail, and the columns it shares with the lane
+// before are computed but not written.
+template <int VW>
+__device__ __forceinline__ int shift_tail(int64_t& n0, int64_t n_dense) {
+  if constexpr (VW > 1) {
+    if (n0 < n_dense && n0 + VW > n_dense) {
+      const int skip = (int)(n0 + VW - n_dense);
+      n0 = n_dense - VW;
+      return skip;
+    }
+  }
+  return 0;
+}
+
+// C[off + skip .. off + VW) = alpha * acc + beta * C (C read only when beta is
+// nonzero): write_out's arithmetic.  One vector store where the window is
+// whole and the values are 16-bit, or the row's lane group is at least 32
+// lanes wide.  Measured on the 1M-row banded matrix in fp32: vector stores
+// took N = 128 (32 lanes) from 798 to 776 us, but were ~2 us slower than VW
+// scalar stores at N = 32 / 64 (8 / 16 lanes).
 template <int G, int VW, typename V, typename A>
 __device__ __forceinline__ void write_vec(V* __restrict__ C, int64_t off, const A (&acc)[VW],
-                                          double alpha, double beta) {
-  constexpr bool kVec = G >= 32 && ((std::is_same<V, float>::value && (VW == 4 || VW == 2)) ||
-                                    (std::is_same<V, double>::value && VW == 2));
+                                          double alpha, double beta, int skip) {
+  using T = std::decay_t<decltype(acc[0].value())>;
+  constexpr bool kVec = VW > 1 && (G >= 32 || sizeof(V) == 2);
   if constexpr (kVec) {
-    using T = std::decay_t<decltype(acc[0].value())>;
-    T v[VW];
+    if (skip == 0) {
+      T v[VW];
 #pragma unroll
-    for (int k = 0; k < VW; ++k) v[k] = alpha == 1.0 ? acc[k].value() : scale(acc[k].value(), alpha);
-    if (beta != 0.0) {
-      T old[VW];
-      load_vec<T, VW>(old, C, off);
+      for (int k = 0; k < VW; ++k) v[k] = alpha == 1.0 ? acc[k].value() : scale(acc[k].value(), alpha);
+      if (beta != 0.0) {
+        T old[VW];
+        load_vec<T, VW>(old, C, off);
 #pragma unroll
-      for (int k = 0; k < VW; ++k) v[k] = add(v[k], scale(old[k], beta));
+        for (int k = 0; k < VW; ++k) v[k] = add(v[k], scale(old[k], beta));
+      }
+      V o[VW];
+#pragma unroll
+      for (int k = 0; k < VW; ++k) store_from(o, k, v[k]);
+      using W = typename WordVec<RawVec<V, VW>::kWords, kElemAlign<V>>::type;
+      W w;
+      __builtin_memcpy(&w, o, sizeof(V) * VW);
+      *reinterpret_cast<W*>(C + off) = w;
+      return;
     }
-    if constexpr (std::is_same<V, float>::value && VW == 4)
-      *reinterpret_cast<float4*>(C + off) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
-    else if constexpr (std::is_same<V, float>::value)
-      *reinterpret_cast<float2*>(C + off) = make_float2((float)v[0], (float)v[1]);
-    else
-      *reinterpret_cast<double2*>(C + off) = make_double2((double)v[0], (double)v[1]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < VW; ++k) write_out(C, off + k, acc[k].value(), alpha, beta);
   }
+#pragma unroll
+  for (int k = 0; k < VW; ++k)
+    if (k >= skip) write_out(C, off + k, acc[k].value(), alpha, beta);
 }
 
 // Accumulate entries j = s + first, s + first + step, ... < e into acc[VW] for
@@ -189,13 +243,16 @@ __device__ __forceinline__ void mm_accumulate(A (&acc)[VW], const I* __restrict_
       col[u] = ldg_index(idx, j + u * step);
       a[u] = load_as<C>(val, j + u * step);
     }
-    C b[U][VW];
+    RawVec<V, VW> r[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) load_vec<C, VW>(b[u], B, col[u] * ldb + n0);
+    for (int u = 0; u < U; ++u) load_raw(r[u], B, col[u] * ldb + n0);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      C b[VW];
+      unpack_raw(b, r[u]);
 #pragma unroll
-      for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[u][k]);
+      for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[k]);
+    }
   }
   if (j < e) {
     // the last, partial batch: all its loads in flight at once, entries past
@@ -219,13 +276,16 @@ __device__ __forceinline__ void mm_accumulate(A (&acc)[VW], const I* __restrict_
       col[u] = (int64_t)ci[u];
       ok |= (unsigned)(j + u * step < e) << u;
     }
-    C b[U][VW];
-    gather_masked<VW, U>(b, B, ldb, col, n0, ok);
+    RawVec<V, VW> r[U];
+    gather_masked(r, B, ldb, col, n0, ok);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      C b[VW];
+      widen_row(b, r[u]);
       if (j + u * step < e)
 #pragma unroll
-        for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[u][k]);
+        for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[k]);
+    }
   }
 }
 
@@ -270,7 +330,7 @@ __device__ __forceinline__ void mm_accumulate_group(A (&acc)[VW], int32_t* slot_
 #pragma unroll
       for (int f = 0; f < F; ++f) {
         slot_col[f * G + g] = fc[f];
-        slot_val[f * G + g] = (C)fv[f];
+        slot_val[f * G + g] = load_as<C>(fv, f);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -292,13 +352,16 @@ __device__ __forceinline__ void mm_accumulate_group(A (&acc)[VW], int32_t* slot_
         unsigned ok = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) ok |= (unsigned)(u0 + u < cnt) << u;
-        C b[U][VW];
-        gather_masked<VW, U>(b, B, ldb, col, n0, ok);
+        RawVec<V, VW> r[U];
+        gather_masked(r, B, ldb, col, n0, ok);
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          C b[VW];
+          widen_row(b, r[u]);
           if (u0 + u < cnt)
 #pragma unroll
-            for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[u][k]);
+            for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[k]);
+        }
       }
     }
     // the slots are rewritten by the next batch
@@ -317,8 +380,9 @@ __device__ __forceinline__ void spmm_chunk_role(const SpmmParams<V, I, P>& p, in
   const int64_t c = item / p.n_tiles, tile = item % p.n_tiles;
   if (c >= p.n_chunks) return;
   const int grp = lane / G, g = lane % G;
-  const int64_t n0 = tile * (G * VW) + (int64_t)g * VW;
+  int64_t n0 = tile * (G * VW) + (int64_t)g * VW;
   const bool colok = n0 < p.n_dense;
+  const int skip = shift_tail<VW>(n0, p.n_dense);
   const int64_t li = p.chunk_long[c];
   const int64_t row = p.long_rows[li];
   const int64_t c0 = p.long_chunk_ptr[li];
@@ -333,13 +397,14 @@ __device__ __forceinline__ void spmm_chunk_role(const SpmmParams<V, I, P>& p, in
 #pragma unroll
   for (int k = 0; k < VW; ++k) cross_group_reduce<G>(acc[k]);
   if (nc == 1) {
-    if (grp == 0 && colok) write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta);
+    if (grp == 0 && colok) write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta, skip);
     return;
   }
   CA* parts = reinterpret_cast<CA*>(p.partials);  // summed by spmm_fixup_kernel
   if (grp == 0 && colok)
 #pragma unroll
-    for (int k = 0; k < VW; ++k) parts[c * p.n_dense + n0 + k] = acc[k];
+    for (int k = 0; k < VW; ++k)
+      if (k >= skip) parts[c * p.n_dense + n0 + k] = acc[k];
 }
 
 // Second pass for rows cut into several chunks: one wavefront per long row;
@@ -367,10 +432,15 @@ template <typename V, typename I>
 constexpr bool kHotSpmm = (std::is_same<V, float>::value || std::is_same<V, double>::value) &&
                           std::is_same<I, int32_t>::value;
 
-// Short rows load their entries group-cooperatively for the fp32 / fp64,
-// int32-column kernels whose lane groups hold whole batches.
+// Short rows load their entries group-cooperatively in the int32-column
+// kernels whose lane groups hold whole batches.
 template <typename V, typename I, int G, int U>
-constexpr bool kGroupLoads = kHotSpmm<V, I> && G >= U && G % U == 0;
+constexpr bool kGroupLoads = std::is_same<I, int32_t>::value && G >= U && G % U == 0;
+
+// Widest lane segment: 16 bytes (int64-column kernels: one column per lane).
+template <typename V, typename I>
+constexpr int kMaxVw = !std::is_same<I, int32_t>::value ? 1
+                       : sizeof(V) == 2 ? 8 : sizeof(V) == 4 ? 4 : sizeof(V) == 8 ? 2 : 1;
 
 // Lane groups narrower than a batch (G < U: few dense columns) take the
 // wavefront's 64 / G consecutive rows together: their entries are
@@ -392,7 +462,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 template <typename A, int G, int VW, int U, typename V, typename I, typename P>
 __device__ __forceinline__ void spmm_staged_rows(const SpmmParams<V, I, P>& p, int64_t rb,
-                                                 int64_t row, int64_t n0) {
+                                                 int64_t row, int64_t n0, int skip) {
   using C = typename A::compute_t;
   __shared__ int32_t st_col[kMmWaves][kMmStage];
   __shared__ C st_val[kMmWaves][kMmStage];
@@ -465,20 +535,23 @@ __device__ __forceinline__ void spmm_staged_rows(const SpmmParams<V, I, P>& p, i
           unsigned ok = 0;
 #pragma unroll
           for (int u = 0; u < U; ++u) ok |= (unsigned)(j + u < hi) << u;
-          C b[U][VW];
-          gather_masked<VW, U>(b, p.B, p.ldb, col, n0, ok);
+          RawVec<V, VW> r[U];
+          gather_masked(r, p.B, p.ldb, col, n0, ok);
 #pragma unroll
-          for (int u = 0; u < U; ++u)
+          for (int u = 0; u < U; ++u) {
+            C b[VW];
+            widen_row(b, r[u]);
             if (j + u < hi)
 #pragma unroll
-              for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[u][k]);
+              for (int k = 0; k < VW; ++k) acc[k].add_prod(a[u], b[k]);
+          }
         }
       }
       wave_lds_sync();  // the window is rewritten next
     }
     if (!mine) return;
   }
-  write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta);
+  write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta, skip);
 }
 
 template <typename V, typename A, typename I, typename P, int G, int VW, int U>
@@ -493,9 +566,10 @@ __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> 
   const int64_t tile = sb % p.n_tiles, rb = sb / p.n_tiles;
   const int64_t row = rb * (kMmBlock / G) + threadIdx.x / G;
   const int g = threadIdx.x % G;
-  const int64_t n0 = tile * (G * VW) + (int64_t)g * VW;
+  int64_t n0 = tile * (G * VW) + (int64_t)g * VW;
+  const int skip = shift_tail<VW>(n0, p.n_dense);
   if constexpr (kWaveStaged<V, I, G, U>) {
-    spmm_staged_rows<A, G, VW, U>(p, rb, row, n0);
+    spmm_staged_rows<A, G, VW, U>(p, rb, row, n0, skip);
     return;
   }
   if (row >= p.n_rows) return;  // the whole group
@@ -518,7 +592,7 @@ __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> 
     if (n0 >= p.n_dense) return;  // lanes past the last column own nothing
     mm_accumulate<VW, U>(acc, p.idx, p.val, p.B, p.ldb, n0, rs, re, 1);
   }
-  write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta);
+  write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta, skip);
 }
 
 template <typename V, typename A, typename I, typename P, int G, int VW>
@@ -570,58 +644,83 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
   return check_launch("fs_spmm_csr");
 }
 
-template <typename V, typename A, typename I, typename P, int VW>
-int launch_spmm_g(int G, const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ldc,
-                  int64_t n_dense, double alpha, double beta, const fs_plan* pl, hipStream_t st) {
-  if constexpr (kHotSpmm<V, I>) {
-    switch (G) {
-      case 1: return launch_spmm_gv<V, A, I, P, 1, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      case 2: return launch_spmm_gv<V, A, I, P, 2, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      case 4: return launch_spmm_gv<V, A, I, P, 4, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      case 8: return launch_spmm_gv<V, A, I, P, 8, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      case 16: return launch_spmm_gv<V, A, I, P, 16, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      case 32: return launch_spmm_gv<V, A, I, P, 32, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-      default: return launch_spmm_gv<V, A, I, P, 64, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-    }
-  } else {
-    if (G <= 4) return launch_spmm_gv<V, A, I, P, 4, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-    if (G <= 16) return launch_spmm_gv<V, A, I, P, 16, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-    return launch_spmm_gv<V, A, I, P, 64, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-  }
-}
-
 static inline int pow2_at_least(int64_t v) {
   int g = 1;
   while (g < v && g < 64) g <<= 1;
   return g;
 }
 
+// Lane groups built per vector width (spmm_tile_shape picks no others): the
+// widest takes 8 to 64 lanes, narrower ones serve B with too few columns for
+// eight lanes of the next width, hence at most 16 lanes.
+template <typename V, typename A, typename I, typename P, int VW>
+int launch_spmm_g(int G, const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ldc,
+                  int64_t n_dense, double alpha, double beta, const fs_plan* pl, hipStream_t st) {
+  constexpr int kMax = kMaxVw<V, I>;
+  if constexpr (VW == 1) {
+    if constexpr (kHotSpmm<V, I>) {
+      if (G == 1) return launch_spmm_gv<V, A, I, P, 1, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+      if (G == 2) return launch_spmm_gv<V, A, I, P, 2, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+    }
+    if (G <= 4) return launch_spmm_gv<V, A, I, P, 4, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  }
+  if constexpr (std::is_same<I, int32_t>::value) {
+    if (G <= 8) return launch_spmm_gv<V, A, I, P, 8, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  }
+  if constexpr (VW < kMax) {
+    return launch_spmm_gv<V, A, I, P, 16, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  } else {
+    if (G <= 16) return launch_spmm_gv<V, A, I, P, 16, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+    if constexpr (std::is_same<I, int32_t>::value) {
+      if (G <= 32) return launch_spmm_gv<V, A, I, P, 32, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+    }
+    return launch_spmm_gv<V, A, I, P, 64, VW>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  }
+}
+
+// Columns per lane and lanes per row for n_dense columns in tiles of col_tile
+// (0: all).  The lane segment is the widest up to 16 bytes that leaves at
+// least eight lanes to a row, so that a row's entries are loaded a whole
+// batch at a time by its group; neither the alignment of B and C nor the
+// divisibility of n_dense narrows it (load_raw, shift_tail).
+template <int MAXV>
+static inline void spmm_tile_shape(int64_t n_dense, int64_t col_tile, int* vw, int* lanes) {
+  // a column tile wider than B would leave the lanes past n_dense idle
+  const int64_t tile = col_tile > 0 && col_tile < n_dense ? col_tile : n_dense;
+  int v = MAXV;
+  while (v > 1 && tile / v < 8) v >>= 1;
+  *vw = v;
+  *lanes = pow2_at_least((tile + v - 1) / v);
+}
+
 template <typename V, typename A, typename I, typename P>
 int launch_spmm(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ldc, int64_t n_dense,
                 double alpha, double beta, const fs_plan* pl, int32_t col_tile, hipStream_t st) {
-  // Vector width: the widest of {4, 2, 1} (fp64: {2, 1}; others: 1) that
-  // divides n_dense and both leading dimensions and keeps B / C aligned.
-  int vw = 1;
-  if constexpr (kHotSpmm<V, I>) {
-    const int maxv = std::is_same<V, float>::value ? 4 : 2;
-    for (int v = maxv; v >= 2; v >>= 1) {
-      const uintptr_t al = (uintptr_t)(v * sizeof(V));
-      if (n_dense % v == 0 && ldb % v == 0 && ldc % v == 0 && ((uintptr_t)B % al) == 0 &&
-          ((uintptr_t)C % al) == 0) {
-        vw = v;
-        break;
-      }
-    }
-  }
-  // a column tile wider than B would leave the lanes past n_dense idle
-  int64_t tile = col_tile > 0 && col_tile < n_dense ? col_tile : n_dense;
-  if (tile % vw != 0) vw = 1;
-  // narrow tiles keep at least 8 lanes per row (narrower loads, more lanes),
-  // so a row's entries are loaded a whole batch at a time by its group
-  while (vw > 1 && tile / vw < 8) vw >>= 1;
-  int G = pow2_at_least((tile + vw - 1) / vw);
-  if (vw == 4) return launch_spmm_g<V, A, I, P, 4>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
-  if (vw == 2) return launch_spmm_g<V, A, I, P, 2>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  constexpr int kMax = kMaxVw<V, I>;
+  // fp64, B rows of 1 KB and more: tiles of 512 bytes unless the last would be
+  // mostly idle.  Tiles of one row go to neighbouring blocks, so with two
+  // tiles each XCD (round-robin by block) gathers only its half of every B
+  // row: N = 128, 250,000 rows of 20 random entries 742 -> 715 us, banded
+  // 200,000 rows 319 -> 292 us; N = 100 (a 36-column last tile) 251 -> 279 us.
+  // fp32 rows of 1 KB gain on random columns (730 -> 703 us) but lose on a
+  // 1M-row band (1744 -> 1820 us).
+  if (std::is_same<V, double>::value && kMax > 1 && col_tile == 0 && n_dense >= 128 &&
+      (n_dense % 64 == 0 || n_dense % 64 >= 32))
+    col_tile = 64;
+  // complex64 rows of 1 KB and more keep one 512-byte tile per wavefront, one
+  // column per lane (100,000 rows of 20 random entries, N = 128 / 192: 275 /
+  // 426 us against 280 / 457 with two columns per lane)
+  if constexpr (std::is_same<V, c64_t>::value && kMax > 1)
+    if (col_tile == 0 && n_dense >= 128)
+      return launch_spmm_gv<V, A, I, P, 64, 1>(M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  int vw, G;
+  spmm_tile_shape<kMax>(n_dense, col_tile, &vw, &G);
+  if constexpr (kMax >= 8)
+    if (vw == 8) return launch_spmm_g<V, A, I, P, 8>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  if constexpr (kMax >= 4)
+    if (vw == 4) return launch_spmm_g<V, A, I, P, 4>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
+  if constexpr (kMax >= 2)
+    if (vw == 2) return launch_spmm_g<V, A, I, P, 2>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
   return launch_spmm_g<V, A, I, P, 1>(G, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
 }
 
