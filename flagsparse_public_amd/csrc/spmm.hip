@@ -407,24 +407,90 @@ __device__ __forceinline__ void spmm_chunk_role(const SpmmParams<V, I, P>& p, in
       if (k >= skip) parts[c * p.n_dense + n0 + k] = acc[k];
 }
 
-// Second pass for rows cut into several chunks: one wavefront per long row;
-// lane n sums column n's chunk partials in chunk order (then n + 64, ...).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Adds the partials of the kU chunks from k on at column n, all loads in flight.
+template <int kU, typename CA>
+__device__ __forceinline__ void fixup_batch(CA& tot, const CA* __restrict__ parts, int64_t n_dense,
+                                            int64_t n, int64_t k) {
+  CA q[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) q[u] = parts[(k + u) * n_dense + n];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) tot.merge(q[u]);
+}
+
+// Sum of the partials of chunks [k0, k1) at column n, in chunk order.
+template <typename CA>
+__device__ __forceinline__ CA fixup_sum(const CA* __restrict__ parts, int64_t n_dense, int64_t n,
+                                        int64_t k0, int64_t k1) {
+  CA tot;
+  tot.init();
+  int64_t k = k0;
+  for (; k + 8 <= k1; k += 8) fixup_batch<8>(tot, parts, n_dense, n, k);
+  for (; k + 2 <= k1; k += 2) fixup_batch<2>(tot, parts, n_dense, n, k);
+  if (k < k1) fixup_batch<1>(tot, parts, n_dense, n, k);
+  return tot;
+}
+
+// Second pass for rows cut into several chunks.  Lanes take `cols` columns
+// (a power of two, at most a wavefront) times 64 / cols ways, each way a
+// contiguous range of the row's chunks; the ways' sums meet in LDS and are
+// added in order.  A row of up to kFixWave chunks per way belongs to one
+// wavefront; a longer one is summed by the block's four.  Bound by the
+// latency of the longest row's chain of partial loads: one wavefront per row
+// with one load at a time took 73 us where power-law rows of up to 100,000
+// entries leave 391 chunks (N = 47, fp64 sums), this form 10 us; with two
+// chunks in every row (20,000 rows of about 300 entries, N = 64) SpMM and
+// fix-up take 137 us in both forms.
+constexpr int kFixWave = 16;
+
 template <typename A, typename V, typename I, typename P>
-__global__ __launch_bounds__(kMmBlock) void spmm_fixup_kernel(SpmmParams<V, I, P> p, int64_t n_long) {
+__global__ __launch_bounds__(kMmBlock) void spmm_fixup_kernel(SpmmParams<V, I, P> p, int64_t n_long,
+                                                              int col_shift) {
   using CA = typename MmChunkAcc<A>::T;
-  const int lane = threadIdx.x % kWave;
-  const int64_t li = (int64_t)blockIdx.x * kMmWaves + threadIdx.x / kWave;
-  if (li >= n_long) return;
-  const int64_t c0 = p.long_chunk_ptr[li];
-  const int64_t nc = p.long_chunk_ptr[li + 1] - c0;
-  if (nc <= 1) return;
-  const int64_t row = p.long_rows[li];
+  __shared__ CA part[kMmBlock];
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  const int cols = 1 << col_shift, ways = kWave >> col_shift;
+  const int c = lane & (cols - 1), way = lane >> col_shift;
   const CA* parts = reinterpret_cast<const CA*>(p.partials);
-  for (int64_t n = lane; n < p.n_dense; n += kWave) {
-    CA tot;
-    tot.init();
-    for (int64_t k = 0; k < nc; ++k) tot.merge(parts[(c0 + k) * p.n_dense + n]);
-    write_out(p.C, row * p.ldc + n, tot.value(), p.alpha, p.beta);
+  const int64_t l0 = (int64_t)blockIdx.x * kMmWaves;
+  int64_t bound[kMmWaves + 1];  // all loaded together; past n_long: no chunks
+#pragma unroll
+  for (int r = 0; r <= kMmWaves; ++r)
+    bound[r] = p.long_chunk_ptr[l0 + r < n_long ? l0 + r : n_long];
+#pragma unroll
+  for (int r = 0; r < kMmWaves; ++r) {  // the long rows of this block, uniform control flow
+    const int64_t li = l0 + r;
+    const int64_t c0 = bound[r];
+    const int64_t nc = bound[r + 1] - c0;
+    if (nc <= 1) continue;  // written by its chunk
+    const bool whole = nc > (int64_t)kFixWave * ways;
+    if (!whole && wv != r) continue;
+    const int64_t row = p.long_rows[li];
+    const int nw = whole ? ways * kMmWaves : ways;
+    const int w = whole ? wv * ways + way : way;
+    const int64_t per = (nc + nw - 1) / nw;
+    const int64_t k0 = c0 + (w * per < nc ? w * per : nc);
+    const int64_t k1 = c0 + ((w + 1) * per < nc ? (w + 1) * per : nc);
+    for (int64_t n0 = 0; n0 < p.n_dense; n0 += cols) {
+      const int64_t n = n0 + c;
+      CA tot;
+      tot.init();
+      if (n < p.n_dense) tot = fixup_sum(parts, p.n_dense, n, k0, k1);
+      if (nw > 1) {
+        part[threadIdx.x] = tot;
+        if (whole) __syncthreads(); else wave_lds_sync();
+        if (w == 0)
+          for (int i = 1; i < nw; ++i) tot.merge(part[(whole ? 0 : wv * kWave) + (i << col_shift) + c]);
+        if (whole) __syncthreads(); else wave_lds_sync();
+      }
+      if (w == 0 && n < p.n_dense) write_out(p.C, row * p.ldc + n, tot.value(), p.alpha, p.beta);
+    }
   }
 }
 
@@ -453,12 +519,6 @@ constexpr bool kWaveStaged = kHotSpmm<V, I> && G < U;
 
 constexpr int kMmStage = 512;          // entries per wavefront window
 constexpr int kMmStageMax = 8 * kMmStage;
-
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 template <typename A, int G, int VW, int U, typename V, typename I, typename P>
 __device__ __forceinline__ void spmm_staged_rows(const SpmmParams<V, I, P>& p, int64_t rb,
@@ -640,7 +700,9 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
   int rc = check_launch("fs_spmm_csr");
   if (rc || pl->n_chunks <= pl->n_long) return rc;  // no row spans several chunks
   const int64_t blocks = (pl->n_long + kMmWaves - 1) / kMmWaves;
-  spmm_fixup_kernel<A><<<dim3((unsigned)blocks), dim3(kMmBlock), 0, st>>>(p, pl->n_long);
+  int col_shift = 0;
+  while (col_shift < 6 && ((int64_t)1 << col_shift) < n_dense) ++col_shift;
+  spmm_fixup_kernel<A><<<dim3((unsigned)blocks), dim3(kMmBlock), 0, st>>>(p, pl->n_long, col_shift);
   return check_launch("fs_spmm_csr");
 }
 
