@@ -10,8 +10,6 @@
 
 namespace fs {
 
-typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
-
 constexpr int kAnBlock = 1024;
 
 enum {
@@ -34,17 +32,26 @@ __global__ void analyze_init(const P* ptr, int64_t n_rows, int64_t* st) {
   }
 }
 
-__device__ __forceinline__ int64_t wave_sum(int64_t v) {
-  for (int k = 32; k >= 1; k >>= 1) v += __shfl_xor(v, k);
-  return v;
+// Wave reductions by a butterfly of DPP / swizzle moves (fs_device.hpp: every
+// lane of a 2K group holds the group's value after step K, so the mirror
+// partners are as good as xor partners).
+struct OpSum { template <typename T> __device__ static T of(T a, T b) { return a + b; } };
+struct OpMax { template <typename T> __device__ static T of(T a, T b) { return a > b ? a : b; } };
+struct OpMin { template <typename T> __device__ static T of(T a, T b) { return a < b ? a : b; } };
+
+template <int K> __device__ __forceinline__ int32_t an_move(int32_t v) { return xmov_i32<K>(v); }
+template <int K> __device__ __forceinline__ int64_t an_move(int64_t v) {
+  const int lo = xmov_i32<K>((int)(v & 0xffffffff));
+  const int hi = xmov_i32<K>((int)(v >> 32));
+  return ((int64_t)hi << 32) | (uint32_t)lo;
 }
-__device__ __forceinline__ int64_t wave_max(int64_t v) {
-  for (int k = 32; k >= 1; k >>= 1) { int64_t o = __shfl_xor(v, k); v = o > v ? o : v; }
-  return v;
-}
-__device__ __forceinline__ int64_t wave_min(int64_t v) {
-  for (int k = 32; k >= 1; k >>= 1) { int64_t o = __shfl_xor(v, k); v = o < v ? o : v; }
-  return v;
+template <typename Op, typename T> __device__ __forceinline__ T wave_reduce(T v) {
+  v = Op::of(v, an_move<1>(v));
+  v = Op::of(v, an_move<2>(v));
+  v = Op::of(v, an_move<4>(v));
+  v = Op::of(v, an_move<8>(v));
+  v = Op::of(v, an_move<16>(v));
+  return Op::of(v, an_move<32>(v));
 }
 
 // Reduction of statistic k: 0 sum, 1 max, 2 min (PTR0 / PTRN are set by
@@ -53,23 +60,21 @@ __device__ __forceinline__ int stat_op(int k) {
   return (k == ST_LMAX || k == ST_CMAX) ? 1 : (k == ST_LMIN || k == ST_CMIN) ? 2 : 0;
 }
 
-// Reduces the block's statistics v[2..FS_STATS_LEN) together: wave reductions,
-// one LDS exchange and one barrier, then thread k applies statistic k with
-// one atomic.
-__device__ __forceinline__ void block_apply_all(int64_t (&v)[FS_STATS_LEN], int64_t* st) {
+// Reduces the block's statistics v[2..FS_STATS_LEN), each already reduced over
+// its wavefront: one LDS exchange and one barrier, then thread k applies
+// statistic k with one atomic.
+__device__ __forceinline__ void block_apply_all(const int64_t (&v)[FS_STATS_LEN], int64_t* st) {
   __shared__ int64_t red[FS_STATS_LEN][kAnBlock / kWave];
   const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (lane == 0)
 #pragma unroll
-  for (int k = 2; k < FS_STATS_LEN; ++k) {
-    const int op = stat_op(k);
-    v[k] = op == 0 ? wave_sum(v[k]) : op == 1 ? wave_max(v[k]) : wave_min(v[k]);
-    if (lane == 0) red[k][w] = v[k];
-  }
+    for (int k = 2; k < FS_STATS_LEN; ++k) red[k][w] = v[k];
   __syncthreads();
   const int k = threadIdx.x;
   if (k >= 2 && k < FS_STATS_LEN) {
     const int op = stat_op(k);
     int64_t r = red[k][0];
+#pragma unroll
     for (int i = 1; i < kAnBlock / kWave; ++i) {
       const int64_t o = red[k][i];
       r = op == 0 ? r + o : op == 1 ? (o > r ? o : r) : (o < r ? o : r);
@@ -81,6 +86,13 @@ __device__ __forceinline__ void block_apply_all(int64_t (&v)[FS_STATS_LEN], int6
   }
 }
 
+// Memory-bound on large matrices and a latency chain on small ones, where the
+// reduction used to be most of it (fourteen 64-bit wave reductions through
+// ds_bpermute).  Counts are ballots summed in scalar registers, and the six
+// statistics left are reduced with DPP moves.  With both launches: 16,384 rows
+// of 16 entries 13.9 -> 8.6 us, 1M rows of 16 34.8 -> 22.8 us (67 MB), 4M rows
+// of 12 51.0 -> 42.9 us (208 MB, 4.8 TB/s); with 64-bit arrays, whose columns
+// took 8-byte loads, 15.6 -> 10.5, 41.3 -> 31.0, 82.0 -> 71.3 us (5.8 TB/s).
 template <typename I, typename P>
 __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ ptr,
                                                           const I* __restrict__ idx,
@@ -88,91 +100,81 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
                                                           int64_t* st) {
   const int64_t stride = (int64_t)gridDim.x * kAnBlock;
   const int64_t t0 = (int64_t)blockIdx.x * kAnBlock + threadIdx.x;
-  int64_t dec = 0, lmax = 0, lmin = INT64_MAX, sumsq = 0, empty = 0, longnnz = 0;
-  int64_t h[6] = {0, 0, 0, 0, 0, 0};
-  // rows: four row pointer pairs in flight; lanes past the end re-read row
-  // i0 and skip it
+  const int lane = threadIdx.x % kWave;
+  int64_t lmax = 0, lmin = INT64_MAX, sumsq = 0, longnnz = 0;
+  // wavefront totals: rows of length < 0, 0, and above each histogram edge
+  int64_t dec = 0, empty = 0, g0 = 0, g4 = 0, g16 = 0, g64 = 0, g256 = 0, g4096 = 0;
+  // rows: four row pointer pairs in flight; lanes past the end re-read the
+  // last row and skip it.  The loop is uniform over the wavefront (ballots).
   constexpr int kRows = 4;
-  for (int64_t i0 = t0; i0 < n_rows; i0 += kRows * stride) {
+  for (int64_t w0 = t0 - lane; w0 < n_rows; w0 += kRows * stride) {
     int64_t len[kRows];
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
-      const int64_t i = i0 + u * stride < n_rows ? i0 + u * stride : i0;
+      const int64_t i = w0 + lane + u * stride < n_rows ? w0 + lane + u * stride : n_rows - 1;
       len[u] = (int64_t)ptr[i + 1] - (int64_t)ptr[i];
     }
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
-      if (i0 + u * stride >= n_rows) break;
+      const bool live = w0 + lane + u * stride < n_rows;
       const int64_t l = len[u];
-      dec += l < 0;
-      lmax = l > lmax ? l : lmax;
-      lmin = l < lmin ? l : lmin;
-      sumsq += l * l;
-      if (l <= 0) empty += l == 0;
-      else if (l <= 4) ++h[0];
-      else if (l <= 16) ++h[1];
-      else if (l <= 64) ++h[2];
-      else if (l <= 256) ++h[3];
-      else if (l <= 4096) ++h[4];
-      else ++h[5];
-      if (l > 256) longnnz += l;
+      dec += __popcll(__ballot(live && l < 0));
+      empty += __popcll(__ballot(live && l == 0));
+      g0 += __popcll(__ballot(live && l > 0));
+      g4 += __popcll(__ballot(live && l > 4));
+      g16 += __popcll(__ballot(live && l > 16));
+      g64 += __popcll(__ballot(live && l > 64));
+      g256 += __popcll(__ballot(live && l > 256));
+      g4096 += __popcll(__ballot(live && l > 4096));
+      if (live) {
+        lmax = l > lmax ? l : lmax;
+        lmin = l < lmin ? l : lmin;
+        sumsq += l * l;
+        if (l > 256) longnnz += l;
+      }
     }
   }
   // columns: only min and max are kept, so a lane past the end re-reads the
-  // iteration's first column instead of branching
-  int64_t cmin = INT64_MAX, cmax = -1;
-  int64_t j0 = 0;
-  if constexpr (sizeof(I) == 4) {
-    // 16-byte loads (four columns), eight in flight per thread, over the
-    // aligned body of the column array.  Non-temporal: the columns are read
-    // once here, and an unprepared call's SpMV follows at once, whose data
-    // they would otherwise push out of the caches (4M-row power-law matrix:
-    // this pass 51.5 -> 53.8 us, the whole repeated unprepared call 268 ->
-    // 254 us).
-    const int64_t head = (int64_t)(((16 - ((uintptr_t)idx & 15)) & 15) / 4);
-    const int64_t h0 = head < nnz ? head : nnz;
-    const int64_t n4 = (nnz - h0) / 4;
-    const int4* q = reinterpret_cast<const int4*>(idx + h0);
-    int32_t mn = INT32_MAX, mx = INT32_MIN;
-    for (int64_t k = t0; k < n4; k += 8 * stride) {
-      int4 c[8];
+  // iteration's first column instead of branching.  16-byte loads (four 32-bit
+  // or two 64-bit columns), eight in flight per thread, over the aligned body
+  // of the column array.  Non-temporal: the columns are read once here, and an
+  // unprepared call's SpMV follows at once, whose data they would otherwise
+  // push out of the caches (4M-row power-law matrix: this pass 51.5 -> 53.8 us,
+  // the whole repeated unprepared call 268 -> 254 us).
+  typedef I vec_t __attribute__((ext_vector_type(16 / sizeof(I))));
+  constexpr int kPer = 16 / (int)sizeof(I);
+  I mn = sizeof(I) == 4 ? (I)INT32_MAX : (I)INT64_MAX, mx = -1;
+  const int64_t head = (int64_t)(((16 - ((uintptr_t)idx & 15)) & 15) / sizeof(I));
+  const int64_t h0 = head < nnz ? head : nnz;
+  const int64_t nv = (nnz - h0) / kPer;
+  const vec_t* q = reinterpret_cast<const vec_t*>(idx + h0);
+  for (int64_t k = t0; k < nv; k += 8 * stride) {
+    vec_t c[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const i32x4_t v = __builtin_nontemporal_load(
-            reinterpret_cast<const i32x4_t*>(q + (k + u * stride < n4 ? k + u * stride : k)));
-        c[u] = make_int4(v.x, v.y, v.z, v.w);
+    for (int u = 0; u < 8; ++u)
+      c[u] = __builtin_nontemporal_load(q + (k + u * stride < nv ? k + u * stride : k));
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        mn = c[u][e] < mn ? c[u][e] : mn;
+        mx = c[u][e] > mx ? c[u][e] : mx;
       }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        mn = min(mn, min(min(c[u].x, c[u].y), min(c[u].z, c[u].w)));
-        mx = max(mx, max(max(c[u].x, c[u].y), max(c[u].z, c[u].w)));
-      }
-    }
-    if (t0 < n4) {
-      cmin = mn;
-      cmax = mx;
-    }
-    // the unaligned head [0, h0); the tail [h0 + 4 n4, nnz) is left to the
-    // loop below
-    if (t0 < h0) {
-      const int64_t c = (int64_t)idx[t0];
-      cmin = c < cmin ? c : cmin;
-      cmax = c > cmax ? c : cmax;
-    }
-    j0 = h0 + 4 * n4;
   }
-  for (int64_t j = j0 + t0; j < nnz; j += 4 * stride) {
-    int64_t c[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) c[u] = (int64_t)idx[j + u * stride < nnz ? j + u * stride : j];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      cmin = c[u] < cmin ? c[u] : cmin;
-      cmax = c[u] > cmax ? c[u] : cmax;
-    }
+  // the unaligned head and the tail: fewer than two vectors of columns
+  const int64_t tail = h0 + kPer * nv;
+  if (t0 < h0 + (nnz - tail)) {
+    const I c = idx[t0 < h0 ? t0 : tail + (t0 - h0)];
+    mn = c < mn ? c : mn;
+    mx = c > mx ? c : mx;
   }
-  int64_t v[FS_STATS_LEN] = {0, 0, dec, cmin, cmax, lmax, lmin, sumsq, empty,
-                             h[0], h[1], h[2], h[3], h[4], h[5], longnnz};
+  // no columns at all: the initial INT64_MAX stays (every 32-bit column is
+  // at most the narrower start value)
+  const int64_t cmin = nnz > 0 ? (int64_t)wave_reduce<OpMin>(mn) : INT64_MAX;
+  const int64_t v[FS_STATS_LEN] = {
+      0, 0, dec, cmin, (int64_t)wave_reduce<OpMax>(mx), wave_reduce<OpMax>(lmax),
+      wave_reduce<OpMin>(lmin), wave_reduce<OpSum>(sumsq), empty, g0 - g4, g4 - g16, g16 - g64,
+      g64 - g256, g256 - g4096, g4096, wave_reduce<OpSum>(longnnz)};
   block_apply_all(v, st);
 }
 
@@ -185,11 +187,12 @@ int launch_analyze(const fs_csr* A, int64_t* st, hipStream_t s) {
   if (rc) return rc;
   const int64_t work = A->n_rows > A->nnz ? A->n_rows : A->nnz;
   if (work == 0) return FS_OK;
-  // few, wide blocks (two per CU): each reduces in LDS first, so every
-  // statistic sees at most `blocks` same-address atomics (they serialise),
-  // while each thread keeps eight 16-byte column loads in flight
+  // few, wide blocks (one per CU): each reduces in LDS first, so every
+  // statistic sees at most `blocks` same-address atomics (they serialise: with
+  // two blocks per CU 1M rows of 16 take 28.2 instead of 22.8 us), while each
+  // thread keeps eight 16-byte column loads in flight
   int64_t blocks = (work + kAnBlock * 32 - 1) / (kAnBlock * 32);
-  if (blocks > 512) blocks = 512;
+  if (blocks > 256) blocks = 256;
   analyze_pass<I, P><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st);
   return check_launch("fs_csr_analyze");
 }
