@@ -188,6 +188,10 @@ _SIGNATURES = {
                                    ctypes.c_double, ctypes.c_double, ctypes.POINTER(FsPlan),
                                    ctypes.c_int32, ctypes.c_void_p]),
     "fs_csr_analyze": (ctypes.c_int, [ctypes.POINTER(FsCsr), ctypes.c_void_p, ctypes.c_void_p]),
+    "fs_csr_analyze_split": (ctypes.c_int, [ctypes.POINTER(FsCsr), ctypes.c_void_p, ctypes.c_int64,
+                                            ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+                                            ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
+                                            ctypes.c_void_p, ctypes.c_void_p]),
     "fs_split_values": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(FsCsr), ctypes.c_void_p,
                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "fs_spmv_csr_split": (ctypes.c_int, [ctypes.POINTER(FsCsr), ctypes.c_int32, ctypes.c_void_p,
@@ -356,6 +360,35 @@ def analyze_device(csr: FsCsr, device):
 def analyze(csr: FsCsr, device) -> list[int]:
     """Run fs_csr_analyze and copy the FS_STATS_LEN statistics to the host."""
     return analyze_device(csr, device).cpu().tolist()
+
+
+SPLIT_CHUNK_BITS = 36  # stats[FS_STATS_LEN] of analyze_split: n_long << 36 | n_chunks
+
+
+def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bool):
+    """Run fs_csr_analyze_split; returns (statistics on the host, long_rows,
+    long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed columns or None).
+    The lists share one allocation; entries past n_long / n_chunks are unset."""
+    lib = load()
+    nnz = int(csr.nnz)
+    cap_long = min(int(csr.n_rows), nnz // (short_max + 1))
+    cap_chunks = min(nnz // chunk_nnz + cap_long, nnz)
+    words = FS_STATS_LEN + 1
+    buf = torch.empty(words + 2 * cap_long + 1 + (cap_chunks + 1) // 2, dtype=torch.int64,
+                      device=device)
+    long_rows = buf[words:words + cap_long]
+    long_chunk_ptr = buf[words + cap_long:words + 2 * cap_long + 1]
+    chunk_long = buf[words + 2 * cap_long + 1:].view(torch.int32)
+    cols32 = torch.empty(nnz, dtype=torch.int32, device=device) if narrow else None
+    with on_device(device):
+        check(lib.fs_csr_analyze_split(ctypes.byref(csr), buf.data_ptr(), short_max, chunk_nnz,
+                                       ptr(long_rows), long_chunk_ptr.data_ptr(), cap_long,
+                                       ptr(chunk_long), cap_chunks, ptr(cols32),
+                                       stream_handle(device)), "fs_csr_analyze_split")
+    stats = buf[:words].cpu().tolist()
+    n_long = stats[FS_STATS_LEN] >> SPLIT_CHUNK_BITS
+    n_chunks = stats[FS_STATS_LEN] & ((1 << SPLIT_CHUNK_BITS) - 1)
+    return (stats[:FS_STATS_LEN], long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, cols32)
 
 
 def features(stats, n_rows: int, n_cols: int, nnz: int, device):

@@ -18,9 +18,68 @@ enum {
 };
 static_assert(ST_LONGNNZ + 1 == FS_STATS_LEN, "statistics layout");
 
+// Row-split outputs of fs_csr_analyze_split (see the header).  st[ST_SPLIT]
+// counts long rows and chunks together, chunks in the low kSplitBits bits, so
+// that one atomic gives a group of rows consecutive long-row ordinals and
+// consecutive chunks at once.
+constexpr int ST_SPLIT = FS_STATS_LEN;
+constexpr int kSplitBits = 36;
+
+struct SplitOut {
+  int64_t short_max = 0, chunk_nnz = 0, cap_long = 0, cap_chunks = 0;
+  int64_t* long_rows = nullptr;
+  int64_t* long_chunk_ptr = nullptr;
+  int32_t* chunk_long = nullptr;
+  int32_t* cols32 = nullptr;
+};
+
+// Lists the wavefront's long rows (`lg`: row `row` of this lane, length l).
+// Rows of one wavefront take consecutive ordinals; the order of wavefronts is
+// free, and so is the order of rows in the list: a row's chunks are its own
+// and are summed in chunk order wherever they lie.  Row pointers are not
+// validated yet, so every write is bounded by the capacities.
+__device__ __forceinline__ void split_rows(const SplitOut& s, int64_t* st, bool lg, int64_t row,
+                                           int64_t l, int lane) {
+  const uint64_t m = __ballot(lg);
+  if (m == 0) return;  // uniform
+  int64_t per = lg ? (l - 1) / s.chunk_nnz + 1 : 0;
+  if (per > s.cap_chunks) per = s.cap_chunks + 1;
+  int64_t scan = per;  // inclusive over the wavefront
+#pragma unroll
+  for (int k = 1; k < kWave; k <<= 1) {
+    const int64_t o = __shfl_up(scan, k);
+    if (lane >= k) scan += o;
+  }
+  const uint64_t total = (uint64_t)__shfl(scan, kWave - 1);
+  uint64_t base = 0;
+  if (lane == 0)
+    base = __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(st + ST_SPLIT),
+                                  ((uint64_t)__popcll(m) << kSplitBits) + total, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+  base = __shfl(base, 0);
+  const int64_t li = (int64_t)(base >> kSplitBits) + __popcll(m & (((uint64_t)1 << lane) - 1));
+  const int64_t c0 = (int64_t)(base & (((uint64_t)1 << kSplitBits) - 1)) + scan - per;
+  if (lg && li < s.cap_long) {
+    s.long_rows[li] = row;
+    s.long_chunk_ptr[li + 1] = c0 + per;  // where the next ordinal's chunks begin
+    if (per == 1 && c0 < s.cap_chunks) s.chunk_long[c0] = (int32_t)li;
+  }
+  // rows of several chunks: the whole wavefront fills each row's chunk list
+  for (uint64_t rest = __ballot(lg && per > 1); rest; rest &= rest - 1) {
+    const int src = __builtin_ctzll(rest);
+    const int64_t n = __shfl(per, src), c = __shfl(c0, src), o = __shfl(li, src);
+    for (int64_t k = lane; k < n; k += kWave)
+      if (o < s.cap_long && c + k < s.cap_chunks) s.chunk_long[c + k] = (int32_t)o;
+  }
+}
+
 template <typename P>
-__global__ void analyze_init(const P* ptr, int64_t n_rows, int64_t* st) {
+__global__ void analyze_init(const P* ptr, int64_t n_rows, int64_t* st, int64_t* long_chunk_ptr) {
   const int t = threadIdx.x;
+  if (t == 0 && long_chunk_ptr) {
+    st[ST_SPLIT] = 0;
+    long_chunk_ptr[0] = 0;
+  }
   if (t < FS_STATS_LEN) {
     int64_t v = 0;
     if (t == ST_CMIN) v = INT64_MAX;
@@ -93,11 +152,11 @@ __device__ __forceinline__ void block_apply_all(const int64_t (&v)[FS_STATS_LEN]
 // of 16 entries 13.9 -> 8.6 us, 1M rows of 16 34.8 -> 22.8 us (67 MB), 4M rows
 // of 12 51.0 -> 42.9 us (208 MB, 4.8 TB/s); with 64-bit arrays, whose columns
 // took 8-byte loads, 15.6 -> 10.5, 41.3 -> 31.0, 82.0 -> 71.3 us (5.8 TB/s).
-template <typename I, typename P>
+template <typename I, typename P, bool SPLIT>
 __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ ptr,
                                                           const I* __restrict__ idx,
                                                           int64_t n_rows, int64_t nnz,
-                                                          int64_t* st) {
+                                                          int64_t* st, SplitOut split) {
   const int64_t stride = (int64_t)gridDim.x * kAnBlock;
   const int64_t t0 = (int64_t)blockIdx.x * kAnBlock + threadIdx.x;
   const int lane = threadIdx.x % kWave;
@@ -132,6 +191,8 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
         sumsq += l * l;
         if (l > 256) longnnz += l;
       }
+      if constexpr (SPLIT)
+        split_rows(split, st, live && l > split.short_max, w0 + lane + u * stride, l, lane);
     }
   }
   // columns: only min and max are kept, so a lane past the end re-reads the
@@ -160,11 +221,25 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
         mn = c[u][e] < mn ? c[u][e] : mn;
         mx = c[u][e] > mx ? c[u][e] : mx;
       }
+    if constexpr (SPLIT && sizeof(I) == 8) {
+      // 32-bit copy of the columns; a vector past the end is vector k again
+      if (split.cols32) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int64_t j = h0 + 2 * (k + u * stride < nv ? k + u * stride : k);
+          split.cols32[j] = (int32_t)c[u][0];
+          split.cols32[j + 1] = (int32_t)c[u][1];
+        }
+      }
+    }
   }
   // the unaligned head and the tail: fewer than two vectors of columns
   const int64_t tail = h0 + kPer * nv;
   if (t0 < h0 + (nnz - tail)) {
-    const I c = idx[t0 < h0 ? t0 : tail + (t0 - h0)];
+    const int64_t j = t0 < h0 ? t0 : tail + (t0 - h0);
+    const I c = idx[j];
+    if constexpr (SPLIT && sizeof(I) == 8)
+      if (split.cols32) split.cols32[j] = (int32_t)c;
     mn = c < mn ? c : mn;
     mx = c > mx ? c : mx;
   }
@@ -179,10 +254,10 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
 }
 
 template <typename I, typename P>
-int launch_analyze(const fs_csr* A, int64_t* st, hipStream_t s) {
+int launch_analyze(const fs_csr* A, int64_t* st, const SplitOut* split, hipStream_t s) {
   const P* ptr = static_cast<const P*>(A->row_ptr);
   const I* idx = static_cast<const I*>(A->col_idx);
-  analyze_init<P><<<1, 64, 0, s>>>(ptr, A->n_rows, st);
+  analyze_init<P><<<1, 64, 0, s>>>(ptr, A->n_rows, st, split ? split->long_chunk_ptr : nullptr);
   int rc = check_launch("fs_csr_analyze");
   if (rc) return rc;
   const int64_t work = A->n_rows > A->nnz ? A->n_rows : A->nnz;
@@ -193,25 +268,59 @@ int launch_analyze(const fs_csr* A, int64_t* st, hipStream_t s) {
   // thread keeps eight 16-byte column loads in flight
   int64_t blocks = (work + kAnBlock * 32 - 1) / (kAnBlock * 32);
   if (blocks > 256) blocks = 256;
-  analyze_pass<I, P><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st);
+  if (split)
+    analyze_pass<I, P, true><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st, *split);
+  else
+    analyze_pass<I, P, false><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st, SplitOut{});
   return check_launch("fs_csr_analyze");
+}
+
+static int analyze_checked(const fs_csr* A, int64_t* stats, const SplitOut* split, void* stream,
+                           const char* who) {
+  if (!A) return fail(FS_ERR_VALUE, "%s: matrix descriptor is null", who);
+  if ((A->index_type != FS_I32 && A->index_type != FS_I64) ||
+      (A->ptr_type != FS_I32 && A->ptr_type != FS_I64))
+    return fail(FS_ERR_TYPE, "%s: index and row-pointer types must be FS_I32 or FS_I64", who);
+  if (A->n_rows < 0 || A->nnz < 0) return fail(FS_ERR_VALUE, "%s: negative size", who);
+  if (!stats) return fail(FS_ERR_VALUE, "%s: stats is null", who);
+  if (!A->row_ptr) return fail(FS_ERR_VALUE, "%s: row_ptr is null", who);
+  if (A->nnz > 0 && !A->col_idx) return fail(FS_ERR_VALUE, "%s: col_idx is null", who);
+  hipStream_t s = as_stream(stream);
+  if (A->index_type == FS_I32 && A->ptr_type == FS_I32) return launch_analyze<int32_t, int32_t>(A, stats, split, s);
+  if (A->index_type == FS_I32 && A->ptr_type == FS_I64) return launch_analyze<int32_t, int64_t>(A, stats, split, s);
+  if (A->index_type == FS_I64 && A->ptr_type == FS_I32) return launch_analyze<int64_t, int32_t>(A, stats, split, s);
+  return launch_analyze<int64_t, int64_t>(A, stats, split, s);
 }
 
 }  // namespace fs
 
+using namespace fs;
+
 extern "C" int fs_csr_analyze(const fs_csr* A, int64_t* stats, void* stream) {
-  using namespace fs;
-  if (!A) return fail(FS_ERR_VALUE, "fs_csr_analyze: matrix descriptor is null");
-  if ((A->index_type != FS_I32 && A->index_type != FS_I64) ||
-      (A->ptr_type != FS_I32 && A->ptr_type != FS_I64))
-    return fail(FS_ERR_TYPE, "fs_csr_analyze: index and row-pointer types must be FS_I32 or FS_I64");
-  if (A->n_rows < 0 || A->nnz < 0) return fail(FS_ERR_VALUE, "fs_csr_analyze: negative size");
-  if (!stats) return fail(FS_ERR_VALUE, "fs_csr_analyze: stats is null");
-  if (!A->row_ptr) return fail(FS_ERR_VALUE, "fs_csr_analyze: row_ptr is null");
-  if (A->nnz > 0 && !A->col_idx) return fail(FS_ERR_VALUE, "fs_csr_analyze: col_idx is null");
-  hipStream_t s = as_stream(stream);
-  if (A->index_type == FS_I32 && A->ptr_type == FS_I32) return launch_analyze<int32_t, int32_t>(A, stats, s);
-  if (A->index_type == FS_I32 && A->ptr_type == FS_I64) return launch_analyze<int32_t, int64_t>(A, stats, s);
-  if (A->index_type == FS_I64 && A->ptr_type == FS_I32) return launch_analyze<int64_t, int32_t>(A, stats, s);
-  return launch_analyze<int64_t, int64_t>(A, stats, s);
+  return analyze_checked(A, stats, nullptr, stream, "fs_csr_analyze");
+}
+
+extern "C" int fs_csr_analyze_split(const fs_csr* A, int64_t* stats, int64_t short_max,
+                                    int64_t chunk_nnz, int64_t* long_rows, int64_t* long_chunk_ptr,
+                                    int64_t cap_long, int32_t* chunk_long, int64_t cap_chunks,
+                                    int32_t* cols32, void* stream) {
+  const char* who = "fs_csr_analyze_split";
+  if (A && A->nnz > INT32_MAX) return fail(FS_ERR_UNSUPPORTED, "%s: more than 2^31 - 1 entries", who);
+  if (short_max < 1) return fail(FS_ERR_VALUE, "%s: short_max must be >= 1", who);
+  if (chunk_nnz <= 0 || chunk_nnz % kWave != 0)
+    return fail(FS_ERR_VALUE, "%s: chunk_nnz must be a positive multiple of 64", who);
+  if (cap_long < 0 || cap_chunks < 0 || cap_long > INT32_MAX || cap_chunks > INT32_MAX)
+    return fail(FS_ERR_VALUE, "%s: capacities must be in [0, 2^31)", who);
+  if (!long_chunk_ptr || (cap_long > 0 && !long_rows) || (cap_chunks > 0 && !chunk_long))
+    return fail(FS_ERR_VALUE, "%s: null list", who);
+  SplitOut s;
+  s.short_max = short_max;
+  s.chunk_nnz = chunk_nnz;
+  s.cap_long = cap_long;
+  s.cap_chunks = cap_chunks;
+  s.long_rows = long_rows;
+  s.long_chunk_ptr = long_chunk_ptr;
+  s.chunk_long = chunk_long;
+  s.cols32 = cols32;
+  return analyze_checked(A, stats, &s, stream, who);
 }

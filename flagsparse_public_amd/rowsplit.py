@@ -235,6 +235,23 @@ class RowSplitPlan:
             self.tile_start = None
             self.n_tiles = 0
 
+    @classmethod
+    def listed(cls, schedule: Schedule, accumulate: int, value_dtype, device, long_rows,
+               long_chunk_ptr, chunk_long, n_long: int, n_chunks: int):
+        """A row-group plan over long-row lists that are already on the
+        device (``_lib.analyze_split``)."""
+        self = cls.__new__(cls)
+        self.schedule = schedule
+        self.accumulate = int(accumulate)
+        self.value_code = _lib.value_code(value_dtype)
+        self.device = device
+        self._work = {}
+        self._structs = {}
+        self.long_rows, self.long_chunk_ptr, self.chunk_long = long_rows, long_chunk_ptr, chunk_long
+        self.n_long, self.n_chunks = int(n_long), int(n_chunks)
+        self.tile_start, self.n_tiles = None, 0
+        return self
+
     ENTRY_ROW_CAP = 768  # owned rows per entry tile (the kernel's LDS row batch)
 
     def _init_entry_tiles(self, indptr, n_rows, schedule):

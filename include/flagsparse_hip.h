@@ -372,6 +372,24 @@ int fs_spmm_csr(const fs_csr *A, const void *B, int64_t ldb, void *C, int64_t ld
 #define FS_STATS_LEN 16
 int fs_csr_analyze(const fs_csr *A, int64_t *stats, void *stream);
 
+/*
+ * fs_csr_analyze that also lists the long rows of a row-split plan in the same
+ * pass (the long_rows / long_chunk_ptr / chunk_long of fs_plan), so that a
+ * call on an unprepared matrix needs no further pass over its row pointers.
+ * stats holds FS_STATS_LEN + 1 values: [16] = n_long * 2^36 + n_chunks, for
+ * rows longer than short_max (>= 1) cut into chunks of chunk_nnz entries (a
+ * multiple of 64).  The row order of the list is not fixed.  The lists take
+ * cap_long (+ 1 for long_chunk_ptr) and cap_chunks elements; a valid matrix
+ * has at most nnz / (short_max + 1) long rows and nnz / chunk_nnz + n_long
+ * chunks, and nothing is written past the capacities for any other.  cols32
+ * (or null): the columns of a matrix with 64-bit indices, narrowed; they mean
+ * something only if the statistics say that every column fits.  At most
+ * 2^31 - 1 entries.
+ */
+int fs_csr_analyze_split(const fs_csr *A, int64_t *stats, int64_t short_max, int64_t chunk_nnz,
+                         int64_t *long_rows, int64_t *long_chunk_ptr, int64_t cap_long,
+                         int32_t *chunk_long, int64_t cap_chunks, int32_t *cols32, void *stream);
+
 /* ------------------------------------------- split-precision value storage */
 /*
  * Storage formats for the values of an fp32 matrix (x, y stay fp32; the sum is
