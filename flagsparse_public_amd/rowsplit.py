@@ -181,8 +181,33 @@ def tile_starts(row_lengths: torch.Tensor, short_max: int, tile_nnz: int,
     return torch.unique(torch.cat(parts))
 
 
+SPMM_FILL_LANES = 1 << 18  # lanes of 256 CUs with 16 wavefronts each
+
+
 def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int) -> Schedule:
-    return Schedule(group_lanes=1, short_max=256, chunk_nnz=256, unroll=4, col_tile=0)
+    """Which SpMM rows one lane group walks alone and which whole wavefronts
+    take in chunks.
+
+    A lane group walks its row serially (a round trip to the B rows per batch
+    of entries), so the longest short row bounds the launch: rows over about
+    twice the mean are chunked.  170,000 power-law rows (mean 12), N = 47: 132
+    us with rows up to 256 short, 96 us with 32; 60,000 fp64 rows, N = 16: 57
+    against 22 us.  Below twice the mean, typical rows would leave the groups
+    (100,000 rows of about 60, N = 64 in bf16: 90 us with 128, 119 with 64, 189
+    with 32); rows of 300, N = 64: 84 us with 1024 against 134 with 256.
+
+    With long rows and too few of them to fill the chip with lane groups,
+    every row gets a wavefront: 5,000 rows of about 300, N = 16: 45 -> 12 us;
+    20,000 rows, N = 8: 77 -> 37 us; at 30,000 rows of 100 the two meet (N = 8,
+    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us)."""
+    mean = nnz / n_rows if n_rows > 0 else 0.0
+    lanes = max(8, _pow2_ceil(n_dense / 4.0))
+    if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
+        return Schedule(group_lanes=1, short_max=32, chunk_nnz=512, unroll=4, col_tile=0)
+    short = 32
+    while short < 2 * mean and short < 1024:
+        short *= 2
+    return Schedule(group_lanes=1, short_max=short, chunk_nnz=256, unroll=4, col_tile=0)
 
 
 class RowSplitPlan:

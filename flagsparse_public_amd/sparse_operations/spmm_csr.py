@@ -195,11 +195,11 @@ def _spmm_call_inputs(data, indices, indptr, B, shape):
     order, with the plan of the call's schedule listed by the analysis pass
     itself and 64-bit columns narrowed by it; row pointers stay as given (the
     kernels take both widths).  One pass and one host read instead of a dozen
-    small launches with three host reads: 170,000 power-law rows, N = 47, 349
-    -> 178 us a
-    call; 250,000 rows of 20, bf16, N = 128, 285 -> 223 us.  Returns (data, columns, indptr, B, n_rows, n_cols,
-    n_dense, plan, max_row_nnz); the plan is None beyond 2^31 - 1 entries,
-    which the pass does not list."""
+    small launches with three host reads: 170,000 power-law rows, N = 47,
+    int64 arrays, 349 -> 178 us a call; 250,000 rows of 20, bf16, N = 128, 285
+    -> 223 us.  Returns (data, columns, indptr, B, n_rows, n_cols, n_dense, plan,
+    max_row_nnz); the plan is None beyond 2^31 - 1 entries, which the pass
+    does not list."""
     if B.ndim != 2:
         raise ValueError("B must be a 2D dense tensor")
     if data.numel() > _INDEX_LIMIT_INT32:
@@ -555,9 +555,17 @@ def spmm_launch_schedule(prepared, n_dense, schedule=None):
     """The (schedule, column tile) an opt / alg2 SpMM call with n_dense
     columns launches."""
     if schedule is None and prepared.library_schedule:
-        sch = prepared.schedule or default_spmm_schedule(prepared.n_rows, prepared.data.numel(),
-                                                         n_dense)
-        return _library_spmm_launch(sch, prepared.data.dtype, n_dense)
+        known = prepared._plans.get(("launch", n_dense))
+        if known is not None and known[0] is prepared.schedule:
+            return known[1]
+        # the row split follows the mean row length whatever variant was
+        # chosen (the variants' own bounds were picked with longer short rows)
+        split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense)
+        sch = dataclasses.replace(prepared.schedule or split, short_max=split.short_max,
+                                  chunk_nnz=split.chunk_nnz)
+        launch = _library_spmm_launch(sch, prepared.data.dtype, n_dense)
+        prepared._plans[("launch", n_dense)] = (prepared.schedule, launch)
+        return launch
     sch = schedule or prepared.schedule or default_spmm_schedule(prepared.n_rows,
                                                                  prepared.data.numel(), n_dense)
     return sch, sch.col_tile
