@@ -192,6 +192,13 @@ _SIGNATURES = {
                                             ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
                                             ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
                                             ctypes.c_void_p, ctypes.c_void_p]),
+    "fs_coo_sort_workspace": (ctypes.c_int64, [ctypes.c_int64] * 3),
+    "fs_coo_sort": (ctypes.c_int, [ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
+                                   ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+                                   ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
+                                   ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
+                                   ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                   ctypes.c_void_p]),
     "fs_split_values": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(FsCsr), ctypes.c_void_p,
                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "fs_spmv_csr_split": (ctypes.c_int, [ctypes.POINTER(FsCsr), ctypes.c_int32, ctypes.c_void_p,
@@ -347,10 +354,12 @@ def stream_handle(device) -> int:
     return int(_RAW_STREAM(idx))
 
 
-def analyze_device(csr: FsCsr, device):
-    """Run fs_csr_analyze; returns the FS_STATS_LEN statistics on the device."""
+def analyze_device(csr: FsCsr, device, stats=None):
+    """Run fs_csr_analyze; returns the FS_STATS_LEN statistics on the device
+    (in ``stats`` when given)."""
     lib = load()
-    stats = torch.empty(FS_STATS_LEN, dtype=torch.int64, device=device)
+    if stats is None:
+        stats = torch.empty(FS_STATS_LEN, dtype=torch.int64, device=device)
     with on_device(device):
         check(lib.fs_csr_analyze(ctypes.byref(csr), stats.data_ptr(), stream_handle(device)),
               "fs_csr_analyze")
@@ -362,33 +371,75 @@ def analyze(csr: FsCsr, device) -> list[int]:
     return analyze_device(csr, device).cpu().tolist()
 
 
+COO_BAD_ROW, COO_BAD_COL, COO_OVERFLOW = 1, 2, 4  # *flags of fs_coo_sort
+
+
+def coo_sort_applies(nnz: int, n_rows: int, n_cols: int) -> bool:
+    """Whether coo_sort takes this size (see fs_coo_sort)."""
+    return nnz > 0 and int(load().fs_coo_sort_workspace(nnz, n_rows, n_cols)) > 0
+
+
+def coo_sort(data, row, col, n_rows: int, n_cols: int, flags, index_dtype=None, want_rows=True,
+             ptr_dtype=torch.int64):
+    """Run fs_coo_sort on contiguous device arrays (row and col of one dtype);
+    returns (values, rows or None, columns, row pointer) in CSR order, rows and
+    columns as ``index_dtype`` (default: theirs).  ``flags`` (one int64 on the
+    device) receives the checks: read it before using the arrays."""
+    lib = load()
+    device, nnz = data.device, data.numel()
+    index_dtype = index_dtype or row.dtype
+    out = torch.empty_like(data)
+    out_row = torch.empty(nnz, dtype=index_dtype, device=device) if want_rows else None
+    out_col = torch.empty(nnz, dtype=index_dtype, device=device)
+    indptr = torch.empty(n_rows + 1, dtype=ptr_dtype, device=device)
+    work = torch.empty(int(lib.fs_coo_sort_workspace(nnz, n_rows, n_cols)), dtype=torch.uint8, device=device)
+    with on_device(device):
+        check(lib.fs_coo_sort(data.element_size(), data.data_ptr(), index_code(row.dtype),
+                              row.data_ptr(), col.data_ptr(), nnz, n_rows, n_cols, out.data_ptr(),
+                              index_code(index_dtype), ptr(out_row), out_col.data_ptr(),
+                              index_code(ptr_dtype), indptr.data_ptr(), work.data_ptr(),
+                              work.numel(), flags.data_ptr(), stream_handle(device)), "fs_coo_sort")
+    return out, out_row, out_col, indptr
+
+
 SPLIT_CHUNK_BITS = 36  # stats[FS_STATS_LEN] of analyze_split: n_long << 36 | n_chunks
 
 
-def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bool):
+def split_lists(nnz: int, n_rows: int, short_max: int, chunk_nnz: int, device):
+    """One allocation for analyze_split: the statistics, their packed counts,
+    one spare word that its host copy also reads (element FS_STATS_LEN + 1 of
+    the first tensor returned), and the lists at their largest sizes for a
+    valid matrix."""
+    cap_long = min(n_rows, nnz // (short_max + 1))
+    cap_chunks = min(nnz // chunk_nnz + cap_long, nnz)
+    at = FS_STATS_LEN + 2
+    buf = torch.empty(at + 2 * cap_long + 1 + (cap_chunks + 1) // 2, dtype=torch.int64,
+                      device=device)
+    return (buf, buf[at:at + cap_long], buf[at + cap_long:at + 2 * cap_long + 1],
+            buf[at + 2 * cap_long + 1:].view(torch.int32), cap_long, cap_chunks)
+
+
+def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bool, lists=None):
     """Run fs_csr_analyze_split; returns (statistics on the host, long_rows,
-    long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed columns or None).
-    The lists share one allocation; entries past n_long / n_chunks are unset."""
+    long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed columns or None, the
+    spare word of ``lists``).  Entries of the lists past n_long / n_chunks are
+    unset.  ``lists``: from split_lists, where the caller uses the spare word."""
     lib = load()
     nnz = int(csr.nnz)
-    cap_long = min(int(csr.n_rows), nnz // (short_max + 1))
-    cap_chunks = min(nnz // chunk_nnz + cap_long, nnz)
-    words = FS_STATS_LEN + 1
-    buf = torch.empty(words + 2 * cap_long + 1 + (cap_chunks + 1) // 2, dtype=torch.int64,
-                      device=device)
-    long_rows = buf[words:words + cap_long]
-    long_chunk_ptr = buf[words + cap_long:words + 2 * cap_long + 1]
-    chunk_long = buf[words + 2 * cap_long + 1:].view(torch.int32)
+    if lists is None:
+        lists = split_lists(nnz, int(csr.n_rows), short_max, chunk_nnz, device)
+    buf, long_rows, long_chunk_ptr, chunk_long, cap_long, cap_chunks = lists
     cols32 = torch.empty(nnz, dtype=torch.int32, device=device) if narrow else None
     with on_device(device):
         check(lib.fs_csr_analyze_split(ctypes.byref(csr), buf.data_ptr(), short_max, chunk_nnz,
                                        ptr(long_rows), long_chunk_ptr.data_ptr(), cap_long,
                                        ptr(chunk_long), cap_chunks, ptr(cols32),
                                        stream_handle(device)), "fs_csr_analyze_split")
-    stats = buf[:words].cpu().tolist()
+    stats = buf[:FS_STATS_LEN + 2].cpu().tolist()
     n_long = stats[FS_STATS_LEN] >> SPLIT_CHUNK_BITS
     n_chunks = stats[FS_STATS_LEN] & ((1 << SPLIT_CHUNK_BITS) - 1)
-    return (stats[:FS_STATS_LEN], long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, cols32)
+    return (stats[:FS_STATS_LEN], long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, cols32,
+            stats[FS_STATS_LEN + 1])
 
 
 def features(stats, n_rows: int, n_cols: int, nnz: int, device):

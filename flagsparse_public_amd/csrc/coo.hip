@@ -1,0 +1,525 @@
+// coo.hip -- COO entries to CSR order on the device (entry point fs_coo_sort):
+// the entries ordered by (row, column), equal pairs in input order, and the row
+// pointer they imply, with the index-range checks in the same passes.
+//
+// A sample sort of packed keys row | column | input position (the bit widths
+// of n_rows, n_cols and nnz, at most 64 together), so that keys are distinct
+// and one comparison decides.  A stratified sample gives splitters for up to
+// 4096 buckets; one pass over the entries finds every entry's bucket and
+// counts; neighbouring buckets are joined into groups of about group_size
+// entries; a second pass moves the keys into their groups; each group is
+// sorted in LDS by one workgroup, so the result does not depend on the order
+// in which the second pass placed the entries.  Skewed rows and repeated pairs
+// need no special case: splitters are whole keys.
+//
+// Why not a radix sort of the key: it takes a pass of key and payload over
+// memory per byte of row bits + column bits, and the row pointer's bincount on
+// top (82 us of same-line atomics for 1.8M entries); here each entry moves
+// once.  Bound by LDS traffic of the group sorts and the latency of its short
+// launches rather than by bytes: 1.8M entries in 125 us (64-bit radix sort,
+// index gathers, range reductions and bincount took 550 us).
+//
+// Bucket sizes vary with the sample (gamma distributed, four samples each).
+// A group beyond kCooLargeCap entries, 8 times the mean at the size limit, is
+// reported in *flags, and the caller sorts by other means.
+#include "fs_host.hpp"
+
+namespace fs {
+
+constexpr int kCooTarget = 768;      // entries per bucket aimed at
+constexpr int kCooMaxBuckets = 4096;
+constexpr int kCooOver = 4;          // sampled entries per bucket
+constexpr int kCooItems = 8;         // entries per thread in the LDS sort
+constexpr int kCooSmallCap = 4096;   // group sizes of the two LDS sorts
+constexpr int kCooLargeCap = 8192;
+constexpr int kCooMinGroup = 512;    // entries per group aimed at
+constexpr int kCooMaxGroup = 2048;
+constexpr int kCooMaxGroups = 2048;
+constexpr int kCooTile = 8192;       // entries per workgroup of the two passes
+constexpr int kCooBlock = 1024;
+constexpr int64_t kCooMaxNnz = (int64_t)kCooMaxGroups * kCooMaxGroup;
+
+constexpr int kCooBadRow = 1, kCooBadCol = 2, kCooOverflow = 4;
+
+struct CooWork {
+  uint64_t* sample;     // [kCooOver * kCooMaxBuckets]
+  uint64_t* splitters;  // [kCooMaxBuckets]
+  uint32_t* counts;     // [kCooMaxBuckets]
+  uint16_t* group_of;   // [kCooMaxBuckets]
+  uint32_t* starts;     // [kCooMaxGroups + 1] first entry of each group
+  uint32_t* cursor;     // [kCooMaxGroups]
+  uint32_t* large;      // [kCooMaxGroups + 1]: count, then group ids
+  uint64_t* keys;       // [nnz] by group
+  int32_t* rows;        // [nnz] sorted rows
+  uint16_t* bucket;     // [nnz] bucket of each input entry
+};
+
+struct CooShape {
+  int64_t nnz, n_rows, n_cols;
+  int col_shift, row_shift;  // key = row << row_shift | column << col_shift | position
+  int n_buckets, n_samples, n_groups, group_size;
+};
+
+static int bits_for(int64_t n) {  // bits of 0 .. n - 1
+  int b = 0;
+  while (b < 63 && ((int64_t)1 << b) < n) ++b;
+  return b;
+}
+
+// False where the packed key or the size does not fit.
+static bool coo_shape(CooShape* s, int64_t nnz, int64_t n_rows, int64_t n_cols) {
+  if (nnz < 1 || nnz > kCooMaxNnz || n_rows < 0 || n_cols < 0 || n_rows > INT32_MAX || n_cols > INT32_MAX)
+    return false;
+  s->nnz = nnz;
+  s->n_rows = n_rows;
+  s->n_cols = n_cols;
+  s->col_shift = bits_for(nnz);
+  s->row_shift = s->col_shift + bits_for(n_cols);
+  if (s->row_shift + bits_for(n_rows) > 64 || s->row_shift > 63) return false;
+  const int64_t nb = (nnz + kCooTarget - 1) / kCooTarget;
+  s->n_buckets = (int)(nb > kCooMaxBuckets ? kCooMaxBuckets : nb);
+  s->n_samples = s->n_buckets == 1 ? 0 : s->n_buckets * kCooOver;
+  // about 1024 groups (four per CU, all resident), within the size limits
+  int64_t g = nnz / 1024;
+  g = g < kCooMinGroup ? kCooMinGroup : g > kCooMaxGroup ? kCooMaxGroup : g;
+  s->group_size = (int)g;
+  s->n_groups = (int)((nnz - 1) / g + 1);
+  return true;
+}
+
+// Carves the workspace (base may be null: only the size is wanted).
+static int64_t coo_carve(CooWork* w, char* base, int64_t nnz) {
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) {
+    char* p = base ? base + at : nullptr;
+    at += (bytes + 255) / 256 * 256;
+    return p;
+  };
+  w->sample = reinterpret_cast<uint64_t*>(take(8 * kCooOver * kCooMaxBuckets));
+  w->splitters = reinterpret_cast<uint64_t*>(take(8 * kCooMaxBuckets));
+  w->counts = reinterpret_cast<uint32_t*>(take(4 * kCooMaxBuckets));
+  w->group_of = reinterpret_cast<uint16_t*>(take(2 * kCooMaxBuckets));
+  w->starts = reinterpret_cast<uint32_t*>(take(4 * (kCooMaxGroups + 1)));
+  w->cursor = reinterpret_cast<uint32_t*>(take(4 * kCooMaxGroups));
+  w->large = reinterpret_cast<uint32_t*>(take(4 * (kCooMaxGroups + 1)));
+  w->keys = reinterpret_cast<uint64_t*>(take(8 * nnz));
+  w->rows = reinterpret_cast<int32_t*>(take(4 * nnz));
+  w->bucket = reinterpret_cast<uint16_t*>(take(2 * nnz));
+  return at;
+}
+
+// Out-of-range rows and columns give some key (they are flagged by coo_count
+// and the outputs are not used): any 64-bit value sorts.
+template <typename I>
+__device__ __forceinline__ uint64_t coo_key(const CooShape& s, I row, I col, int64_t e) {
+  return ((uint64_t)row << s.row_shift) | ((uint64_t)col << s.col_shift) | (uint64_t)e;
+}
+
+// Sample i: from the i-th of equal ranges of the input, at a hashed place
+// inside it.  Also clears the counters of the passes that follow.
+template <typename I>
+__global__ __launch_bounds__(256) void coo_sample(const I* __restrict__ row,
+                                                  const I* __restrict__ col, CooShape s, CooWork w,
+                                                  int64_t* flags) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < s.n_buckets) w.counts[i] = 0;
+  if (i == 0) {
+    w.large[0] = 0;
+    *flags = 0;
+  }
+  if (i >= s.n_samples) return;
+  const int64_t a = (int64_t)i * s.nnz / s.n_samples, z = (int64_t)(i + 1) * s.nnz / s.n_samples;
+  uint32_t h = (uint32_t)i * 2654435761u;
+  h = (h ^ (h >> 15)) * 2246822519u;
+  const int64_t e = a + (int64_t)((h ^ (h >> 13)) % (uint32_t)(z - a));
+  w.sample[i] = coo_key(s, row[e], col[e], e);
+}
+
+// Splitters: every workgroup holds the whole sample in LDS and ranks 32 of its
+// members by counting the smaller ones, 32 slices of the sample in parallel;
+// the members of rank kCooOver * k are the splitters (keys are distinct).
+__global__ __launch_bounds__(kCooBlock) void coo_splitters(CooShape s, CooWork w) {
+  extern __shared__ uint64_t sample[];
+  __shared__ int rank[32];
+  const int t = threadIdx.x, n = s.n_samples;
+  for (int i = t; i < n; i += kCooBlock) sample[i] = w.sample[i];
+  if (t < 32) rank[t] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * 32 + (t & 31);
+  const int per = (n + 31) / 32, k0 = (t >> 5) * per;
+  const int k1 = k0 + per < n ? k0 + per : n;
+  const uint64_t mine = sample[i < n ? i : 0];
+  int below = 0, k = k0;
+  for (; k + 8 <= k1; k += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) below += sample[k + u] < mine;
+  for (; k < k1; ++k) below += sample[k] < mine;
+  if (i < n && below) atomicAdd(&rank[t & 31], below);
+  __syncthreads();
+  if (t < 32 && i < n) {
+    const int r = rank[t];
+    if (r > 0 && r % kCooOver == 0) w.splitters[r / kCooOver - 1] = mine;
+  }
+}
+
+// Bucket of every entry (the number of splitters <= its key), bucket sizes,
+// and the range checks.
+template <typename I>
+__global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row,
+                                                       const I* __restrict__ col, CooShape s,
+                                                       CooWork w, int64_t* flags) {
+  __shared__ uint64_t split[kCooMaxBuckets];
+  __shared__ uint32_t hist[kCooMaxBuckets];
+  const int t = threadIdx.x;
+  for (int b = t; b < s.n_buckets; b += kCooBlock) {
+    hist[b] = 0;
+    if (b < s.n_buckets - 1) split[b] = w.splitters[b];
+  }
+  const int64_t e0 = (int64_t)blockIdx.x * kCooTile + t;
+  constexpr int kU = kCooTile / kCooBlock;
+  I r[kU], c[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
+    r[u] = row[e];
+    c[u] = col[e];
+  }
+  __syncthreads();
+  int bad = 0;
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int64_t e = e0 + u * kCooBlock;
+    if (e >= s.nnz) break;
+    bad |= ((int64_t)r[u] < 0 || (int64_t)r[u] >= s.n_rows ? kCooBadRow : 0) |
+           ((int64_t)c[u] < 0 || (int64_t)c[u] >= s.n_cols ? kCooBadCol : 0);
+    const uint64_t key = coo_key(s, r[u], c[u], e);
+    int lo = 0, hi = s.n_buckets - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (split[mid] <= key) lo = mid + 1; else hi = mid;
+    }
+    w.bucket[e] = (uint16_t)lo;
+    atomicAdd(&hist[lo], 1u);
+  }
+  if (bad) atomicOr(reinterpret_cast<unsigned long long*>(flags), (unsigned long long)bad);
+  __syncthreads();
+  for (int b = t; b < s.n_buckets; b += kCooBlock)
+    if (hist[b]) atomicAdd(&w.counts[b], hist[b]);
+}
+
+// Groups: bucket b belongs to group (entries before b) / group_size, so a
+// group holds neighbouring buckets of group_size entries and at most one
+// bucket more; starts of the groups (groups that begin no bucket are empty).
+__global__ __launch_bounds__(kCooBlock) void coo_groups(CooShape s, CooWork w) {
+  __shared__ uint32_t part[kCooBlock / kWave];
+  __shared__ uint32_t start[kCooMaxGroups + 1];
+  const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  constexpr int kPer = kCooMaxBuckets / kCooBlock;
+  for (int g = t; g <= s.n_groups; g += kCooBlock) start[g] = ~0u;
+  uint32_t c[kPer], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int b = t * kPer + k;
+    c[k] = b < s.n_buckets ? w.counts[b] : 0;
+    sum += c[k];
+  }
+  uint32_t scan = sum;
+#pragma unroll
+  for (int k = 1; k < kWave; k <<= 1) {
+    const uint32_t o = __shfl_up(scan, k);
+    if (lane >= k) scan += o;
+  }
+  if (lane == kWave - 1) part[wv] = scan;
+  __syncthreads();
+  uint32_t at = scan - sum;
+  for (int i = 0; i < wv; ++i) at += part[i];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int b = t * kPer + k;
+    if (b < s.n_buckets) {
+      // a bucket without entries may begin at nnz: it goes to the last group
+      const uint32_t g = at / (uint32_t)s.group_size;
+      const uint32_t grp = g < (uint32_t)s.n_groups ? g : (uint32_t)(s.n_groups - 1);
+      w.group_of[b] = (uint16_t)grp;
+      atomicMin(&start[grp], at);
+      at += c[k];
+    }
+  }
+  __syncthreads();
+  for (int g = t; g <= s.n_groups; g += kCooBlock) {
+    // an empty group starts where the next one that is not empty does
+    uint32_t v = ~0u;
+    for (int h = g; h < s.n_groups && v == ~0u; ++h) v = start[h];
+    if (v == ~0u) v = (uint32_t)s.nnz;
+    w.starts[g] = v;
+    if (g < s.n_groups) w.cursor[g] = v;
+  }
+}
+
+// Moves the keys into their groups: a workgroup reserves its share of every
+// group with one atomic and places its entries there.
+template <typename I>
+__global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ row,
+                                                         const I* __restrict__ col, CooShape s,
+                                                         CooWork w) {
+  __shared__ uint32_t hist[kCooMaxGroups];
+  __shared__ uint16_t group_of[kCooMaxBuckets];
+  const int t = threadIdx.x;
+  for (int g = t; g < s.n_groups; g += kCooBlock) hist[g] = 0;
+  for (int b = t; b < s.n_buckets; b += kCooBlock) group_of[b] = w.group_of[b];
+  const int64_t e0 = (int64_t)blockIdx.x * kCooTile + t;
+  constexpr int kU = kCooTile / kCooBlock;
+  uint64_t key[kU];
+  uint32_t g[kU], r[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
+    key[u] = coo_key(s, row[e], col[e], e);
+    g[u] = w.bucket[e];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    g[u] = group_of[g[u]];
+    if (e0 + u * kCooBlock < s.nnz) r[u] = atomicAdd(&hist[g[u]], 1u);
+  }
+  __syncthreads();
+  for (int k = t; k < s.n_groups; k += kCooBlock) {
+    const uint32_t n = hist[k];
+    if (n) hist[k] = atomicAdd(&w.cursor[k], n);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kU; ++u)  // < nnz: the same entries were counted
+    if (e0 + u * kCooBlock < s.nnz) w.keys[hist[g[u]] + r[u]] = key[u];
+}
+
+template <typename O, int VB> struct CooOut {
+  const char* values;
+  char* out_values;
+  O* out_row;  // or null
+  O* out_col;
+};
+
+template <int VB>
+__device__ __forceinline__ void copy_value(char* dst, const char* src, int64_t i, int64_t j) {
+  if constexpr (VB == 2) reinterpret_cast<uint16_t*>(dst)[i] = reinterpret_cast<const uint16_t*>(src)[j];
+  else if constexpr (VB == 4) reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[j];
+  else if constexpr (VB == 8) reinterpret_cast<uint64_t*>(dst)[i] = reinterpret_cast<const uint64_t*>(src)[j];
+  else {
+    reinterpret_cast<uint64_t*>(dst)[2 * i] = reinterpret_cast<const uint64_t*>(src)[2 * j];
+    reinterpret_cast<uint64_t*>(dst)[2 * i + 1] = reinterpret_cast<const uint64_t*>(src)[2 * j + 1];
+  }
+}
+
+// One LDS slot of padding per thread's items keeps the blocked accesses off
+// each other's banks.
+__device__ __forceinline__ int coo_pad(int i) { return i + i / kCooItems; }
+template <int CAP> constexpr int kCooLds = CAP + CAP / kCooItems;
+
+// Sorts the n <= CAP keys from entry s on in LDS and writes the entries out:
+// every thread sorts eight keys in registers, then runs of 8, 16, ... are
+// merged pairwise, each thread finding its eight outputs by a merge-path
+// search.  n is rounded up to whole threads with keys above all others.
+template <typename O, int VB>
+__device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOut<O, VB>& o,
+                               uint32_t s, int n, uint64_t* key) {
+  constexpr int kN = kCooItems;
+  const int t = threadIdx.x, m = (n + kN - 1) / kN * kN;
+  const bool live = t * kN < m;
+  uint64_t k[kN];
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const int j = t * kN + i;
+      k[i] = j < n ? w.keys[s + j] : ~(uint64_t)0;
+    }
+#pragma unroll
+    for (int r = 0; r < kN; ++r)
+#pragma unroll
+      for (int i = r & 1; i + 1 < kN; i += 2) {
+        const uint64_t a = k[i], b = k[i + 1];
+        k[i] = a < b ? a : b;
+        k[i + 1] = a < b ? b : a;
+      }
+#pragma unroll
+    for (int i = 0; i < kN; ++i) key[coo_pad(t * kN + i)] = k[i];
+  }
+  __syncthreads();
+  for (int run = kN; run < m; run <<= 1) {
+    if (live) {
+      const int out0 = t * kN, a0 = out0 & ~(2 * run - 1), d = out0 - a0;
+      const int la = run < m - a0 ? run : m - a0;  // the last runs may be short
+      const int b0 = a0 + la, lb = run < m - b0 ? run : m - b0;
+      int lo = d > lb ? d - lb : 0, hi = d < la ? d : la;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (key[coo_pad(b0 + d - 1 - mid)] < key[coo_pad(a0 + mid)]) hi = mid; else lo = mid + 1;
+      }
+      int a = lo, b = d - lo;
+      uint64_t ka = a < la ? key[coo_pad(a0 + a)] : ~(uint64_t)0;
+      uint64_t kb = b < lb ? key[coo_pad(b0 + b)] : ~(uint64_t)0;
+#pragma unroll
+      for (int i = 0; i < kN; ++i) {
+        // an exhausted run reads as the largest key, which only the padding
+        // equals: either side then gives the same value
+        if (ka <= kb) {
+          k[i] = ka;
+          ++a;
+          ka = a < la ? key[coo_pad(a0 + a)] : ~(uint64_t)0;
+        } else {
+          k[i] = kb;
+          ++b;
+          kb = b < lb ? key[coo_pad(b0 + b)] : ~(uint64_t)0;
+        }
+      }
+    }
+    __syncthreads();
+    if (live)
+#pragma unroll
+      for (int i = 0; i < kN; ++i) key[coo_pad(t * kN + i)] = k[i];
+    __syncthreads();
+  }
+  const uint64_t pos_mask = ((uint64_t)1 << sh.col_shift) - 1;
+  const uint64_t col_mask = ((uint64_t)1 << (sh.row_shift - sh.col_shift)) - 1;
+  for (int i = t; i < n; i += blockDim.x) {
+    const uint64_t kk = key[coo_pad(i)];
+    const int64_t at = (int64_t)s + i;
+    const int32_t r = (int32_t)(kk >> sh.row_shift);
+    w.rows[at] = r;
+    if (o.out_row) o.out_row[at] = (O)r;
+    o.out_col[at] = (O)(int32_t)((kk >> sh.col_shift) & col_mask);
+    // the position of a valid key; flagged input may hold any bits there
+    const int64_t p = (int64_t)(kk & pos_mask);
+    copy_value<VB>(o.out_values, o.values, at, p < sh.nnz ? p : 0);
+  }
+}
+
+template <typename O, int VB>
+__global__ __launch_bounds__(kCooSmallCap / kCooItems) void coo_sort_small(CooShape sh, CooWork w,
+                                                                           CooOut<O, VB> o,
+                                                                           int64_t* flags) {
+  __shared__ uint64_t key[kCooLds<kCooSmallCap>];
+  const uint32_t s = w.starts[blockIdx.x];
+  const int n = (int)(w.starts[blockIdx.x + 1] - s);
+  if (n > kCooSmallCap) {  // left to coo_sort_large
+    if (threadIdx.x == 0) {
+      if (n > kCooLargeCap)
+        atomicOr(reinterpret_cast<unsigned long long*>(flags), (unsigned long long)kCooOverflow);
+      else
+        w.large[1 + atomicAdd(w.large, 1u)] = blockIdx.x;
+    }
+    return;
+  }
+  coo_sort_group<O, VB>(sh, w, o, s, n, key);
+}
+
+template <typename O, int VB>
+__global__ __launch_bounds__(kCooLargeCap / kCooItems) void coo_sort_large(CooShape sh, CooWork w,
+                                                                           CooOut<O, VB> o) {
+  __shared__ uint64_t key[kCooLds<kCooLargeCap>];
+  const uint32_t n_large = w.large[0];
+  for (uint32_t i = blockIdx.x; i < n_large; i += gridDim.x) {
+    const uint32_t g = w.large[1 + i], s = w.starts[g];
+    coo_sort_group<O, VB>(sh, w, o, s, (int)(w.starts[g + 1] - s), key);
+    __syncthreads();  // the next group reuses the LDS
+  }
+}
+
+// Row pointer of the sorted rows: ptr[r] = entries in rows before r, by binary
+// search (no dependence on gaps between rows).
+template <typename P>
+__global__ __launch_bounds__(256) void coo_row_ptr(const int32_t* __restrict__ rows, int64_t nnz,
+                                                   int64_t n_rows, P* __restrict__ ptr) {
+  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r > n_rows) return;
+  int64_t lo = 0, hi = nnz;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if ((int64_t)rows[mid] < r) lo = mid + 1; else hi = mid;
+  }
+  ptr[r] = (P)lo;
+}
+
+template <typename I, typename O, int VB>
+int coo_run(const CooShape& s, const CooWork& w, const void* values, const I* row, const I* col,
+            void* out_values, O* out_row, O* out_col, int64_t* flags, hipStream_t st) {
+  const unsigned tiles = (unsigned)((s.nnz + kCooTile - 1) / kCooTile);
+  const int first = s.n_samples > s.n_buckets ? s.n_samples : s.n_buckets;
+  coo_sample<I><<<(first + 255) / 256, 256, 0, st>>>(row, col, s, w, flags);
+  if (s.n_buckets > 1)
+    coo_splitters<<<(s.n_samples + 31) / 32, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, w);
+  coo_count<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, flags);
+  coo_groups<<<1, kCooBlock, 0, st>>>(s, w);
+  coo_scatter<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w);
+  const CooOut<O, VB> o{static_cast<const char*>(values), static_cast<char*>(out_values), out_row, out_col};
+  coo_sort_small<O, VB><<<s.n_groups, kCooSmallCap / kCooItems, 0, st>>>(s, w, o, flags);
+  if (s.nnz > kCooSmallCap)
+    coo_sort_large<O, VB><<<s.n_groups < 64 ? s.n_groups : 64, kCooLargeCap / kCooItems, 0, st>>>(s, w, o);
+  return check_launch("fs_coo_sort");
+}
+
+template <typename I, typename O>
+int coo_run_vb(int vb, const CooShape& s, const CooWork& w, const void* values, const void* row,
+               const void* col, void* out_values, void* out_row, void* out_col, int64_t* flags,
+               hipStream_t st) {
+  const I* r = static_cast<const I*>(row);
+  const I* c = static_cast<const I*>(col);
+  O* orow = static_cast<O*>(out_row);
+  O* ocol = static_cast<O*>(out_col);
+  switch (vb) {
+    case 2: return coo_run<I, O, 2>(s, w, values, r, c, out_values, orow, ocol, flags, st);
+    case 4: return coo_run<I, O, 4>(s, w, values, r, c, out_values, orow, ocol, flags, st);
+    case 8: return coo_run<I, O, 8>(s, w, values, r, c, out_values, orow, ocol, flags, st);
+    default: return coo_run<I, O, 16>(s, w, values, r, c, out_values, orow, ocol, flags, st);
+  }
+}
+
+}  // namespace fs
+
+using namespace fs;
+
+extern "C" int64_t fs_coo_sort_workspace(int64_t nnz, int64_t n_rows, int64_t n_cols) {
+  CooShape s;
+  CooWork w;
+  return coo_shape(&s, nnz, n_rows, n_cols) ? coo_carve(&w, nullptr, nnz) : 0;
+}
+
+extern "C" int fs_coo_sort(int32_t value_bytes, const void* values, int32_t index_type,
+                           const void* row, const void* col, int64_t nnz, int64_t n_rows,
+                           int64_t n_cols, void* out_values, int32_t out_index_type, void* out_row,
+                           void* out_col, int32_t ptr_type, void* out_ptr, void* workspace,
+                           int64_t workspace_bytes, int64_t* flags, void* stream) {
+  const char* who = "fs_coo_sort";
+  if (value_bytes != 2 && value_bytes != 4 && value_bytes != 8 && value_bytes != 16)
+    return fail(FS_ERR_TYPE, "%s: values must have 2, 4, 8 or 16 bytes", who);
+  if ((index_type != FS_I32 && index_type != FS_I64) ||
+      (out_index_type != FS_I32 && out_index_type != FS_I64) ||
+      (ptr_type != FS_I32 && ptr_type != FS_I64))
+    return fail(FS_ERR_TYPE, "%s: index types must be FS_I32 or FS_I64", who);
+  if (nnz < 1 || n_rows < 0 || n_cols < 0) return fail(FS_ERR_VALUE, "%s: bad size", who);
+  CooShape s;
+  if (!coo_shape(&s, nnz, n_rows, n_cols)) return fail(FS_ERR_UNSUPPORTED, "%s: too large", who);
+  if (!values || !row || !col || !out_values || !out_col || !out_ptr || !workspace || !flags)
+    return fail(FS_ERR_VALUE, "%s: null pointer", who);
+  CooWork w;
+  if (workspace_bytes < coo_carve(&w, static_cast<char*>(workspace), nnz))
+    return fail(FS_ERR_VALUE, "%s: workspace too small", who);
+  hipStream_t st = as_stream(stream);
+  int rc;
+  if (index_type == FS_I32)
+    rc = out_index_type == FS_I32
+             ? coo_run_vb<int32_t, int32_t>(value_bytes, s, w, values, row, col, out_values, out_row, out_col, flags, st)
+             : coo_run_vb<int32_t, int64_t>(value_bytes, s, w, values, row, col, out_values, out_row, out_col, flags, st);
+  else
+    rc = out_index_type == FS_I32
+             ? coo_run_vb<int64_t, int32_t>(value_bytes, s, w, values, row, col, out_values, out_row, out_col, flags, st)
+             : coo_run_vb<int64_t, int64_t>(value_bytes, s, w, values, row, col, out_values, out_row, out_col, flags, st);
+  if (rc) return rc;
+  const unsigned blocks = (unsigned)((n_rows + 256) / 256);
+  if (ptr_type == FS_I32)
+    coo_row_ptr<int32_t><<<blocks, 256, 0, st>>>(w.rows, nnz, n_rows, static_cast<int32_t*>(out_ptr));
+  else
+    coo_row_ptr<int64_t><<<blocks, 256, 0, st>>>(w.rows, nnz, n_rows, static_cast<int64_t*>(out_ptr));
+  return check_launch(who);
+}

@@ -18,6 +18,8 @@ import time
 
 import torch
 
+from .. import _lib
+from ..rowsplit import RowSplitPlan, default_spmm_schedule
 from ..sortkey import stable_order
 from ._common import SUPPORTED_INDEX_DTYPES, _INDEX_LIMIT_INT32
 from .spmm_csr import SUPPORTED_SPMM_VALUE_DTYPES, _select_spmm_alg1_warp_and_factor
@@ -30,8 +32,9 @@ def _normalize_spmm_coo_route(route):
     return route
 
 
-def _prepare_spmm_coo_inputs(data, row, col, B, shape):
-    """Checks of spmm_coo.py:312-371, in the same order with the same messages."""
+def _check_spmm_coo_arrays(data, row, col, B, shape):
+    """The host-side checks of spmm_coo.py:312-345, in the same order with the
+    same messages."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
     if data.ndim != 1 or row.ndim != 1 or col.ndim != 1:
@@ -58,10 +61,15 @@ def _prepare_spmm_coo_inputs(data, row, col, B, shape):
         raise TypeError("row dtype must be torch.int32 or torch.int64")
     if col.dtype not in SUPPORTED_INDEX_DTYPES:
         raise TypeError("col dtype must be torch.int32 or torch.int64")
-    nnz = data.numel()
-    if nnz > _INDEX_LIMIT_INT32:
+    if data.numel() > _INDEX_LIMIT_INT32:
         raise ValueError("nnz exceeds the int32 range supported by the Triton COO kernel")
-    if nnz > 0:
+    return n_rows, n_cols
+
+
+def _prepare_spmm_coo_inputs(data, row, col, B, shape):
+    """Checks of spmm_coo.py:312-371, in the same order with the same messages."""
+    n_rows, n_cols = _check_spmm_coo_arrays(data, row, col, B, shape)
+    if data.numel() > 0:
         min_row, max_row = int(row.min().item()), int(row.max().item())
         min_col, max_col = int(col.min().item()), int(col.max().item())
         if min_row < 0 or max_row >= n_rows:
@@ -107,16 +115,56 @@ def _sorted_csr(data, row, col, n_rows):
     return data[order].contiguous(), col[order].contiguous(), indptr
 
 
+def _native_spmm_coo_csr(data, row, col, B, shape):
+    """The entries in CSR order with their row-split plan, by fs_coo_sort and
+    fs_csr_analyze_split with one host read for the index checks and the
+    lists: (values, columns, row pointer, plan), or None where the sort does not
+    apply.  The sort orders equal (row, col) pairs by input position, as
+    _sorted_csr does."""
+    from .spmm_csr import _spmm_default_accumulate
+    n_rows, n_cols = _check_spmm_coo_arrays(data, row, col, B, shape)
+    nnz, n_dense, device = data.numel(), int(B.shape[1]), data.device
+    if not _lib.coo_sort_applies(nnz, n_rows, n_cols):
+        return None
+    index = torch.promote_types(row.dtype, col.dtype)
+    sch = default_spmm_schedule(n_rows, nnz, n_dense)
+    lists = _lib.split_lists(nnz, n_rows, sch.short_max, sch.chunk_nnz, device)
+    d, _, c, indptr = _lib.coo_sort(
+        data.contiguous(), row.to(index).contiguous(), col.to(index).contiguous(), n_rows, n_cols,
+        lists[0][_lib.FS_STATS_LEN + 1:], index_dtype=torch.int32, want_rows=False,
+        ptr_dtype=torch.int32)
+    _, long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, _, bad = _lib.analyze_split(
+        _lib.make_csr(d, c, indptr, n_rows, n_cols), device, sch.short_max, sch.chunk_nnz, False,
+        lists)
+    if bad & _lib.COO_BAD_ROW:
+        raise IndexError("row indices out of range for n_rows")
+    if bad & _lib.COO_BAD_COL:
+        raise IndexError("col indices out of range for n_cols")
+    if bad:
+        return None
+    plan = RowSplitPlan.listed(sch, _spmm_default_accumulate(data.dtype), data.dtype, device,
+                               long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks)
+    return d, c, indptr, plan
+
+
 def _run_spmm_coo_route(data, row, col, B, shape, block_n=None, block_nnz=256, out=None,
                         return_time=False, route="rowrun"):
-    from .spmm_csr import flagsparse_spmm_csr
+    from .spmm_csr import _hip_spmm_csr_impl, flagsparse_spmm_csr
     route = _normalize_spmm_coo_route(route)
     if block_n is not None and block_n <= 0:
         raise ValueError("block_n must be positive when provided")
     if block_nnz is not None and block_nnz <= 0:
         raise ValueError("block_nnz must be positive when provided")
-    data, krow, kcol, B, n_rows, n_cols, n_dense = _prepare_spmm_coo_inputs(data, row, col, B,
-                                                                           shape)
+    t0 = None
+    if return_time and torch.cuda.is_available():
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+    native = _native_spmm_coo_csr(data, row, col, B, shape)
+    if native is None:
+        data, krow, kcol, B, n_rows, n_cols, n_dense = _prepare_spmm_coo_inputs(data, row, col, B,
+                                                                               shape)
+    else:
+        n_rows, n_cols, n_dense = int(shape[0]), int(shape[1]), int(B.shape[1])
     _resolve_spmm_coo_launch_config(n_dense, data.numel(), block_n=block_n, block_nnz=block_nnz)
     if out is not None:
         if not out.is_cuda:
@@ -125,12 +173,13 @@ def _run_spmm_coo_route(data, row, col, B, shape, block_n=None, block_nnz=256, o
             raise ValueError("out must be on the same CUDA device as the inputs")
         if tuple(out.shape) != (n_rows, n_dense) or out.dtype != data.dtype:
             raise ValueError("out shape/dtype must match result")
-    t0 = None
-    if return_time:
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-    d, c, indptr = _sorted_csr(data, krow, kcol, n_rows)
-    C = flagsparse_spmm_csr(d, c, indptr, B, (n_rows, n_cols))
+    if native is None:
+        d, c, indptr = _sorted_csr(data, krow, kcol, n_rows)
+        C = flagsparse_spmm_csr(d, c, indptr, B, (n_rows, n_cols))
+    else:
+        d, c, indptr, plan = native
+        C = _hip_spmm_csr_impl(d, c, indptr, B.contiguous(), n_rows, n_dense, block_n, block_nnz,
+                               n_cols=n_cols, plan=plan)
     elapsed_ms = None
     if return_time:
         torch.cuda.synchronize()

@@ -209,7 +209,8 @@ def _spmm_call_inputs(data, indices, indptr, B, shape):
     data, cols, indptr, n_rows, n_cols = _check_spmm_csr_arrays(data, indices, indptr, shape)
     n_dense = int(B.shape[1])
     sch = default_spmm_schedule(n_rows, data.numel(), n_dense)
-    (stats, long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed) = _lib.analyze_split(
+    (stats, long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed,
+     _) = _lib.analyze_split(
         _lib.make_csr(data, cols, indptr, n_rows, n_cols), data.device, sch.short_max,
         sch.chunk_nnz, cols.dtype == torch.int64)
     _check_spmm_csr_stats(stats, data.numel(), n_cols)

@@ -19,6 +19,7 @@ import time
 
 import torch
 
+from .. import _lib
 from ._common import SUPPORTED_INDEX_DTYPES, _INDEX_LIMIT_INT32, _is_complex_dtype
 
 SUPPORTED_SPMV_COO_VALUE_DTYPES = (torch.float32, torch.float64, torch.complex64,
@@ -69,13 +70,15 @@ def _normalize_spmv_coo_index_fallback_policy(index_fallback_policy):
     return policy
 
 
+_SEGS_ON_READ = object()
+
+
 class PreparedCoo:
     """Sorted COO + row-run bounds ``seg_starts`` (spmv_coo.py:77-129), plus
     the row pointer of the sorted entries for the CSR kernels."""
 
-    __slots__ = ("data", "row", "col", "shape", "n_rows", "n_cols", "nnz", "seg_starts",
-                 "n_segs", "use_seg_kernel", "op", "transpose", "index_fallback_policy",
-                 "index_fallback_applied", "index_fallback_reason", "_csr")
+    __slots__ = ("data", "row", "col", "shape", "n_rows", "n_cols", "nnz", "_seg_starts", "use_seg_kernel", "op", "transpose", "index_fallback_policy",
+                 "index_fallback_applied", "index_fallback_reason", "_csr", "_ordered")
 
     def __init__(self, data, row, col, shape, seg_starts=None, transpose=False, op=None,
                  index_fallback_policy="auto", index_fallback_applied=False,
@@ -86,19 +89,36 @@ class PreparedCoo:
         self.shape = (int(shape[0]), int(shape[1]))
         self.n_rows, self.n_cols = self.shape
         self.nnz = int(data.numel())
-        self.seg_starts = seg_starts
+        self._seg_starts = seg_starts
         if seg_starts is None:
-            self.n_segs = 0
             self.use_seg_kernel = False
+        elif seg_starts is _SEGS_ON_READ:
+            self.use_seg_kernel = self.nnz > 0
         else:
-            self.n_segs = int(seg_starts.numel()) - 1
-            self.use_seg_kernel = self.n_segs > 0
+            self.use_seg_kernel = int(seg_starts.numel()) > 1
         self.op = _normalize_spmv_coo_op(op, transpose=transpose)
         self.transpose = _spmv_coo_op_transposes(self.op)
         self.index_fallback_policy = str(index_fallback_policy).lower()
         self.index_fallback_applied = bool(index_fallback_applied)
         self.index_fallback_reason = index_fallback_reason
         self._csr = None
+        self._ordered = None  # (row pointer, statistics) of the native sort, until _csr_of
+
+    @property
+    def seg_starts(self):
+        """Bounds of the constant-row runs; built on first read where the
+        constructor was told so (no kernel here reads them)."""
+        if self._seg_starts is _SEGS_ON_READ:
+            self._seg_starts = _seg_starts_from_sorted_rows(self.row, self.nnz, self.data.device)
+        return self._seg_starts
+
+    @seg_starts.setter
+    def seg_starts(self, value):
+        self._seg_starts = value
+
+    @property
+    def n_segs(self):
+        return 0 if self.seg_starts is None else int(self.seg_starts.numel()) - 1
 
 
 def _sort_coo_lex(data, row, col, n_cols):
@@ -141,15 +161,34 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
     if col.dtype not in SUPPORTED_INDEX_DTYPES:
         raise TypeError("col dtype must be torch.int32 or torch.int64")
     # both orders are sorted here (deterministic sums); seg_starts only when asked
+    seg = _SEGS_ON_READ if sort_by_row and data.numel() > 0 else None
+    if (_lib.coo_sort_applies(data.numel(), n_rows, n_cols) and row.device == data.device
+            and col.device == data.device):
+        # one native sort that also checks the index ranges, the analysis of
+        # the result behind it, one host read for both
+        index_dtype = torch.promote_types(row.dtype, col.dtype)
+        words = torch.empty(_lib.FS_STATS_LEN + 1, dtype=torch.int64, device=data.device)
+        flags = words[_lib.FS_STATS_LEN:]
+        d, kr, kc, indptr = _lib.coo_sort(
+            data.contiguous(), row.to(index_dtype).contiguous(), col.to(index_dtype).contiguous(),
+            n_rows, n_cols, flags, ptr_dtype=torch.int32)
+        _lib.analyze_device(_lib.make_csr(d, kc, indptr, n_rows, n_cols), data.device, words)
+        stats = words.cpu().tolist()
+        bad = stats.pop()
+        if bad & _lib.COO_BAD_ROW:
+            raise IndexError("row indices out of range")
+        if bad & _lib.COO_BAD_COL:
+            raise IndexError("col indices out of range")
+        if bad == 0:
+            return d, kr, kc, seg, (indptr, words[:_lib.FS_STATS_LEN], stats)
     data, kr, kc = _sort_coo_lex(data, row, col, n_cols)
-    seg = _seg_starts_from_sorted_rows(kr, data.numel(), data.device) if sort_by_row else None
     if data.numel() > 0:
         r64, c64 = kr.to(torch.int64), kc.to(torch.int64)
         if int(r64.min().item()) < 0 or int(r64.max().item()) >= n_rows:
             raise IndexError("row indices out of range")
         if int(c64.min().item()) < 0 or int(c64.max().item()) >= n_cols:
             raise IndexError("col indices out of range")
-    return data, kr, kc, seg
+    return data, kr, kc, seg, None
 
 
 def prepare_spmv_coo(data, row, col, shape, sort_by_row=True, transpose=False, op=None,
@@ -167,9 +206,11 @@ def prepare_spmv_coo(data, row, col, shape, sort_by_row=True, transpose=False, o
             data = data.conj()
             if hasattr(data, "resolve_conj"):
                 data = data.resolve_conj()
-    d, kr, kc, seg = _prepare_coo_tensors(data, row, col, shape, sort_by_row)
-    return PreparedCoo(d, kr, kc, shape, seg_starts=seg, transpose=transpose, op=op_code,
-                       index_fallback_policy=index_fallback_policy)
+    d, kr, kc, seg, ordered = _prepare_coo_tensors(data, row, col, shape, sort_by_row)
+    prepared = PreparedCoo(d, kr, kc, shape, seg_starts=seg, transpose=transpose, op=op_code,
+                           index_fallback_policy=index_fallback_policy)
+    prepared._ordered = ordered
+    return prepared
 
 
 def _validate_x_coo(x, prepared):
@@ -193,6 +234,12 @@ def _csr_of(prepared):
     """PreparedCsrSpmv over the sorted entries (row pointer from the rows)."""
     if prepared._csr is None:
         from .spmv_csr import prepare_spmv_csr
+        if prepared._ordered is not None:
+            indptr, stats_dev, stats = prepared._ordered
+            prepared._csr = prepare_spmv_csr(prepared.data, prepared.col, indptr, prepared.shape,
+                                             _analyzed=(stats_dev, stats))
+            prepared._ordered = None
+            return prepared._csr
         counts = torch.bincount(prepared.row.to(torch.int64), minlength=prepared.n_rows)
         ptr_dtype = torch.int32 if prepared.nnz <= _INDEX_LIMIT_INT32 else torch.int64
         indptr = torch.zeros(prepared.n_rows + 1, dtype=torch.int64, device=prepared.data.device)

@@ -262,12 +262,13 @@ def _transpose_csr_for_spmv(data, indices, indptr, shape):
 
 
 def _prepare_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy="auto",
-                             _stats_out=None, _lengths=True):
+                             _stats_out=None, _lengths=True, _analyzed=None):
     """Validation with the reference's checks, order and messages
     (spmv_csr.py:497-551); the device-side checks run as one fs_csr_analyze
     pass.  Returns (data, indices, indptr, n_rows, n_cols, row_lengths,
     max_row_nnz); row_lengths is None when ``_lengths`` is false (a
-    validation-only pass)."""
+    validation-only pass).  ``_analyzed``: (device, host) statistics of an
+    analysis pass that the caller has already run on these arrays."""
     _normalize_spmv_index_fallback_policy(index_fallback_policy)
     if not all(torch.is_tensor(t) for t in (data, indices, indptr)):
         raise TypeError("data, indices, indptr must all be torch.Tensor")
@@ -292,8 +293,12 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy
     indices = indices.contiguous()
     indptr = indptr.contiguous()
     nnz = data.numel()
-    stats_dev = _lib.analyze_device(_lib.make_csr(data, indices, indptr, n_rows, n_cols), data.device)
-    stats = stats_dev.cpu().tolist()
+    if _analyzed is not None:
+        stats_dev, stats = _analyzed
+    else:
+        stats_dev = _lib.analyze_device(_lib.make_csr(data, indices, indptr, n_rows, n_cols),
+                                        data.device)
+        stats = stats_dev.cpu().tolist()
     if _stats_out is not None:
         _stats_out.append((stats_dev, stats))
     if stats[0] != 0:
@@ -327,7 +332,8 @@ def _validate_spmv_x(x, prepared):
 
 
 def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=None,
-                     transpose=False, op=None, index_fallback_policy="auto", schedule=None):
+                     transpose=False, op=None, index_fallback_policy="auto", schedule=None,
+                     _analyzed=None):
     """Validate once and cache metadata (spmv_csr.py:570-649).
 
     ``block_nnz`` / ``max_segments`` are validated and recorded with the
@@ -353,7 +359,7 @@ def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=N
     (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths,
      max_row_nnz) = _prepare_spmv_csr_matrix(data, indices, indptr, shape,
                                              index_fallback_policy=index_fallback_policy,
-                                             _stats_out=stats_out)
+                                             _stats_out=stats_out, _analyzed=_analyzed)
     block_nnz_use = block_nnz
     if max_segments is None:
         max_segments_use = max((max_row_nnz + block_nnz_use - 1) // block_nnz_use, 1)
@@ -689,6 +695,17 @@ def coo_to_csr_for_spmv(data, row, col, shape, assume_sorted=False):
     if assume_sorted or _coo_is_sorted_lex(row64, col64, n_cols):
         row_s, col_s, data_s = row64, col64, data
     else:
+        if (_lib.coo_sort_applies(row.numel(), n_rows, n_cols) and row.is_cuda
+                and row.dtype in SUPPORTED_INDEX_DTYPES and col.dtype in SUPPORTED_INDEX_DTYPES
+                and row.device == data.device and col.device == data.device):
+            flags = torch.empty(1, dtype=torch.int64, device=data.device)
+            dtype = torch.promote_types(row.dtype, col.dtype)
+            data_s, _, col_s, indptr = _lib.coo_sort(
+                data.contiguous(), row.to(dtype).contiguous(), col.to(dtype).contiguous(), n_rows,
+                n_cols, flags, index_dtype=torch.int32, want_rows=False)
+            if int(flags.item()) == 0:
+                return data_s, col_s, indptr
+        # larger, or out-of-range indices (reported by what follows)
         order = torch.argsort(row64 * max(1, n_cols) + col64, stable=True)
         row_s, col_s, data_s = row64[order], col64[order], data[order]
     indptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=data.device)

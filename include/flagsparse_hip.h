@@ -390,6 +390,29 @@ int fs_csr_analyze_split(const fs_csr *A, int64_t *stats, int64_t short_max, int
                          int64_t *long_rows, int64_t *long_chunk_ptr, int64_t cap_long,
                          int32_t *chunk_long, int64_t cap_chunks, int32_t *cols32, void *stream);
 
+/* ---------------------------------------------------------- COO to CSR order */
+/*
+ * Entries (row, col, value) in any order to row-major order: out_col and
+ * out_values hold the entries sorted by (row, column), equal pairs in input
+ * order; out_row (or null) their rows; out_ptr the n_rows + 1 row pointers.
+ * row and col have index_type, out_row and out_col out_index_type, out_ptr
+ * ptr_type; values of value_bytes (2, 4, 8 or 16) are moved as they are.
+ * *flags (device) is set to a sum of 1: a row outside [0, n_rows), 2: a column
+ * outside [0, n_cols), 4: this sort's sample did not suit the entries; the
+ * outputs mean something only if it is 0.  workspace: device memory of
+ * fs_coo_sort_workspace(nnz, n_rows, n_cols) bytes, 256-byte aligned; that is
+ * 0 where the sort does not apply: nnz of 0 or above 2^22, n_rows or n_cols
+ * above 2^31 - 1, or bit widths of nnz, n_rows and n_cols above 64 together.  Replaces the
+ * sort + unique + cumsum preparation of spmv_coo.py:297-327 and
+ * spmv_csr.py:885-912.
+ */
+int64_t fs_coo_sort_workspace(int64_t nnz, int64_t n_rows, int64_t n_cols);
+int fs_coo_sort(int32_t value_bytes, const void *values, int32_t index_type, const void *row,
+                const void *col, int64_t nnz, int64_t n_rows, int64_t n_cols, void *out_values,
+                int32_t out_index_type, void *out_row, void *out_col, int32_t ptr_type,
+                void *out_ptr, void *workspace, int64_t workspace_bytes, int64_t *flags,
+                void *stream);
+
 /* ------------------------------------------- split-precision value storage */
 /*
  * Storage formats for the values of an fp32 matrix (x, y stay fp32; the sum is

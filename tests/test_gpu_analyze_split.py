@@ -42,7 +42,7 @@ def test_lists(name, idx, ptr):
     ip, cols, cd, pd = _matrix(lens, idx, ptr)
     vals = torch.zeros(cols.size, device=DEV)
     csr = _lib.make_csr(vals, cd, pd, lens.size, 1000)
-    stats, rows, cptr, owner, n_long, n_chunks, narrow = _lib.analyze_split(
+    stats, rows, cptr, owner, n_long, n_chunks, narrow, _ = _lib.analyze_split(
         csr, DEV, short, chunk, idx == torch.int64)
     assert stats == _lib.analyze(csr, DEV)
     per = -(-lens // chunk)
