@@ -16,7 +16,7 @@
 // memory per byte of row bits + column bits, and the row pointer's bincount on
 // top (82 us of same-line atomics for 1.8M entries); here each entry moves
 // once.  Bound by LDS traffic of the group sorts and the latency of its short
-// launches rather than by bytes: 1.8M entries in 125 us (64-bit radix sort,
+// launches rather than by bytes: 1.8M entries in 110 us (64-bit radix sort,
 // index gathers, range reductions and bincount took 550 us).
 //
 // Bucket sizes vary with the sample (gamma distributed, four samples each).
@@ -29,12 +29,14 @@ namespace fs {
 constexpr int kCooTarget = 768;      // entries per bucket aimed at
 constexpr int kCooMaxBuckets = 4096;
 constexpr int kCooOver = 4;          // sampled entries per bucket
-constexpr int kCooItems = 8;         // entries per thread in the LDS sort
-constexpr int kCooSmallCap = 4096;   // group sizes of the two LDS sorts
+constexpr int kCooItems = 8;         // entries per thread in the LDS sorts
+constexpr int kCooSmallCap = 3584;   // group sizes of the two sort launches
 constexpr int kCooLargeCap = 8192;
 constexpr int kCooMinGroup = 512;    // entries per group aimed at
 constexpr int kCooMaxGroup = 2048;
 constexpr int kCooMaxGroups = 2048;
+constexpr int kCooBins = 2048;       // bins of the in-group sort
+constexpr int kCooBinMax = 32;       // entries of one bin it takes
 constexpr int kCooTile = 8192;       // entries per workgroup of the two passes
 constexpr int kCooBlock = 1024;
 constexpr int64_t kCooMaxNnz = (int64_t)kCooMaxGroups * kCooMaxGroup;
@@ -135,30 +137,40 @@ __global__ __launch_bounds__(256) void coo_sample(const I* __restrict__ row,
   w.sample[i] = coo_key(s, row[e], col[e], e);
 }
 
-// Splitters: every workgroup holds the whole sample in LDS and ranks 32 of its
-// members by counting the smaller ones, 32 slices of the sample in parallel;
-// the members of rank kCooOver * k are the splitters (keys are distinct).
+// Splitters: every workgroup holds the whole sample in LDS and ranks 64 of its
+// members by counting the smaller ones, two members per lane and 32 slices of
+// the sample in parallel (the LDS reads bound it: every key read serves 128
+// comparisons of a wavefront); the members of rank kCooOver * k are the
+// splitters (keys are distinct).
+constexpr int kCooRanked = 64;
+
 __global__ __launch_bounds__(kCooBlock) void coo_splitters(CooShape s, CooWork w) {
   extern __shared__ uint64_t sample[];
-  __shared__ int rank[32];
-  const int t = threadIdx.x, n = s.n_samples;
+  __shared__ int rank[kCooRanked];
+  const int t = threadIdx.x, n = s.n_samples;  // n: a multiple of kCooOver
   for (int i = t; i < n; i += kCooBlock) sample[i] = w.sample[i];
-  if (t < 32) rank[t] = 0;
+  if (t < kCooRanked) rank[t] = 0;
   __syncthreads();
-  const int i = blockIdx.x * 32 + (t & 31);
-  const int per = (n + 31) / 32, k0 = (t >> 5) * per;
-  const int k1 = k0 + per < n ? k0 + per : n;
-  const uint64_t mine = sample[i < n ? i : 0];
-  int below = 0, k = k0;
-  for (; k + 8 <= k1; k += 8)
+  const int i0 = blockIdx.x * kCooRanked + (t & 31), i1 = i0 + 32;
+  const int quads = n / kCooOver, per = (quads + 31) / 32 * kCooOver;
+  const int k0 = (t >> 5) * per, k1 = k0 + per < n ? k0 + per : n;
+  const uint64_t m0 = sample[i0 < n ? i0 : 0], m1 = sample[i1 < n ? i1 : 0];
+  int b0 = 0, b1 = 0;
+#pragma unroll 2
+  for (int k = k0; k < k1; k += kCooOver)
 #pragma unroll
-    for (int u = 0; u < 8; ++u) below += sample[k + u] < mine;
-  for (; k < k1; ++k) below += sample[k] < mine;
-  if (i < n && below) atomicAdd(&rank[t & 31], below);
+    for (int u = 0; u < kCooOver; ++u) {
+      const uint64_t o = sample[k + u];
+      b0 += o < m0;
+      b1 += o < m1;
+    }
+  if (b0) atomicAdd(&rank[t & 31], b0);
+  if (b1) atomicAdd(&rank[(t & 31) + 32], b1);
   __syncthreads();
-  if (t < 32 && i < n) {
+  const int i = blockIdx.x * kCooRanked + t;
+  if (t < kCooRanked && i < n) {
     const int r = rank[t];
-    if (r > 0 && r % kCooOver == 0) w.splitters[r / kCooOver - 1] = mine;
+    if (r > 0 && r % kCooOver == 0) w.splitters[r / kCooOver - 1] = sample[i];
   }
 }
 
@@ -317,13 +329,11 @@ __device__ __forceinline__ void copy_value(char* dst, const char* src, int64_t i
 __device__ __forceinline__ int coo_pad(int i) { return i + i / kCooItems; }
 template <int CAP> constexpr int kCooLds = CAP + CAP / kCooItems;
 
-// Sorts the n <= CAP keys from entry s on in LDS and writes the entries out:
-// every thread sorts eight keys in registers, then runs of 8, 16, ... are
-// merged pairwise, each thread finding its eight outputs by a merge-path
-// search.  n is rounded up to whole threads with keys above all others.
-template <typename O, int VB>
-__device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOut<O, VB>& o,
-                               uint32_t s, int n, uint64_t* key) {
+// Merge sort of the n keys from entry s on into key[coo_pad(0 .. n - 1)]: every
+// thread sorts eight keys in registers, then runs of 8, 16, ... are merged
+// pairwise, each thread finding its eight outputs by a merge-path search.  n
+// is rounded up to whole threads with keys above all others.
+__device__ void coo_merge_sort(const CooWork& w, uint32_t s, int n, uint64_t* key) {
   constexpr int kN = kCooItems;
   const int t = threadIdx.x, m = (n + kN - 1) / kN * kN;
   const bool live = t * kN < m;
@@ -380,14 +390,135 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
       for (int i = 0; i < kN; ++i) key[coo_pad(t * kN + i)] = k[i];
     __syncthreads();
   }
+}
+
+struct CooBlockStats {
+  uint64_t lo[16], hi[16];
+  uint32_t sum[16], most[16];
+};
+
+// Sorts the n <= CAP keys from entry s on and writes the entries out.  Keys
+// are binned by their leading bits below the group's range (about one key a
+// bin where columns spread evenly inside rows), placed bin by bin, and ranked
+// by counting the smaller keys of their bin.  Groups with a bin of more than
+// kCooBinMax keys (clustered columns) are merge-sorted instead.  1.8M entries:
+// 44 us with the merge sort alone, 35 us in this form (of which about half is
+// the random gather of the values).
+template <int CAP, typename O, int VB>
+__device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOut<O, VB>& o,
+                               uint32_t s, int n, char* smem, CooBlockStats& bs) {
+  constexpr int kT = CAP / kCooItems, kWaves = kT / kWave, kU = kCooItems;
+  uint64_t* key = reinterpret_cast<uint64_t*>(smem);
+  uint32_t* bin = reinterpret_cast<uint32_t*>(smem + 8 * CAP);
+  const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  if (n == 0) return;  // uniform
+  uint64_t k[kU], lo = ~(uint64_t)0, hi = 0;
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int j = t + u * kT;
+    k[u] = w.keys[s + (j < n ? j : 0)];
+  }
+  for (int b = t; b < kCooBins; b += kT) bin[b] = 0;
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {  // past n: key 0 of the group again
+    lo = k[u] < lo ? k[u] : lo;
+    hi = k[u] > hi ? k[u] : hi;
+  }
+#pragma unroll
+  for (int q = 32; q >= 1; q >>= 1) {
+    const uint64_t a = __shfl_xor(lo, q), b = __shfl_xor(hi, q);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  if (lane == 0) {
+    bs.lo[wv] = lo;
+    bs.hi[wv] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    lo = bs.lo[i] < lo ? bs.lo[i] : lo;
+    hi = bs.hi[i] > hi ? bs.hi[i] : hi;
+  }
+  // (hi - lo) >> shift < kCooBins
+  const int width = 64 - (hi > lo ? __builtin_clzll(hi - lo) : 64);
+  constexpr int kBinBits = 11;
+  static_assert(kCooBins == 1 << kBinBits, "bin bits");
+  const int shift = width > kBinBits ? width - kBinBits : 0;
+  uint32_t r[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (t + u * kT < n) r[u] = atomicAdd(&bin[(k[u] - lo) >> shift], 1u);
+  __syncthreads();
+  // exclusive scan of the bins in place; a bin keeps its size in the top bits
+  constexpr int kPer = (kCooBins + kT - 1) / kT;
+  uint32_t c[kPer], sum = 0, most = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int b = t * kPer + i;
+    c[i] = b < kCooBins ? bin[b] : 0;
+    sum += c[i];
+    most = c[i] > most ? c[i] : most;
+  }
+  uint32_t scan = sum;
+#pragma unroll
+  for (int q = 1; q < kWave; q <<= 1) {
+    const uint32_t a = __shfl_up(scan, q), b = __shfl_xor(most, q);
+    if (lane >= q) scan += a;
+    most = b > most ? b : most;
+  }
+  if (lane == kWave - 1) {
+    bs.sum[wv] = scan;
+    bs.most[wv] = most;
+  }
+  __syncthreads();
+  uint32_t at = scan - sum;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    at += i < wv ? bs.sum[i] : 0;
+    most = bs.most[i] > most ? bs.most[i] : most;
+  }
+  const bool binned = most <= (uint32_t)kCooBinMax;  // uniform
+  if (binned) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int b = t * kPer + i;
+      if (b < kCooBins) bin[b] = at | c[i] << 16;  // at <= CAP < 2^16
+      at += c[i];
+    }
+    __syncthreads();
+    uint32_t start[kU], size[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const bool ok = t + u * kT < n;
+      const uint32_t v = ok ? bin[(k[u] - lo) >> shift] : 0;
+      start[u] = v & 0xffffu;
+      size[u] = v >> 16;
+      if (ok) key[start[u] + r[u]] = k[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      r[u] = start[u];
+      for (uint32_t i = 0; i < size[u]; ++i) r[u] += key[start[u] + i] < k[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (t + u * kT < n) key[r[u]] = k[u];
+    __syncthreads();
+  } else {
+    __syncthreads();  // the bins' memory is the merge sort's
+    coo_merge_sort(w, s, n, key);
+  }
   const uint64_t pos_mask = ((uint64_t)1 << sh.col_shift) - 1;
   const uint64_t col_mask = ((uint64_t)1 << (sh.row_shift - sh.col_shift)) - 1;
-  for (int i = t; i < n; i += blockDim.x) {
-    const uint64_t kk = key[coo_pad(i)];
+  for (int i = t; i < n; i += kT) {
+    const uint64_t kk = key[binned ? i : coo_pad(i)];
     const int64_t at = (int64_t)s + i;
-    const int32_t r = (int32_t)(kk >> sh.row_shift);
-    w.rows[at] = r;
-    if (o.out_row) o.out_row[at] = (O)r;
+    const int32_t row = (int32_t)(kk >> sh.row_shift);
+    w.rows[at] = row;
+    if (o.out_row) o.out_row[at] = (O)row;
     o.out_col[at] = (O)(int32_t)((kk >> sh.col_shift) & col_mask);
     // the position of a valid key; flagged input may hold any bits there
     const int64_t p = (int64_t)(kk & pos_mask);
@@ -395,11 +526,16 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
   }
 }
 
+// keys and bins of the binned sort, or the padded keys of the merge sort
+template <int CAP> constexpr int kCooSmem =
+    8 * CAP + 4 * kCooBins > 8 * kCooLds<CAP> ? 8 * CAP + 4 * kCooBins : 8 * kCooLds<CAP>;
+
 template <typename O, int VB>
 __global__ __launch_bounds__(kCooSmallCap / kCooItems) void coo_sort_small(CooShape sh, CooWork w,
                                                                            CooOut<O, VB> o,
                                                                            int64_t* flags) {
-  __shared__ uint64_t key[kCooLds<kCooSmallCap>];
+  __shared__ __align__(8) char smem[kCooSmem<kCooSmallCap>];
+  __shared__ CooBlockStats bs;
   const uint32_t s = w.starts[blockIdx.x];
   const int n = (int)(w.starts[blockIdx.x + 1] - s);
   if (n > kCooSmallCap) {  // left to coo_sort_large
@@ -411,17 +547,18 @@ __global__ __launch_bounds__(kCooSmallCap / kCooItems) void coo_sort_small(CooSh
     }
     return;
   }
-  coo_sort_group<O, VB>(sh, w, o, s, n, key);
+  coo_sort_group<kCooSmallCap, O, VB>(sh, w, o, s, n, smem, bs);
 }
 
 template <typename O, int VB>
 __global__ __launch_bounds__(kCooLargeCap / kCooItems) void coo_sort_large(CooShape sh, CooWork w,
                                                                            CooOut<O, VB> o) {
-  __shared__ uint64_t key[kCooLds<kCooLargeCap>];
+  __shared__ __align__(8) char smem[kCooSmem<kCooLargeCap>];
+  __shared__ CooBlockStats bs;
   const uint32_t n_large = w.large[0];
   for (uint32_t i = blockIdx.x; i < n_large; i += gridDim.x) {
     const uint32_t g = w.large[1 + i], s = w.starts[g];
-    coo_sort_group<O, VB>(sh, w, o, s, (int)(w.starts[g + 1] - s), key);
+    coo_sort_group<kCooLargeCap, O, VB>(sh, w, o, s, (int)(w.starts[g + 1] - s), smem, bs);
     __syncthreads();  // the next group reuses the LDS
   }
 }
@@ -448,7 +585,7 @@ int coo_run(const CooShape& s, const CooWork& w, const void* values, const I* ro
   const int first = s.n_samples > s.n_buckets ? s.n_samples : s.n_buckets;
   coo_sample<I><<<(first + 255) / 256, 256, 0, st>>>(row, col, s, w, flags);
   if (s.n_buckets > 1)
-    coo_splitters<<<(s.n_samples + 31) / 32, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, w);
+    coo_splitters<<<(s.n_samples + kCooRanked - 1) / kCooRanked, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, w);
   coo_count<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, flags);
   coo_groups<<<1, kCooBlock, 0, st>>>(s, w);
   coo_scatter<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w);
