@@ -218,7 +218,8 @@ class RowSplitPlan:
     """
 
     def __init__(self, indptr: torch.Tensor, n_rows: int, value_dtype, schedule: Schedule,
-                 accumulate: int, row_lengths: torch.Tensor | None = None):
+                 accumulate: int, row_lengths: torch.Tensor | None = None,
+                 max_row: int | None = None):
         device = indptr.device
         self.schedule = schedule
         self.accumulate = int(accumulate)
@@ -232,6 +233,15 @@ class RowSplitPlan:
         self.xg_runs = None
         if schedule.tile_nnz > 0 and schedule.tile_mode == _lib.FS_TILE_ENTRIES:
             self._init_entry_tiles(indptr, n_rows, schedule)
+            return
+        if max_row is not None and max_row <= schedule.short_max and schedule.tile_nnz == 0:
+            # no long rows (max_row: the longest, where the caller knows it):
+            # nothing to list, no pass over the row lengths and no host read
+            self.long_rows = torch.empty(0, dtype=torch.int64, device=device)
+            self.long_chunk_ptr = torch.empty(0, dtype=torch.int64, device=device)
+            self.chunk_long = torch.empty(0, dtype=torch.int32, device=device)
+            self.n_long, self.n_chunks = 0, 0
+            self.tile_start, self.n_tiles = None, 0
             return
         if row_lengths is None:
             row_lengths = (indptr[1:].to(torch.int64) - indptr[:-1].to(torch.int64)) if n_rows > 0 \

@@ -23,9 +23,34 @@ from .rowsplit import Schedule, default_spmm_schedule, default_spmv_schedule
 _MODES = ("learned", "default", "exhaustive")
 
 
-def choose_schedule(op, request, data, n_rows, n_cols, stats_dev, indptr=None, indices=None):
+def packaged_selector(op, dtype, device, n_rows, n_cols, nnz):
+    """(Selector, None) for a matrix that the learned mode selects for, else
+    (None, how the fixed rule came to be used)."""
+    if n_rows == 0 or (dtype != torch.float32
+                       and not (op == "spmv" and dtype == torch.float64)):
+        return None, "default"
+    from .selector import load_default
+    sel = None
+    if op == "spmv" and dtype == torch.float64:
+        # the model trained on fp64 timings where one is packaged; else the
+        # fp32-trained one (its features describe only the sparsity structure)
+        sel = load_default(op, device, "f64")
+    if sel is None:
+        sel = load_default(op, device)
+    if sel is None:
+        return None, "default"
+    if not sel.covers(n_rows, n_cols, nnz):
+        # outside the sizes the network was trained on: the fixed rule
+        return None, "default (outside the selector's training range)"
+    return sel, None
+
+
+def choose_schedule(op, request, data, n_rows, n_cols, stats_dev, indptr=None, indices=None,
+                    selected=None):
     """``indptr`` / ``indices``: the matrix's row pointers and columns, which
-    the SpMV fixed rule samples for column locality when x is large."""
+    the SpMV fixed rule samples for column locality when x is large.
+    ``selected``: the variant index where the caller has already run the
+    packaged selector on these statistics."""
     nnz = data.numel()
     if isinstance(request, Schedule):
         return request, "given"
@@ -43,21 +68,11 @@ def choose_schedule(op, request, data, n_rows, n_cols, stats_dev, indptr=None, i
         if op != "spmv":
             raise ValueError("exhaustive schedule search is offered for SpMV")
         return fallback(), "exhaustive"
-    if data.dtype != torch.float32 and not (op == "spmv" and data.dtype == torch.float64):
-        return fallback(), "default"
-    from .selector import load_default
-    sel = None
-    if op == "spmv" and data.dtype == torch.float64:
-        # the model trained on fp64 timings where one is packaged; else the
-        # fp32-trained one (its features describe only the sparsity structure)
-        sel = load_default(op, data.device, "f64")
+    sel, why = packaged_selector(op, data.dtype, data.device, n_rows, n_cols, nnz)
     if sel is None:
-        sel = load_default(op, data.device)
-    if sel is None:
-        return fallback(), "default"
-    if not sel.covers(n_rows, n_cols, nnz):
-        # outside the sizes the network was trained on: the fixed rule
-        return fallback(), "default (outside the selector's training range)"
+        return fallback(), why
+    if selected is not None:
+        return sel.variants[selected], f"learned:{selected}"
     sch, idx = sel.schedule_for(stats_dev, n_rows, n_cols, nnz)
     return sch, f"learned:{idx}"
 

@@ -163,9 +163,11 @@ class Selector:
             return False
         return True
 
-    def select_on_device(self, feats_dev):
-        """Variant index (device int32 tensor) for one feature vector on the device."""
-        choice = torch.empty(1, dtype=torch.int32, device=self.mlp.device)
+    def select_on_device(self, feats_dev, choice=None):
+        """Variant index (device int32 tensor, ``choice`` when given) for one
+        feature vector on the device."""
+        if choice is None:
+            choice = torch.empty(1, dtype=torch.int32, device=self.mlp.device)
         _lib.mlp_select(self.mlp.net, feats_dev, self.mu, self.sd, choice, None, self.mlp.device)
         return choice
 

@@ -20,6 +20,7 @@ import time
 import torch
 
 from .. import _lib
+from ..schedule_choice import packaged_selector
 from ._common import SUPPORTED_INDEX_DTYPES, _INDEX_LIMIT_INT32, _is_complex_dtype
 
 SUPPORTED_SPMV_COO_VALUE_DTYPES = (torch.float32, torch.float64, torch.complex64,
@@ -102,7 +103,9 @@ class PreparedCoo:
         self.index_fallback_applied = bool(index_fallback_applied)
         self.index_fallback_reason = index_fallback_reason
         self._csr = None
-        self._ordered = None  # (row pointer, statistics) of the native sort, until _csr_of
+        # (row pointer, device and host statistics, chosen variant) of the
+        # native sort, until _csr_of
+        self._ordered = None
 
     @property
     def seg_starts(self):
@@ -165,22 +168,29 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
     if (_lib.coo_sort_applies(data.numel(), n_rows, n_cols) and row.device == data.device
             and col.device == data.device):
         # one native sort that also checks the index ranges, the analysis of
-        # the result behind it, one host read for both
+        # the result and the schedule selection behind it, one host read for
+        # the three
         index_dtype = torch.promote_types(row.dtype, col.dtype)
-        words = torch.empty(_lib.FS_STATS_LEN + 1, dtype=torch.int64, device=data.device)
-        flags = words[_lib.FS_STATS_LEN:]
+        words = torch.empty(_lib.FS_STATS_LEN + 2, dtype=torch.int64, device=data.device)
+        stats_dev = words[:_lib.FS_STATS_LEN]
+        flags = words[_lib.FS_STATS_LEN:_lib.FS_STATS_LEN + 1]
         d, kr, kc, indptr = _lib.coo_sort(
             data.contiguous(), row.to(index_dtype).contiguous(), col.to(index_dtype).contiguous(),
             n_rows, n_cols, flags, ptr_dtype=torch.int32)
-        _lib.analyze_device(_lib.make_csr(d, kc, indptr, n_rows, n_cols), data.device, words)
+        _lib.analyze_device(_lib.make_csr(d, kc, indptr, n_rows, n_cols), data.device, stats_dev)
+        sel, _ = packaged_selector("spmv", data.dtype, data.device, n_rows, n_cols, data.numel())
+        if sel is not None:
+            sel.select_on_device(_lib.features(stats_dev, n_rows, n_cols, data.numel(), data.device),
+                                 words[_lib.FS_STATS_LEN + 1:].view(torch.int32))
         stats = words.cpu().tolist()
-        bad = stats.pop()
+        chosen = None if sel is None else stats[-1] & 0xFFFFFFFF  # the word's low half
+        bad = stats[-2]
         if bad & _lib.COO_BAD_ROW:
             raise IndexError("row indices out of range")
         if bad & _lib.COO_BAD_COL:
             raise IndexError("col indices out of range")
         if bad == 0:
-            return d, kr, kc, seg, (indptr, words[:_lib.FS_STATS_LEN], stats)
+            return d, kr, kc, seg, (indptr, stats_dev, stats[:_lib.FS_STATS_LEN], chosen)
     data, kr, kc = _sort_coo_lex(data, row, col, n_cols)
     if data.numel() > 0:
         r64, c64 = kr.to(torch.int64), kc.to(torch.int64)
@@ -235,9 +245,9 @@ def _csr_of(prepared):
     if prepared._csr is None:
         from .spmv_csr import prepare_spmv_csr
         if prepared._ordered is not None:
-            indptr, stats_dev, stats = prepared._ordered
+            indptr, *analyzed = prepared._ordered
             prepared._csr = prepare_spmv_csr(prepared.data, prepared.col, indptr, prepared.shape,
-                                             _analyzed=(stats_dev, stats))
+                                             _analyzed=analyzed)
             prepared._ordered = None
             return prepared._csr
         counts = torch.bincount(prepared.row.to(torch.int64), minlength=prepared.n_rows)

@@ -167,7 +167,8 @@ class PreparedCsrSpmv:
         p = self._plans.get(key)
         if p is None:
             p = RowSplitPlan(self.kernel_indptr, self.n_rows, self.data.dtype, sch, accumulate,
-                             row_lengths=self.row_lengths)
+                             row_lengths=self.row_lengths,
+                             max_row=None if self._stats is None else self.max_row_nnz)
             self._plans[key] = p
         return p
 
@@ -268,7 +269,8 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy
     pass.  Returns (data, indices, indptr, n_rows, n_cols, row_lengths,
     max_row_nnz); row_lengths is None when ``_lengths`` is false (a
     validation-only pass).  ``_analyzed``: (device, host) statistics of an
-    analysis pass that the caller has already run on these arrays."""
+    analysis pass that the caller has already run on these arrays, and the
+    variant its selector chose (or None)."""
     _normalize_spmv_index_fallback_policy(index_fallback_policy)
     if not all(torch.is_tensor(t) for t in (data, indices, indptr)):
         raise TypeError("data, indices, indptr must all be torch.Tensor")
@@ -294,7 +296,7 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape, index_fallback_policy
     indptr = indptr.contiguous()
     nnz = data.numel()
     if _analyzed is not None:
-        stats_dev, stats = _analyzed
+        stats_dev, stats = _analyzed[:2]
     else:
         stats_dev = _lib.analyze_device(_lib.make_csr(data, indices, indptr, n_rows, n_cols),
                                         data.device)
@@ -359,7 +361,8 @@ def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=N
     (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths,
      max_row_nnz) = _prepare_spmv_csr_matrix(data, indices, indptr, shape,
                                              index_fallback_policy=index_fallback_policy,
-                                             _stats_out=stats_out, _analyzed=_analyzed)
+                                             _stats_out=stats_out, _analyzed=_analyzed,
+                                             _lengths=_analyzed is None)
     block_nnz_use = block_nnz
     if max_segments is None:
         max_segments_use = max((max_row_nnz + block_nnz_use - 1) // block_nnz_use, 1)
@@ -369,7 +372,8 @@ def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=N
     else:
         max_segments_use = max_segments
     sch, how = choose_schedule("spmv", schedule, data, n_rows, n_cols, stats_out[0][0],
-                               kernel_indptr, kernel_indices)
+                               kernel_indptr, kernel_indices,
+                               None if _analyzed is None else _analyzed[2])
     if how != "given":  # a library choice runs as what is built for these dtypes
         sch = supported_spmv_schedule(sch, data.dtype, kernel_indices.dtype, data.numel())
     prepared = PreparedCsrSpmv(
