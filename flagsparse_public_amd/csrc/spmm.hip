@@ -296,7 +296,11 @@ __device__ __forceinline__ void mm_accumulate(A (&acc)[VW], const I* __restrict_
 // past the last dense column (colok false) still load their share.  The
 // products are added in entry order, as in mm_accumulate.
 // F fills per round: each lane loads F entries (F * G slots per group), so a
-// row of up to F * G entries needs one fill round trip instead of F.
+// row of up to F * G entries needs one fill round trip instead of F.  The next
+// round's entries are loaded before this round's gathers, and the slots are
+// ordered by LDS-only fences, which do not wait for them: fp64 N = 8, 200,000
+// rows of 24 80.7 -> 73.8 us; bf16 N = 32, 100,000 rows of 34 40.3 -> 37.2 us;
+// rows of one round (1M-row band of 15) unchanged.
 template <int G> constexpr int kMmFill = G <= 8 ? 2 : 1;
 
 template <int VW, int U, int G, typename A, typename V>
@@ -310,32 +314,32 @@ __device__ __forceinline__ void mm_accumulate_group(A (&acc)[VW], int32_t* slot_
   using C = typename A::compute_t;
   constexpr int F = kMmFill<G>;
   static_assert(G % U == 0, "batches of U entries tile the group's G slots");
-  for (int64_t j0 = s; j0 < e; j0 += G * F) {
-    if constexpr (F == 1) {
-      const int64_t jj = j0 + g;
-      slot_col[g] = jj < e ? idx[jj] : 0;
-      slot_val[g] = jj < e ? load_as<C>(val, jj) : zero<C>();
-    } else {
-      // unconditional loads (past e: entry j0 again), then the LDS stores,
-      // so the F loads of a lane are in flight together
-      int32_t fc[F];
-      V fv[F];
+  // lane g's share of the fill from j0 on, unconditional (past e: the fill's
+  // first entry again), so that the loads of a lane are in flight together;
+  // the next fill is loaded before the gathers of this one, so its latency
+  // (the entries stream from memory) passes behind theirs
+  int32_t fc[F];
+  V fv[F];
+  auto fetch = [&](int64_t j0) {
 #pragma unroll
-      for (int f = 0; f < F; ++f) {
-        const int64_t jj = j0 + f * G + g;
-        const int64_t q = jj < e ? jj : j0;
-        fc[f] = idx[q];
-        fv[f] = val[q];
-      }
-#pragma unroll
-      for (int f = 0; f < F; ++f) {
-        slot_col[f * G + g] = fc[f];
-        slot_val[f * G + g] = load_as<C>(fv, f);
-      }
+    for (int f = 0; f < F; ++f) {
+      const int64_t jj = j0 + f * G + g;
+      const int64_t q = jj < e ? jj : j0;
+      fc[f] = idx[q];
+      fv[f] = val[q];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  };
+  if (s < e) fetch(s);
+  for (int64_t j0 = s; j0 < e; j0 += G * F) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      slot_col[f * G + g] = fc[f];
+      slot_val[f * G + g] = load_as<C>(fv, f);
+    }
+    if (j0 + G * F < e) fetch(j0 + G * F);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     const int cnt = e - j0 < G * F ? (int)(e - j0) : G * F;
     if (colok) {
       for (int u0 = 0; u0 < cnt; u0 += U) {
@@ -365,9 +369,9 @@ __device__ __forceinline__ void mm_accumulate_group(A (&acc)[VW], int32_t* slot_
       }
     }
     // the slots are rewritten by the next batch
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   }
 }
 
