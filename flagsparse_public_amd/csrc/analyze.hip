@@ -11,6 +11,7 @@
 namespace fs {
 
 constexpr int kAnBlock = 1024;
+constexpr int kAnRows = 4;  // row pointer pairs in flight per thread
 
 enum {
   ST_PTR0 = 0, ST_PTRN = 1, ST_DEC = 2, ST_CMIN = 3, ST_CMAX = 4, ST_LMAX = 5, ST_LMIN = 6,
@@ -26,50 +27,89 @@ constexpr int ST_SPLIT = FS_STATS_LEN;
 constexpr int kSplitBits = 36;
 
 struct SplitOut {
-  int64_t short_max = 0, chunk_nnz = 0, cap_long = 0, cap_chunks = 0;
+  int64_t short_max = 0, cap_long = 0;
+  uint32_t chunk_nnz = 1, cap_chunks = 0;
   int64_t* long_rows = nullptr;
   int64_t* long_chunk_ptr = nullptr;
   int32_t* chunk_long = nullptr;
   int32_t* cols32 = nullptr;
 };
 
-// Lists the wavefront's long rows (`lg`: row `row` of this lane, length l).
-// Rows of one wavefront take consecutive ordinals; the order of wavefronts is
-// free, and so is the order of rows in the list: a row's chunks are its own
-// and are summed in chunk order wherever they lie.  Row pointers are not
-// validated yet, so every write is bounded by the capacities.
-__device__ __forceinline__ void split_rows(const SplitOut& s, int64_t* st, bool lg, int64_t row,
-                                           int64_t l, int lane) {
-  const uint64_t m = __ballot(lg);
-  if (m == 0) return;  // uniform
-  int64_t per = lg ? (l - 1) / s.chunk_nnz + 1 : 0;
-  if (per > s.cap_chunks) per = s.cap_chunks + 1;
-  int64_t scan = per;  // inclusive over the wavefront
-#pragma unroll
-  for (int k = 1; k < kWave; k <<= 1) {
-    const int64_t o = __shfl_up(scan, k);
-    if (lane >= k) scan += o;
+// Lists the block's long rows among kAnRows rows a thread (`row` + u * stride,
+// long where bit u of `lg` is set).  The rows of a block take consecutive
+// ordinals and chunks, so the counter sees one atomic per block and iteration;
+// same-address atomics serialise, and with one per 64 rows that hold a long row
+// they were most of the pass (both launches: 170,000 power-law rows, 2M 64-bit
+// columns 40.5 -> 18.2 us; 1M such rows, 12M 32-bit columns 175 -> 24.6 us; no
+// long row, 4.5M columns 14.2 -> 14.8 us).  The order of blocks is free, and so
+// is the order of rows in the list: a row's chunks are its own and are summed in
+// chunk order wherever they lie.  Row pointers are not validated yet, so every
+// write is bounded by the capacities.
+//
+// Kept small (rolled loops, lengths read again): where no row is long, the
+// pass pays for this only by the size of its code.
+template <typename P>
+__device__ __forceinline__ void split_rows(const SplitOut& s, int64_t* st, const P* ptr,
+                                           uint32_t lg, int64_t row, int64_t stride, int turn) {
+  // two turns' sums: those of one turn are written again only after the
+  // barrier of the next, when nobody reads them any more
+  __shared__ uint64_t wave_sum[2][kAnBlock / kWave];
+  __shared__ uint64_t block_base;
+  uint64_t* sums = wave_sum[turn & 1];
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  auto chunks = [&](int u) {
+    const int64_t i = row + u * stride, l = (int64_t)ptr[i + 1] - (int64_t)ptr[i];
+    const uint32_t c = (uint32_t)((l < INT32_MAX ? l : INT32_MAX) - 1) / s.chunk_nnz + 1;
+    return c > s.cap_chunks ? s.cap_chunks + 1 : c;
+  };
+  uint64_t own = 0, scan = 0;  // scan: inclusive over the wavefront
+  const bool some = __ballot(lg != 0) != 0;
+  if (some) {
+#pragma unroll 1
+    for (uint32_t m = lg; m; m &= m - 1)
+      own += ((uint64_t)1 << kSplitBits) + chunks(__builtin_ctz(m));
+    scan = own;
+#pragma unroll 1
+    for (int k = 1; k < kWave; k <<= 1) {
+      const uint64_t o = __shfl_up(scan, k);
+      if (lane >= k) scan += o;
+    }
   }
-  const uint64_t total = (uint64_t)__shfl(scan, kWave - 1);
-  uint64_t base = 0;
-  if (lane == 0)
-    base = __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(st + ST_SPLIT),
-                                  ((uint64_t)__popcll(m) << kSplitBits) + total, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
-  base = __shfl(base, 0);
-  const int64_t li = (int64_t)(base >> kSplitBits) + __popcll(m & (((uint64_t)1 << lane) - 1));
-  const int64_t c0 = (int64_t)(base & (((uint64_t)1 << kSplitBits) - 1)) + scan - per;
-  if (lg && li < s.cap_long) {
-    s.long_rows[li] = row;
-    s.long_chunk_ptr[li + 1] = c0 + per;  // where the next ordinal's chunks begin
-    if (per == 1 && c0 < s.cap_chunks) s.chunk_long[c0] = (int32_t)li;
+  if (lane == kWave - 1) sums[wv] = scan;
+  __syncthreads();
+  if (!__ballot(sums[lane % (kAnBlock / kWave)] != 0)) return;  // uniform over the block
+  uint64_t before = 0, total = 0;
+#pragma unroll 1
+  for (int i = 0; i < kAnBlock / kWave; ++i) {
+    before += i < wv ? sums[i] : 0;
+    total += sums[i];
   }
-  // rows of several chunks: the whole wavefront fills each row's chunk list
-  for (uint64_t rest = __ballot(lg && per > 1); rest; rest &= rest - 1) {
-    const int src = __builtin_ctzll(rest);
-    const int64_t n = __shfl(per, src), c = __shfl(c0, src), o = __shfl(li, src);
-    for (int64_t k = lane; k < n; k += kWave)
-      if (o < s.cap_long && c + k < s.cap_chunks) s.chunk_long[c + k] = (int32_t)o;
+  if (threadIdx.x == 0)
+    block_base = __hip_atomic_fetch_add(reinterpret_cast<unsigned long long*>(st + ST_SPLIT), total,
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (!some) return;
+  uint64_t at = block_base + before + scan - own;
+#pragma unroll 1
+  for (int u = 0; u < kAnRows; ++u) {
+    const bool is_long = lg >> u & 1;
+    const uint32_t per = is_long ? chunks(u) : 0;
+    const int64_t li = (int64_t)(at >> kSplitBits);
+    const int64_t c0 = (int64_t)(at & (((uint64_t)1 << kSplitBits) - 1));
+    if (is_long && li < s.cap_long) {
+      s.long_rows[li] = row + u * stride;
+      s.long_chunk_ptr[li + 1] = c0 + per;  // where the next ordinal's chunks begin
+      if (per == 1 && c0 < s.cap_chunks) s.chunk_long[c0] = (int32_t)li;
+    }
+    // rows of several chunks: the whole wavefront fills each row's chunk list
+    for (uint64_t rest = __ballot(is_long && per > 1); rest; rest &= rest - 1) {
+      const int src = __builtin_ctzll(rest);
+      const uint32_t n = __shfl(per, src);
+      const int64_t c = __shfl(c0, src), o = __shfl(li, src);
+      for (uint32_t k = lane; k < n; k += kWave)
+        if (o < s.cap_long && c + k < s.cap_chunks) s.chunk_long[c + k] = (int32_t)o;
+    }
+    at += ((uint64_t)is_long << kSplitBits) + per;
   }
 }
 
@@ -164,18 +204,21 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
   // wavefront totals: rows of length < 0, 0, and above each histogram edge
   int64_t dec = 0, empty = 0, g0 = 0, g4 = 0, g16 = 0, g64 = 0, g256 = 0, g4096 = 0;
   // rows: four row pointer pairs in flight; lanes past the end re-read the
-  // last row and skip it.  The loop is uniform over the wavefront (ballots).
-  constexpr int kRows = 4;
-  for (int64_t w0 = t0 - lane; w0 < n_rows; w0 += kRows * stride) {
-    int64_t len[kRows];
+  // last row and skip it.  The loop is uniform over the wavefront (ballots),
+  // and where long rows are listed over the block (barriers).
+  int turn = 0;
+  for (int64_t w0 = SPLIT ? t0 - threadIdx.x : t0 - lane; w0 < n_rows; w0 += kAnRows * stride) {
+    const int64_t w = SPLIT ? w0 + threadIdx.x : w0 + lane;
+    uint32_t lg = 0;
+    int64_t len[kAnRows];
 #pragma unroll
-    for (int u = 0; u < kRows; ++u) {
-      const int64_t i = w0 + lane + u * stride < n_rows ? w0 + lane + u * stride : n_rows - 1;
+    for (int u = 0; u < kAnRows; ++u) {
+      const int64_t i = w + u * stride < n_rows ? w + u * stride : n_rows - 1;
       len[u] = (int64_t)ptr[i + 1] - (int64_t)ptr[i];
     }
 #pragma unroll
-    for (int u = 0; u < kRows; ++u) {
-      const bool live = w0 + lane + u * stride < n_rows;
+    for (int u = 0; u < kAnRows; ++u) {
+      const bool live = w + u * stride < n_rows;
       const int64_t l = len[u];
       dec += __popcll(__ballot(live && l < 0));
       empty += __popcll(__ballot(live && l == 0));
@@ -191,9 +234,9 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
         sumsq += l * l;
         if (l > 256) longnnz += l;
       }
-      if constexpr (SPLIT)
-        split_rows(split, st, live && l > split.short_max, w0 + lane + u * stride, l, lane);
+      if constexpr (SPLIT) lg |= (uint32_t)(live && l > split.short_max) << u;
     }
+    if constexpr (SPLIT) split_rows(split, st, ptr, lg, w, stride, turn++);
   }
   // columns: only min and max are kept, so a lane past the end re-reads the
   // iteration's first column instead of branching.  16-byte loads (four 32-bit
@@ -315,9 +358,9 @@ extern "C" int fs_csr_analyze_split(const fs_csr* A, int64_t* stats, int64_t sho
     return fail(FS_ERR_VALUE, "%s: null list", who);
   SplitOut s;
   s.short_max = short_max;
-  s.chunk_nnz = chunk_nnz;
+  s.chunk_nnz = (uint32_t)(chunk_nnz < INT32_MAX ? chunk_nnz : INT32_MAX);  // rows are no longer
   s.cap_long = cap_long;
-  s.cap_chunks = cap_chunks;
+  s.cap_chunks = (uint32_t)cap_chunks;
   s.long_rows = long_rows;
   s.long_chunk_ptr = long_chunk_ptr;
   s.chunk_long = chunk_long;
