@@ -7,17 +7,18 @@
 // and one comparison decides.  A stratified sample gives splitters for up to
 // 4096 buckets; one pass over the entries finds every entry's bucket and
 // counts; neighbouring buckets are joined into groups of about group_size
-// entries; a second pass moves the keys into their groups; each group is
-// sorted in LDS by one workgroup, so the result does not depend on the order
-// in which the second pass placed the entries.  Skewed rows and repeated pairs
-// need no special case: splitters are whole keys.
+// entries; a second pass moves the keys and values into their groups; each
+// group is sorted in LDS by one workgroup, so the result does not depend on the
+// order in which the second pass placed the entries.  Skewed rows and repeated
+// pairs need no special case: splitters are whole keys.
 //
 // Why not a radix sort of the key: it takes a pass of key and payload over
 // memory per byte of row bits + column bits, and the row pointer's bincount on
 // top (82 us of same-line atomics for 1.8M entries); here each entry moves
-// once.  Bound by LDS traffic of the group sorts and the latency of its short
-// launches rather than by bytes: 1.8M entries in 110 us (64-bit radix sort,
-// index gathers, range reductions and bincount took 550 us).
+// twice.  Bound by LDS traffic, the latency of its short launches and the
+// atomics with which tiles reserve their places rather than by bytes: 1.8M
+// entries in 89 us (64-bit radix sort, index gathers, range reductions and
+// bincount took 550 us), 4M power-law entries 190 us.
 //
 // Bucket sizes vary with the sample (gamma distributed, four samples each).
 // A group beyond kCooLargeCap entries, 8 times the mean at the size limit, is
@@ -26,7 +27,9 @@
 
 namespace fs {
 
-constexpr int kCooTarget = 768;      // entries per bucket aimed at
+// Entries per bucket aimed at: at 768 a group of 1.8M entries now and then
+// passed kCooSmallCap, and sorting that one took 13 us more.
+constexpr int kCooTarget = 448;
 constexpr int kCooMaxBuckets = 4096;
 constexpr int kCooOver = 4;          // sampled entries per bucket
 constexpr int kCooItems = 8;         // entries per thread in the LDS sorts
@@ -37,6 +40,7 @@ constexpr int kCooMaxGroup = 2048;
 constexpr int kCooMaxGroups = 2048;
 constexpr int kCooBins = 2048;       // bins of the in-group sort
 constexpr int kCooBinMax = 32;       // entries of one bin it takes
+constexpr int kCooTable = 2048;      // leading key bits that narrow the bucket search
 constexpr int kCooTile = 8192;       // entries per workgroup of the two passes
 constexpr int kCooBlock = 1024;
 constexpr int64_t kCooMaxNnz = (int64_t)kCooMaxGroups * kCooMaxGroup;
@@ -59,6 +63,7 @@ struct CooWork {
 struct CooShape {
   int64_t nnz, n_rows, n_cols;
   int col_shift, row_shift;  // key = row << row_shift | column << col_shift | position
+  int table_shift;           // key >> table_shift < kCooTable for rows in range
   int n_buckets, n_samples, n_groups, group_size;
 };
 
@@ -77,7 +82,10 @@ static bool coo_shape(CooShape* s, int64_t nnz, int64_t n_rows, int64_t n_cols) 
   s->n_cols = n_cols;
   s->col_shift = bits_for(nnz);
   s->row_shift = s->col_shift + bits_for(n_cols);
-  if (s->row_shift + bits_for(n_rows) > 64 || s->row_shift > 63) return false;
+  const int bits = s->row_shift + bits_for(n_rows);
+  if (bits > 64 || s->row_shift > 63) return false;
+  s->table_shift = bits > 11 ? bits - 11 : 0;
+  static_assert(kCooTable == 1 << 11, "table bits");
   const int64_t nb = (nnz + kCooTarget - 1) / kCooTarget;
   s->n_buckets = (int)(nb > kCooMaxBuckets ? kCooMaxBuckets : nb);
   s->n_samples = s->n_buckets == 1 ? 0 : s->n_buckets * kCooOver;
@@ -137,56 +145,79 @@ __global__ __launch_bounds__(256) void coo_sample(const I* __restrict__ row,
   w.sample[i] = coo_key(s, row[e], col[e], e);
 }
 
-// Splitters: every workgroup holds the whole sample in LDS and ranks 64 of its
-// members by counting the smaller ones, two members per lane and 32 slices of
-// the sample in parallel (the LDS reads bound it: every key read serves 128
-// comparisons of a wavefront); the members of rank kCooOver * k are the
-// splitters (keys are distinct).
+// Splitters: every workgroup bins the whole sample by its leading key bits in
+// LDS and ranks 64 of its members, 16 lanes counting the smaller keys of the
+// member's bin; the members of rank kCooOver * k are the splitters (keys are
+// distinct).  A bin may hold any part of the sample (skewed rows), hence the
+// many workgroups.  Counting over the
+// whole sample instead took 15 us where this takes 7 (9,400 samples).
 constexpr int kCooRanked = 64;
 
 __global__ __launch_bounds__(kCooBlock) void coo_splitters(CooShape s, CooWork w) {
-  extern __shared__ uint64_t sample[];
-  __shared__ int rank[kCooRanked];
-  const int t = threadIdx.x, n = s.n_samples;  // n: a multiple of kCooOver
-  for (int i = t; i < n; i += kCooBlock) sample[i] = w.sample[i];
-  if (t < kCooRanked) rank[t] = 0;
-  __syncthreads();
-  const int i0 = blockIdx.x * kCooRanked + (t & 31), i1 = i0 + 32;
-  const int quads = n / kCooOver, per = (quads + 31) / 32 * kCooOver;
-  const int k0 = (t >> 5) * per, k1 = k0 + per < n ? k0 + per : n;
-  const uint64_t m0 = sample[i0 < n ? i0 : 0], m1 = sample[i1 < n ? i1 : 0];
-  int b0 = 0, b1 = 0;
-#pragma unroll 2
-  for (int k = k0; k < k1; k += kCooOver)
+  extern __shared__ uint64_t binned[];
+  __shared__ uint32_t bin[kCooTable + 1];
+  __shared__ uint32_t part[kCooBlock / kWave];
+  constexpr int kU = kCooOver * kCooMaxBuckets / kCooBlock;
+  static_assert(kCooTable == 2 * kCooBlock, "two bins a thread");
+  const int t = threadIdx.x, lane = t % kWave, wv = t / kWave, n = s.n_samples;
+  auto bin_of = [&](uint64_t key) {
+    const uint64_t h = key >> s.table_shift;
+    return h < kCooTable ? (int)h : kCooTable - 1;
+  };
+  uint64_t k[kU];
+  uint32_t r[kU];
 #pragma unroll
-    for (int u = 0; u < kCooOver; ++u) {
-      const uint64_t o = sample[k + u];
-      b0 += o < m0;
-      b1 += o < m1;
-    }
-  if (b0) atomicAdd(&rank[t & 31], b0);
-  if (b1) atomicAdd(&rank[(t & 31) + 32], b1);
+  for (int u = 0; u < kU; ++u)
+    if (t + u * kCooBlock < n) k[u] = w.sample[t + u * kCooBlock];
+  bin[t] = bin[t + kCooBlock] = 0;
   __syncthreads();
-  const int i = blockIdx.x * kCooRanked + t;
-  if (t < kCooRanked && i < n) {
-    const int r = rank[t];
-    if (r > 0 && r % kCooOver == 0) w.splitters[r / kCooOver - 1] = sample[i];
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (t + u * kCooBlock < n) r[u] = atomicAdd(&bin[bin_of(k[u])], 1u);
+  __syncthreads();
+  const uint32_t n0 = bin[2 * t], n1 = bin[2 * t + 1];
+  uint32_t scan = n0 + n1;
+#pragma unroll
+  for (int q = 1; q < kWave; q <<= 1) {
+    const uint32_t o = __shfl_up(scan, q);
+    if (lane >= q) scan += o;
   }
+  if (lane == kWave - 1) part[wv] = scan;
+  __syncthreads();
+  uint32_t at = scan - n0 - n1;
+  for (int i = 0; i < wv; ++i) at += part[i];
+  bin[2 * t] = at;
+  bin[2 * t + 1] = at + n0;
+  if (t == 0) bin[kCooTable] = (uint32_t)n;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kU; ++u)
+    if (t + u * kCooBlock < n) binned[bin[bin_of(k[u])] + r[u]] = k[u];
+  __syncthreads();
+  const int i = blockIdx.x * kCooRanked + t / 16;
+  const uint64_t m = w.sample[i < n ? i : 0];
+  const int b = bin_of(m);
+  uint32_t rank = 0;
+  for (uint32_t q = bin[b] + t % 16; q < bin[b + 1]; q += 16) rank += binned[q] < m;
+#pragma unroll
+  for (int q = 1; q < 16; q <<= 1) rank += __shfl_xor(rank, q);
+  rank += bin[b];
+  if (t % 16 == 0 && i < n && rank > 0 && rank % kCooOver == 0)
+    w.splitters[rank / kCooOver - 1] = m;
 }
 
 // Bucket of every entry (the number of splitters <= its key), bucket sizes,
-// and the range checks.
+// and the range checks.  A table over the leading key bits leaves a step or two
+// of the search where rows are filled evenly (3.7M entries, 4096 buckets: 44 ->
+// 21 us; 1.8M: 17 -> 15 us, the rest being atomics).
 template <typename I>
 __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row,
                                                        const I* __restrict__ col, CooShape s,
                                                        CooWork w, int64_t* flags) {
   __shared__ uint64_t split[kCooMaxBuckets];
   __shared__ uint32_t hist[kCooMaxBuckets];
-  const int t = threadIdx.x;
-  for (int b = t; b < s.n_buckets; b += kCooBlock) {
-    hist[b] = 0;
-    if (b < s.n_buckets - 1) split[b] = w.splitters[b];
-  }
+  __shared__ uint16_t table[kCooTable + 1];
+  const int t = threadIdx.x, last = s.n_buckets - 1;
   const int64_t e0 = (int64_t)blockIdx.x * kCooTile + t;
   constexpr int kU = kCooTile / kCooBlock;
   I r[kU], c[kU];
@@ -195,6 +226,21 @@ __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row
     const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
     r[u] = row[e];
     c[u] = col[e];
+  }
+  for (int b = t; b < s.n_buckets; b += kCooBlock) {
+    hist[b] = 0;
+    if (b < last) split[b] = w.splitters[b];
+  }
+  __syncthreads();
+  // splitters in an earlier slot of the table; keys past the table's range
+  // (flagged rows) search from its last slot on
+  for (int h = t; h <= kCooTable; h += kCooBlock) {
+    int lo = 0, hi = last;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (split[mid] >> s.table_shift < (uint64_t)h) lo = mid + 1; else hi = mid;
+    }
+    table[h] = (uint16_t)(h < kCooTable ? lo : last);
   }
   __syncthreads();
   int bad = 0;
@@ -205,7 +251,9 @@ __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row
     bad |= ((int64_t)r[u] < 0 || (int64_t)r[u] >= s.n_rows ? kCooBadRow : 0) |
            ((int64_t)c[u] < 0 || (int64_t)c[u] >= s.n_cols ? kCooBadCol : 0);
     const uint64_t key = coo_key(s, r[u], c[u], e);
-    int lo = 0, hi = s.n_buckets - 1;
+    const uint64_t h = key >> s.table_shift;
+    const int slot = h < kCooTable ? (int)h : kCooTable - 1;
+    int lo = table[slot], hi = table[slot + 1];
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
       if (split[mid] <= key) lo = mid + 1; else hi = mid;
@@ -215,8 +263,12 @@ __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row
   }
   if (bad) atomicOr(reinterpret_cast<unsigned long long*>(flags), (unsigned long long)bad);
   __syncthreads();
-  for (int b = t; b < s.n_buckets; b += kCooBlock)
+  // blocks begin at different buckets, so that they do not queue for one line
+  const int turn = (int)(blockIdx.x * kWave % (unsigned)s.n_buckets);
+  for (int i = t; i < s.n_buckets; i += kCooBlock) {
+    const int b = i + turn < s.n_buckets ? i + turn : i + turn - s.n_buckets;
     if (hist[b]) atomicAdd(&w.counts[b], hist[b]);
+  }
 }
 
 // Groups: bucket b belongs to group (entries before b) / group_size, so a
@@ -268,26 +320,64 @@ __global__ __launch_bounds__(kCooBlock) void coo_groups(CooShape s, CooWork w) {
   }
 }
 
-// Moves the keys into their groups: a workgroup reserves its share of every
-// group with one atomic and places its entries there.
-template <typename I>
+template <typename O, int VB> struct CooOut {
+  const char* values;
+  char* out_values;
+  O* out_row;  // or null
+  O* out_col;
+};
+
+template <int VB> struct CooValue {
+  typedef uint64_t type __attribute__((ext_vector_type(2)));
+  type x;
+};
+template <> struct CooValue<2> { uint16_t x; };
+template <> struct CooValue<4> { uint32_t x; };
+template <> struct CooValue<8> { uint64_t x; };
+
+// Values are aligned to their components only (8 bytes of a 16-byte one).
+template <int VB> __device__ __forceinline__ CooValue<VB> load_value(const char* p, int64_t i) {
+  CooValue<VB> v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p + i * VB, VB < 8 ? VB : VB == 8 ? 4 : 8), VB);
+  return v;
+}
+template <int VB> __device__ __forceinline__ void store_value(char* p, int64_t i, CooValue<VB> v) {
+  __builtin_memcpy(__builtin_assume_aligned(p + i * VB, VB < 8 ? VB : VB == 8 ? 4 : 8), &v, VB);
+}
+
+// Moves the keys and the values into their groups: a workgroup reserves its
+// share of every group with one atomic and places its entries there, brought
+// into group order in LDS first, so that a group's share is one run of a store.
+// Stores from input order to scattered places bound this pass (1.8M entries: 19
+// us for the keys alone, 44 us with 4-byte values; 18.6 and 22 us in runs), and
+// with the values here the sort reads them in order instead of at random.
+// 16-byte values stay where they are: the sort gathers them.  Tiles of 6144 and
+// 4096 entries: 30 and 32 us (more atomics).
+template <typename I, int VB>
 __global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ row,
                                                          const I* __restrict__ col, CooShape s,
-                                                         CooWork w) {
-  __shared__ uint32_t hist[kCooMaxGroups];
-  __shared__ uint16_t group_of[kCooMaxBuckets];
-  const int t = threadIdx.x;
+                                                         CooWork w, const char* __restrict__ values,
+                                                         char* __restrict__ out_values) {
+  __shared__ uint64_t stage[kCooTile];
+  __shared__ uint16_t owner[kCooTile];
+  __shared__ uint32_t hist[kCooMaxGroups];   // entries, then first place of the tile's share
+  __shared__ uint16_t first[kCooMaxGroups];  // first slot in the stage
+  __shared__ uint32_t part[kCooBlock / kWave];
+  uint16_t* group_of = reinterpret_cast<uint16_t*>(stage);  // until the stage is filled
+  const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
   for (int g = t; g < s.n_groups; g += kCooBlock) hist[g] = 0;
   for (int b = t; b < s.n_buckets; b += kCooBlock) group_of[b] = w.group_of[b];
-  const int64_t e0 = (int64_t)blockIdx.x * kCooTile + t;
+  const int64_t tile0 = (int64_t)blockIdx.x * kCooTile, e0 = tile0 + t;
   constexpr int kU = kCooTile / kCooBlock;
   uint64_t key[kU];
+  CooValue<VB> v[kU];
   uint32_t g[kU], r[kU];
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
     key[u] = coo_key(s, row[e], col[e], e);
     g[u] = w.bucket[e];
+    if (VB <= 8) v[u] = load_value<VB>(values, e);
   }
   __syncthreads();
 #pragma unroll
@@ -296,31 +386,55 @@ __global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ r
     if (e0 + u * kCooBlock < s.nnz) r[u] = atomicAdd(&hist[g[u]], 1u);
   }
   __syncthreads();
-  for (int k = t; k < s.n_groups; k += kCooBlock) {
-    const uint32_t n = hist[k];
-    if (n) hist[k] = atomicAdd(&w.cursor[k], n);
+  // slots: exclusive scan of the counts, two groups a thread
+  static_assert(kCooMaxGroups == 2 * kCooBlock, "two groups a thread");
+  const uint32_t n0 = 2 * t < s.n_groups ? hist[2 * t] : 0;
+  const uint32_t n1 = 2 * t + 1 < s.n_groups ? hist[2 * t + 1] : 0;
+  uint32_t scan = n0 + n1;
+#pragma unroll
+  for (int k = 1; k < kWave; k <<= 1) {
+    const uint32_t o = __shfl_up(scan, k);
+    if (lane >= k) scan += o;
   }
+  if (lane == kWave - 1) part[wv] = scan;
+  __syncthreads();
+  uint32_t at = scan - n0 - n1;
+  for (int i = 0; i < wv; ++i) at += part[i];
+  first[2 * t] = (uint16_t)at;
+  first[2 * t + 1] = (uint16_t)(at + n0);
   __syncthreads();
 #pragma unroll
-  for (int u = 0; u < kU; ++u)  // < nnz: the same entries were counted
-    if (e0 + u * kCooBlock < s.nnz) w.keys[hist[g[u]] + r[u]] = key[u];
-}
-
-template <typename O, int VB> struct CooOut {
-  const char* values;
-  char* out_values;
-  O* out_row;  // or null
-  O* out_col;
-};
-
-template <int VB>
-__device__ __forceinline__ void copy_value(char* dst, const char* src, int64_t i, int64_t j) {
-  if constexpr (VB == 2) reinterpret_cast<uint16_t*>(dst)[i] = reinterpret_cast<const uint16_t*>(src)[j];
-  else if constexpr (VB == 4) reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[j];
-  else if constexpr (VB == 8) reinterpret_cast<uint64_t*>(dst)[i] = reinterpret_cast<const uint64_t*>(src)[j];
-  else {
-    reinterpret_cast<uint64_t*>(dst)[2 * i] = reinterpret_cast<const uint64_t*>(src)[2 * j];
-    reinterpret_cast<uint64_t*>(dst)[2 * i + 1] = reinterpret_cast<const uint64_t*>(src)[2 * j + 1];
+  for (int u = 0; u < kU; ++u)
+    if (e0 + u * kCooBlock < s.nnz) {
+      r[u] += first[g[u]];
+      stage[r[u]] = key[u];
+      owner[r[u]] = (uint16_t)g[u];
+    }
+  __syncthreads();
+  // the thread that holds group k's count reserves its places
+  if (n0) hist[2 * t] = atomicAdd(&w.cursor[2 * t], n0) - at;
+  if (n1) hist[2 * t + 1] = atomicAdd(&w.cursor[2 * t + 1], n1) - (at + n0);
+  __syncthreads();
+  const int n = s.nnz - tile0 < kCooTile ? (int)(s.nnz - tile0) : kCooTile;
+  uint32_t to[kU];
+#pragma unroll
+  for (int u = 0; u < kU; ++u) {
+    const int i = t + u * kCooBlock;
+    if (i < n) {
+      to[u] = hist[owner[i]] + i;  // < nnz: the same entries were counted
+      w.keys[to[u]] = stage[i];
+    }
+  }
+  if constexpr (VB <= 8) {
+    __syncthreads();
+    CooValue<VB>* vs = reinterpret_cast<CooValue<VB>*>(stage);
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (e0 + u * kCooBlock < s.nnz) vs[r[u]] = v[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (t + u * kCooBlock < n) store_value<VB>(out_values, to[u], vs[t + u * kCooBlock]);
   }
 }
 
@@ -397,13 +511,39 @@ struct CooBlockStats {
   uint32_t sum[16], most[16];
 };
 
+// at: the sum over the threads before this one; most: the maximum over all.
+template <int WAVES>
+__device__ __forceinline__ void coo_scan(uint32_t sum, uint32_t& most, uint32_t& at, CooBlockStats& bs) {
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  uint32_t scan = sum;
+#pragma unroll
+  for (int q = 1; q < kWave; q <<= 1) {
+    const uint32_t a = __shfl_up(scan, q), b = __shfl_xor(most, q);
+    if (lane >= q) scan += a;
+    most = b > most ? b : most;
+  }
+  if (lane == kWave - 1) {
+    bs.sum[wv] = scan;
+    bs.most[wv] = most;
+  }
+  __syncthreads();
+  at = scan - sum;
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) {
+    at += i < wv ? bs.sum[i] : 0;
+    most = bs.most[i] > most ? bs.most[i] : most;
+  }
+}
+
 // Sorts the n <= CAP keys from entry s on and writes the entries out.  Keys
 // are binned by their leading bits below the group's range (about one key a
 // bin where columns spread evenly inside rows), placed bin by bin, and ranked
-// by counting the smaller keys of their bin.  Groups with a bin of more than
-// kCooBinMax keys (clustered columns) are merge-sorted instead.  1.8M entries:
-// 44 us with the merge sort alone, 35 us in this form (of which about half is
-// the random gather of the values).
+// by counting the smaller keys of their bin.  Where a long row crowds one bin
+// among many short ones, the bins are cut once more by their own ranges (2M
+// power-law entries: 58 + 33 -> 38 + 15 us in the two launches, the rest from
+// the values in place); groups that crowd there too (clustered columns) are
+// merge-sorted.  1.8M even entries: 44 us with the merge sort alone, 34 us
+// binned, 25 us with the values in place.
 template <int CAP, typename O, int VB>
 __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOut<O, VB>& o,
                                uint32_t s, int n, char* smem, CooBlockStats& bs) {
@@ -412,11 +552,14 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
   uint32_t* bin = reinterpret_cast<uint32_t*>(smem + 8 * CAP);
   const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
   if (n == 0) return;  // uniform
+  // values from coo_scatter: read before the barriers, written back after them
+  CooValue<VB> v[kU];
   uint64_t k[kU], lo = ~(uint64_t)0, hi = 0;
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     const int j = t + u * kT;
     k[u] = w.keys[s + (j < n ? j : 0)];
+    if (VB <= 8) v[u] = load_value<VB>(o.out_values, s + (j < n ? j : 0));
   }
   for (int b = t; b < kCooBins; b += kT) bin[b] = 0;
 #pragma unroll
@@ -460,42 +603,65 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
     sum += c[i];
     most = c[i] > most ? c[i] : most;
   }
-  uint32_t scan = sum;
+  uint32_t at;
+  coo_scan<kWaves>(sum, most, at, bs);
 #pragma unroll
-  for (int q = 1; q < kWave; q <<= 1) {
-    const uint32_t a = __shfl_up(scan, q), b = __shfl_xor(most, q);
-    if (lane >= q) scan += a;
-    most = b > most ? b : most;
-  }
-  if (lane == kWave - 1) {
-    bs.sum[wv] = scan;
-    bs.most[wv] = most;
+  for (int i = 0; i < kPer; ++i) {
+    const int b = t * kPer + i;
+    if (b < kCooBins) bin[b] = at | c[i] << 16;  // at <= CAP < 2^16
+    at += c[i];
   }
   __syncthreads();
-  uint32_t at = scan - sum;
+  uint32_t start[kU], size[kU];
 #pragma unroll
-  for (int i = 0; i < kWaves; ++i) {
-    at += i < wv ? bs.sum[i] : 0;
-    most = bs.most[i] > most ? bs.most[i] : most;
+  for (int u = 0; u < kU; ++u) {
+    const uint32_t b = t + u * kT < n ? bin[(k[u] - lo) >> shift] : 0;
+    start[u] = b & 0xffffu;
+    size[u] = b >> 16;
+  }
+  if (most > (uint32_t)kCooBinMax) {  // uniform
+    // second level: a bin of m keys is cut into m equal parts, which the places
+    // of the sorted keys count; then as above
+    uint32_t* part = reinterpret_cast<uint32_t*>(smem);
+    for (int i = t; i < CAP; i += kT) part[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (t + u * kT < n) {
+        const uint64_t in = (k[u] - lo) & (((uint64_t)1 << shift) - 1);
+        const int drop = shift > 32 ? shift - 32 : 0;
+        start[u] += (uint32_t)((in >> drop) * size[u] >> (shift - drop));
+        r[u] = atomicAdd(&part[start[u]], 1u);
+      }
+    __syncthreads();
+    uint32_t d[kU];
+    sum = most = 0;
+#pragma unroll
+    for (int i = 0; i < kU; ++i) {
+      d[i] = part[t * kU + i];
+      sum += d[i];
+      most = d[i] > most ? d[i] : most;
+    }
+    coo_scan<kWaves>(sum, most, at, bs);
+#pragma unroll
+    for (int i = 0; i < kU; ++i) {
+      part[t * kU + i] = at | d[i] << 16;
+      at += d[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t b = t + u * kT < n ? part[start[u]] : 0;
+      start[u] = b & 0xffffu;
+      size[u] = b >> 16;
+    }
+    __syncthreads();
   }
   const bool binned = most <= (uint32_t)kCooBinMax;  // uniform
   if (binned) {
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int b = t * kPer + i;
-      if (b < kCooBins) bin[b] = at | c[i] << 16;  // at <= CAP < 2^16
-      at += c[i];
-    }
-    __syncthreads();
-    uint32_t start[kU], size[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const bool ok = t + u * kT < n;
-      const uint32_t v = ok ? bin[(k[u] - lo) >> shift] : 0;
-      start[u] = v & 0xffffu;
-      size[u] = v >> 16;
-      if (ok) key[start[u] + r[u]] = k[u];
-    }
+    for (int u = 0; u < kU; ++u)
+      if (t + u * kT < n) key[start[u] + r[u]] = k[u];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
@@ -505,7 +671,10 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kU; ++u)
-      if (t + u * kT < n) key[r[u]] = k[u];
+      if (t + u * kT < n) {
+        key[r[u]] = k[u];
+        if (VB <= 8) store_value<VB>(o.out_values, (int64_t)s + r[u], v[u]);
+      }
     __syncthreads();
   } else {
     __syncthreads();  // the bins' memory is the merge sort's
@@ -522,7 +691,7 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
     o.out_col[at] = (O)(int32_t)((kk >> sh.col_shift) & col_mask);
     // the position of a valid key; flagged input may hold any bits there
     const int64_t p = (int64_t)(kk & pos_mask);
-    copy_value<VB>(o.out_values, o.values, at, p < sh.nnz ? p : 0);
+    if (VB > 8 || !binned) store_value<VB>(o.out_values, at, load_value<VB>(o.values, p < sh.nnz ? p : 0));
   }
 }
 
@@ -588,8 +757,8 @@ int coo_run(const CooShape& s, const CooWork& w, const void* values, const I* ro
     coo_splitters<<<(s.n_samples + kCooRanked - 1) / kCooRanked, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, w);
   coo_count<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, flags);
   coo_groups<<<1, kCooBlock, 0, st>>>(s, w);
-  coo_scatter<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w);
   const CooOut<O, VB> o{static_cast<const char*>(values), static_cast<char*>(out_values), out_row, out_col};
+  coo_scatter<I, VB><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, o.values, o.out_values);
   coo_sort_small<O, VB><<<s.n_groups, kCooSmallCap / kCooItems, 0, st>>>(s, w, o, flags);
   if (s.nnz > kCooSmallCap)
     coo_sort_large<O, VB><<<s.n_groups < 64 ? s.n_groups : 64, kCooLargeCap / kCooItems, 0, st>>>(s, w, o);
