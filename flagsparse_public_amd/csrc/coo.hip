@@ -20,6 +20,12 @@
 // entries in 89 us (64-bit radix sort, index gathers, range reductions and
 // bincount took 550 us), 4M power-law entries 190 us.
 //
+// Above 2^22 entries, where groups would outgrow the LDS, the same passes first
+// move the entries into parts of about 1.8M keys (runs of hundreds of entries, at
+// the rate of a copy) and then sort all parts at once, one per grid row, with
+// the parts' sizes read on the device: 4.25M random entries 217 us, 14.4M banded
+// 532 us (with the 64-bit radix sort and its follow-up passes about 2.9 ms).
+//
 // Bucket sizes vary with the sample (gamma distributed, four samples each).
 // A group beyond kCooLargeCap entries, 8 times the mean at the size limit, is
 // reported in *flags, and the caller sorts by other means.
@@ -43,29 +49,53 @@ constexpr int kCooBinMax = 32;       // entries of one bin it takes
 constexpr int kCooTable = 2048;      // leading key bits that narrow the bucket search
 constexpr int kCooTile = 8192;       // entries per workgroup of the two passes
 constexpr int kCooBlock = 1024;
-constexpr int64_t kCooMaxNnz = (int64_t)kCooMaxGroups * kCooMaxGroup;
+constexpr int64_t kCooMaxNnz = (int64_t)kCooMaxGroups * kCooMaxGroup;  // one part
+// Larger inputs are first moved into parts of about this size (kCooMaxBuckets
+// buckets of kCooTarget entries each); a part may be half as large again.
+constexpr int64_t kCooPart = (int64_t)kCooMaxBuckets * kCooTarget;
+constexpr int kCooMaxParts = 64;
+constexpr int kCooMaxSamples = kCooOver * kCooMaxBuckets;
+static_assert(kCooPart * 3 / 2 <= kCooMaxNnz, "part sizes");
 
 constexpr int kCooBadRow = 1, kCooBadCol = 2, kCooOverflow = 4;
 
 struct CooWork {
-  uint64_t* sample;     // [kCooOver * kCooMaxBuckets]
+  uint64_t* sample;     // [kCooMaxSamples]; this and the next five: one per part
   uint64_t* splitters;  // [kCooMaxBuckets]
   uint32_t* counts;     // [kCooMaxBuckets]
   uint16_t* group_of;   // [kCooMaxBuckets]
   uint32_t* starts;     // [kCooMaxGroups + 1] first entry of each group
   uint32_t* cursor;     // [kCooMaxGroups]
-  uint32_t* large;      // [kCooMaxGroups + 1]: count, then group ids
+  uint32_t* large;      // [parts * kCooMaxGroups + 1]: count, then part << 16 | group
   uint64_t* keys;       // [nnz] by group
   int32_t* rows;        // [nnz] sorted rows
   uint16_t* bucket;     // [nnz] bucket of each input entry
+  uint64_t* part_keys;  // [nnz] by part, if there are several (then rows lie here too)
+  char* part_values;    // [8 * nnz] likewise
+  uint32_t* part_start; // [parts + 1]
 };
 
 struct CooShape {
   int64_t nnz, n_rows, n_cols;
   int col_shift, row_shift;  // key = row << row_shift | column << col_shift | position
   int table_shift;           // key >> table_shift < kCooTable for rows in range
-  int n_buckets, n_samples, n_groups, group_size;
+  int parts;
+  int64_t total;  // entries of all parts
+  int n_buckets, n_samples, n_groups, group_size, over;  // over: samples per bucket
 };
+
+// The sizes that follow from nnz (at most kCooMaxNnz).
+__host__ __device__ inline void coo_sizes(CooShape& s) {
+  const uint32_t n = (uint32_t)s.nnz, nb = (n + kCooTarget - 1) / kCooTarget;
+  s.over = kCooOver;
+  s.n_buckets = (int)(nb > kCooMaxBuckets ? kCooMaxBuckets : nb);
+  s.n_samples = s.n_buckets == 1 ? 0 : s.n_buckets * kCooOver;
+  // about 1024 groups (four per CU, all resident), within the size limits
+  uint32_t g = n / 1024;
+  g = g < kCooMinGroup ? kCooMinGroup : g > kCooMaxGroup ? kCooMaxGroup : g;
+  s.group_size = (int)g;
+  s.n_groups = (int)((n - 1) / g + 1);
+}
 
 static int bits_for(int64_t n) {  // bits of 0 .. n - 1
   int b = 0;
@@ -75,9 +105,9 @@ static int bits_for(int64_t n) {  // bits of 0 .. n - 1
 
 // False where the packed key or the size does not fit.
 static bool coo_shape(CooShape* s, int64_t nnz, int64_t n_rows, int64_t n_cols) {
-  if (nnz < 1 || nnz > kCooMaxNnz || n_rows < 0 || n_cols < 0 || n_rows > INT32_MAX || n_cols > INT32_MAX)
+  if (nnz < 1 || nnz > kCooPart * kCooMaxParts || n_rows < 0 || n_cols < 0 || n_rows > INT32_MAX || n_cols > INT32_MAX)
     return false;
-  s->nnz = nnz;
+  s->nnz = s->total = nnz;
   s->n_rows = n_rows;
   s->n_cols = n_cols;
   s->col_shift = bits_for(nnz);
@@ -86,54 +116,111 @@ static bool coo_shape(CooShape* s, int64_t nnz, int64_t n_rows, int64_t n_cols) 
   if (bits > 64 || s->row_shift > 63) return false;
   s->table_shift = bits > 11 ? bits - 11 : 0;
   static_assert(kCooTable == 1 << 11, "table bits");
-  const int64_t nb = (nnz + kCooTarget - 1) / kCooTarget;
-  s->n_buckets = (int)(nb > kCooMaxBuckets ? kCooMaxBuckets : nb);
-  s->n_samples = s->n_buckets == 1 ? 0 : s->n_buckets * kCooOver;
-  // about 1024 groups (four per CU, all resident), within the size limits
-  int64_t g = nnz / 1024;
-  g = g < kCooMinGroup ? kCooMinGroup : g > kCooMaxGroup ? kCooMaxGroup : g;
-  s->group_size = (int)g;
-  s->n_groups = (int)((nnz - 1) / g + 1);
+  s->parts = nnz <= kCooMaxNnz ? 1 : (int)((nnz + kCooPart - 1) / kCooPart);
+  if (s->parts == 1) {
+    coo_sizes(*s);
+  } else {  // the buckets and groups of the first move are the parts
+    s->n_buckets = s->n_groups = s->parts;
+    s->over = kCooMaxSamples / s->parts;
+    s->n_samples = s->parts * s->over;
+    s->group_size = 0;
+  }
   return true;
 }
 
 // Carves the workspace (base may be null: only the size is wanted).
-static int64_t coo_carve(CooWork* w, char* base, int64_t nnz) {
+static int64_t coo_carve(CooWork* w, char* base, const CooShape& s) {
   int64_t at = 0;
   auto take = [&](int64_t bytes) {
     char* p = base ? base + at : nullptr;
     at += (bytes + 255) / 256 * 256;
     return p;
   };
-  w->sample = reinterpret_cast<uint64_t*>(take(8 * kCooOver * kCooMaxBuckets));
-  w->splitters = reinterpret_cast<uint64_t*>(take(8 * kCooMaxBuckets));
-  w->counts = reinterpret_cast<uint32_t*>(take(4 * kCooMaxBuckets));
-  w->group_of = reinterpret_cast<uint16_t*>(take(2 * kCooMaxBuckets));
-  w->starts = reinterpret_cast<uint32_t*>(take(4 * (kCooMaxGroups + 1)));
-  w->cursor = reinterpret_cast<uint32_t*>(take(4 * kCooMaxGroups));
-  w->large = reinterpret_cast<uint32_t*>(take(4 * (kCooMaxGroups + 1)));
-  w->keys = reinterpret_cast<uint64_t*>(take(8 * nnz));
-  w->rows = reinterpret_cast<int32_t*>(take(4 * nnz));
-  w->bucket = reinterpret_cast<uint16_t*>(take(2 * nnz));
+  const int64_t sets = s.parts == 1 ? 1 : s.parts + 1;  // the last for the move into parts
+  w->sample = reinterpret_cast<uint64_t*>(take(8 * sets * kCooMaxSamples));
+  w->splitters = reinterpret_cast<uint64_t*>(take(8 * sets * kCooMaxBuckets));
+  w->counts = reinterpret_cast<uint32_t*>(take(4 * sets * kCooMaxBuckets));
+  w->group_of = reinterpret_cast<uint16_t*>(take(2 * sets * kCooMaxBuckets));
+  w->starts = reinterpret_cast<uint32_t*>(take(4 * sets * (kCooMaxGroups + 1)));
+  w->cursor = reinterpret_cast<uint32_t*>(take(4 * sets * kCooMaxGroups));
+  w->large = reinterpret_cast<uint32_t*>(take(4 * (sets * kCooMaxGroups + 1)));
+  w->keys = reinterpret_cast<uint64_t*>(take(8 * s.nnz));
+  w->bucket = reinterpret_cast<uint16_t*>(take(2 * s.nnz));
+  w->part_keys = nullptr;
+  w->part_values = nullptr;
+  w->part_start = nullptr;
+  if (s.parts == 1) {
+    w->rows = reinterpret_cast<int32_t*>(take(4 * s.nnz));
+  } else {
+    w->part_keys = reinterpret_cast<uint64_t*>(take(8 * s.nnz));
+    w->part_values = take(8 * s.nnz);
+    w->part_start = reinterpret_cast<uint32_t*>(take(4 * (s.parts + 1)));
+    w->rows = reinterpret_cast<int32_t*>(w->part_keys);  // read for the last time before
+  }
   return at;
 }
 
-// Out-of-range rows and columns give some key (they are flagged by coo_count
-// and the outputs are not used): any 64-bit value sorts.
-template <typename I>
-__device__ __forceinline__ uint64_t coo_key(const CooShape& s, I row, I col, int64_t e) {
-  return ((uint64_t)row << s.row_shift) | ((uint64_t)col << s.col_shift) | (uint64_t)e;
+// Set p of the work arrays that there is one of per part.
+__host__ __device__ inline void coo_set(CooWork& w, int64_t p) {
+  w.sample += p * kCooMaxSamples;
+  w.splitters += p * kCooMaxBuckets;
+  w.counts += p * kCooMaxBuckets;
+  w.group_of += p * kCooMaxBuckets;
+  w.starts += p * (kCooMaxGroups + 1);
+  w.cursor += p * kCooMaxGroups;
 }
+
+// Turns to part p: its sizes and its share of the arrays; returns its first
+// entry, or -1 if there is nothing to do (coo_parts flags a part that is too
+// large).  PARTS: whether there are several.
+template <bool PARTS>
+__device__ __forceinline__ int64_t coo_enter(CooShape& s, CooWork& w, int p) {
+  if constexpr (!PARTS) return 0;
+  const int64_t a = w.part_start[p], n = (int64_t)w.part_start[p + 1] - a;
+  if (n < 1 || n > kCooPart * 3 / 2) return -1;
+  s.nnz = n;
+  coo_sizes(s);
+  coo_set(w, p);
+  w.keys += a;
+  w.rows += a;
+  w.bucket += a;
+  w.part_keys += a;
+  return a;
+}
+
+// The entries a pass reads: index pairs, or the keys of a part.
+template <typename I> struct CooPairs {
+  static constexpr bool kParts = false;
+  typedef struct { I row, col; } entry;
+  const I* __restrict__ row;
+  const I* __restrict__ col;
+  __device__ entry load(const CooWork&, int64_t e) const { return {row[e], col[e]}; }
+  // Out-of-range rows and columns give some key (they are flagged by coo_count
+  // and the outputs are not used): any 64-bit value sorts.
+  __device__ uint64_t key(const CooShape& s, entry x, int64_t e) const {
+    return ((uint64_t)x.row << s.row_shift) | ((uint64_t)x.col << s.col_shift) | (uint64_t)e;
+  }
+  __device__ int bad(const CooShape& s, entry x) const {
+    return ((int64_t)x.row < 0 || (int64_t)x.row >= s.n_rows ? kCooBadRow : 0) |
+           ((int64_t)x.col < 0 || (int64_t)x.col >= s.n_cols ? kCooBadCol : 0);
+  }
+};
+struct CooKeys {
+  static constexpr bool kParts = true;
+  typedef uint64_t entry;
+  __device__ entry load(const CooWork& w, int64_t e) const { return w.part_keys[e]; }
+  __device__ uint64_t key(const CooShape&, entry x, int64_t) const { return x; }
+  __device__ int bad(const CooShape&, entry) const { return 0; }
+};
 
 // Sample i: from the i-th of equal ranges of the input, at a hashed place
 // inside it.  Also clears the counters of the passes that follow.
-template <typename I>
-__global__ __launch_bounds__(256) void coo_sample(const I* __restrict__ row,
-                                                  const I* __restrict__ col, CooShape s, CooWork w,
-                                                  int64_t* flags) {
+template <typename In>
+__global__ __launch_bounds__(256) void coo_sample(In in, CooShape s, CooWork w, int64_t* flags) {
+  if (coo_enter<In::kParts>(s, w, blockIdx.y) < 0) return;
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < s.n_buckets) w.counts[i] = 0;
-  if (i == 0) {
+  if (i == 0 && !In::kParts) {
     w.large[0] = 0;
     *flags = 0;
   }
@@ -142,22 +229,24 @@ __global__ __launch_bounds__(256) void coo_sample(const I* __restrict__ row,
   uint32_t h = (uint32_t)i * 2654435761u;
   h = (h ^ (h >> 15)) * 2246822519u;
   const int64_t e = a + (int64_t)((h ^ (h >> 13)) % (uint32_t)(z - a));
-  w.sample[i] = coo_key(s, row[e], col[e], e);
+  w.sample[i] = in.key(s, in.load(w, e), e);
 }
 
 // Splitters: every workgroup bins the whole sample by its leading key bits in
-// LDS and ranks 64 of its members, 16 lanes counting the smaller keys of the
-// member's bin; the members of rank kCooOver * k are the splitters (keys are
+// LDS and ranks some of its members, 16 lanes counting the smaller keys of the
+// member's bin; the members of rank over * k are the splitters (keys are
 // distinct).  A bin may hold any part of the sample (skewed rows), hence the
-// many workgroups.  Counting over the
-// whole sample instead took 15 us where this takes 7 (9,400 samples).
-constexpr int kCooRanked = 64;
+// many workgroups.  Counting over the whole sample instead took 15 us where
+// this takes 7 (9,400 samples).
+constexpr int kCooRanked = 64;  // members a workgroup ranks at a time
 
+template <bool PARTS>
 __global__ __launch_bounds__(kCooBlock) void coo_splitters(CooShape s, CooWork w) {
   extern __shared__ uint64_t binned[];
   __shared__ uint32_t bin[kCooTable + 1];
   __shared__ uint32_t part[kCooBlock / kWave];
-  constexpr int kU = kCooOver * kCooMaxBuckets / kCooBlock;
+  if (coo_enter<PARTS>(s, w, blockIdx.y) < 0) return;
+  constexpr int kU = kCooMaxSamples / kCooBlock;
   static_assert(kCooTable == 2 * kCooBlock, "two bins a thread");
   const int t = threadIdx.x, lane = t % kWave, wv = t / kWave, n = s.n_samples;
   auto bin_of = [&](uint64_t key) {
@@ -194,39 +283,36 @@ __global__ __launch_bounds__(kCooBlock) void coo_splitters(CooShape s, CooWork w
   for (int u = 0; u < kU; ++u)
     if (t + u * kCooBlock < n) binned[bin[bin_of(k[u])] + r[u]] = k[u];
   __syncthreads();
-  const int i = blockIdx.x * kCooRanked + t / 16;
-  const uint64_t m = w.sample[i < n ? i : 0];
-  const int b = bin_of(m);
-  uint32_t rank = 0;
-  for (uint32_t q = bin[b] + t % 16; q < bin[b + 1]; q += 16) rank += binned[q] < m;
+  for (int i = blockIdx.x * kCooRanked + t / 16; i < n; i += gridDim.x * kCooRanked) {
+    const uint64_t m = w.sample[i];
+    const int b = bin_of(m);
+    uint32_t rank = 0;
+    for (uint32_t q = bin[b] + t % 16; q < bin[b + 1]; q += 16) rank += binned[q] < m;
 #pragma unroll
-  for (int q = 1; q < 16; q <<= 1) rank += __shfl_xor(rank, q);
-  rank += bin[b];
-  if (t % 16 == 0 && i < n && rank > 0 && rank % kCooOver == 0)
-    w.splitters[rank / kCooOver - 1] = m;
+    for (int q = 1; q < 16; q <<= 1) rank += __shfl_xor(rank, q);
+    rank += bin[b];
+    if (t % 16 == 0 && rank > 0 && rank % s.over == 0) w.splitters[rank / s.over - 1] = m;
+  }
 }
 
 // Bucket of every entry (the number of splitters <= its key), bucket sizes,
 // and the range checks.  A table over the leading key bits leaves a step or two
 // of the search where rows are filled evenly (3.7M entries, 4096 buckets: 44 ->
 // 21 us; 1.8M: 17 -> 15 us, the rest being atomics).
-template <typename I>
-__global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row,
-                                                       const I* __restrict__ col, CooShape s,
-                                                       CooWork w, int64_t* flags) {
+template <typename In>
+__global__ __launch_bounds__(kCooBlock) void coo_count(In in, CooShape s, CooWork w, int64_t* flags) {
   __shared__ uint64_t split[kCooMaxBuckets];
   __shared__ uint32_t hist[kCooMaxBuckets];
   __shared__ uint16_t table[kCooTable + 1];
+  if (coo_enter<In::kParts>(s, w, blockIdx.y) < 0) return;
   const int t = threadIdx.x, last = s.n_buckets - 1;
   const int64_t e0 = (int64_t)blockIdx.x * kCooTile + t;
+  if (e0 - t >= s.nnz) return;  // uniform: a part of fewer tiles
   constexpr int kU = kCooTile / kCooBlock;
-  I r[kU], c[kU];
+  typename In::entry x[kU];
 #pragma unroll
-  for (int u = 0; u < kU; ++u) {
-    const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
-    r[u] = row[e];
-    c[u] = col[e];
-  }
+  for (int u = 0; u < kU; ++u)
+    x[u] = in.load(w, e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1);
   for (int b = t; b < s.n_buckets; b += kCooBlock) {
     hist[b] = 0;
     if (b < last) split[b] = w.splitters[b];
@@ -248,9 +334,8 @@ __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row
   for (int u = 0; u < kU; ++u) {
     const int64_t e = e0 + u * kCooBlock;
     if (e >= s.nnz) break;
-    bad |= ((int64_t)r[u] < 0 || (int64_t)r[u] >= s.n_rows ? kCooBadRow : 0) |
-           ((int64_t)c[u] < 0 || (int64_t)c[u] >= s.n_cols ? kCooBadCol : 0);
-    const uint64_t key = coo_key(s, r[u], c[u], e);
+    bad |= in.bad(s, x[u]);
+    const uint64_t key = in.key(s, x[u], e);
     const uint64_t h = key >> s.table_shift;
     const int slot = h < kCooTable ? (int)h : kCooTable - 1;
     int lo = table[slot], hi = table[slot + 1];
@@ -274,10 +359,12 @@ __global__ __launch_bounds__(kCooBlock) void coo_count(const I* __restrict__ row
 // Groups: bucket b belongs to group (entries before b) / group_size, so a
 // group holds neighbouring buckets of group_size entries and at most one
 // bucket more; starts of the groups (groups that begin no bucket are empty).
+template <bool PARTS>
 __global__ __launch_bounds__(kCooBlock) void coo_groups(CooShape s, CooWork w) {
   __shared__ uint32_t part[kCooBlock / kWave];
   __shared__ uint32_t start[kCooMaxGroups + 1];
   const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  if (coo_enter<PARTS>(s, w, blockIdx.y) < 0) return;
   constexpr int kPer = kCooMaxBuckets / kCooBlock;
   for (int g = t; g <= s.n_groups; g += kCooBlock) start[g] = ~0u;
   uint32_t c[kPer], sum = 0;
@@ -320,6 +407,27 @@ __global__ __launch_bounds__(kCooBlock) void coo_groups(CooShape s, CooWork w) {
   }
 }
 
+// The parts of the first move: its buckets, each a group of its own (w: its
+// set of the work arrays).  One wavefront.
+__global__ __launch_bounds__(kWave) void coo_parts(CooShape s, CooWork w, int64_t* flags) {
+  static_assert(kCooMaxParts == kWave, "one part a lane");
+  const int p = threadIdx.x;
+  const uint32_t n = p < s.parts ? w.counts[p] : 0;
+  uint32_t scan = n;
+#pragma unroll
+  for (int k = 1; k < kWave; k <<= 1) {
+    const uint32_t o = __shfl_up(scan, k);
+    if (p >= k) scan += o;
+  }
+  if (p < s.parts) {
+    w.group_of[p] = (uint16_t)p;
+    w.cursor[p] = w.part_start[p] = scan - n;
+    if (p == s.parts - 1) w.part_start[s.parts] = scan;
+  }
+  if ((int64_t)n > kCooPart * 3 / 2)
+    atomicOr(reinterpret_cast<unsigned long long*>(flags), (unsigned long long)kCooOverflow);
+}
+
 template <typename O, int VB> struct CooOut {
   const char* values;
   char* out_values;
@@ -353,10 +461,10 @@ template <int VB> __device__ __forceinline__ void store_value(char* p, int64_t i
 // with the values here the sort reads them in order instead of at random.
 // 16-byte values stay where they are: the sort gathers them.  Tiles of 6144 and
 // 4096 entries: 30 and 32 us (more atomics).
-template <typename I, int VB>
-__global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ row,
-                                                         const I* __restrict__ col, CooShape s,
-                                                         CooWork w, const char* __restrict__ values,
+template <typename In, int VB>
+__global__ __launch_bounds__(kCooBlock) void coo_scatter(In in, CooShape s, CooWork w,
+                                                         const char* __restrict__ values,
+                                                         uint64_t* __restrict__ out_keys,
                                                          char* __restrict__ out_values) {
   __shared__ uint64_t stage[kCooTile];
   __shared__ uint16_t owner[kCooTile];
@@ -365,9 +473,14 @@ __global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ r
   __shared__ uint32_t part[kCooBlock / kWave];
   uint16_t* group_of = reinterpret_cast<uint16_t*>(stage);  // until the stage is filled
   const int t = threadIdx.x, lane = t % kWave, wv = t / kWave;
+  const int64_t a = coo_enter<In::kParts>(s, w, blockIdx.y);
+  const int64_t tile0 = (int64_t)blockIdx.x * kCooTile, e0 = tile0 + t;
+  if (a < 0 || tile0 >= s.nnz) return;  // uniform
+  values += a * VB;
+  out_keys += a;
+  out_values += a * VB;
   for (int g = t; g < s.n_groups; g += kCooBlock) hist[g] = 0;
   for (int b = t; b < s.n_buckets; b += kCooBlock) group_of[b] = w.group_of[b];
-  const int64_t tile0 = (int64_t)blockIdx.x * kCooTile, e0 = tile0 + t;
   constexpr int kU = kCooTile / kCooBlock;
   uint64_t key[kU];
   CooValue<VB> v[kU];
@@ -375,7 +488,7 @@ __global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ r
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     const int64_t e = e0 + u * kCooBlock < s.nnz ? e0 + u * kCooBlock : s.nnz - 1;
-    key[u] = coo_key(s, row[e], col[e], e);
+    key[u] = in.key(s, in.load(w, e), e);
     g[u] = w.bucket[e];
     if (VB <= 8) v[u] = load_value<VB>(values, e);
   }
@@ -422,7 +535,7 @@ __global__ __launch_bounds__(kCooBlock) void coo_scatter(const I* __restrict__ r
     const int i = t + u * kCooBlock;
     if (i < n) {
       to[u] = hist[owner[i]] + i;  // < nnz: the same entries were counted
-      w.keys[to[u]] = stage[i];
+      out_keys[to[u]] = stage[i];
     }
   }
   if constexpr (VB <= 8) {
@@ -691,7 +804,7 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
     o.out_col[at] = (O)(int32_t)((kk >> sh.col_shift) & col_mask);
     // the position of a valid key; flagged input may hold any bits there
     const int64_t p = (int64_t)(kk & pos_mask);
-    if (VB > 8 || !binned) store_value<VB>(o.out_values, at, load_value<VB>(o.values, p < sh.nnz ? p : 0));
+    if (VB > 8 || !binned) store_value<VB>(o.out_values, at, load_value<VB>(o.values, p < sh.total ? p : 0));
   }
 }
 
@@ -699,12 +812,22 @@ __device__ void coo_sort_group(const CooShape& sh, const CooWork& w, const CooOu
 template <int CAP> constexpr int kCooSmem =
     8 * CAP + 4 * kCooBins > 8 * kCooLds<CAP> ? 8 * CAP + 4 * kCooBins : 8 * kCooLds<CAP>;
 
-template <typename O, int VB>
+// Turns the outputs to the part that begins at entry a.
+template <typename O, int VB> __device__ __forceinline__ void coo_out(CooOut<O, VB>& o, int64_t a) {
+  o.out_values += a * VB;
+  o.out_col += a;
+  if (o.out_row) o.out_row += a;
+}
+
+template <typename O, int VB, bool PARTS>
 __global__ __launch_bounds__(kCooSmallCap / kCooItems) void coo_sort_small(CooShape sh, CooWork w,
                                                                            CooOut<O, VB> o,
                                                                            int64_t* flags) {
   __shared__ __align__(8) char smem[kCooSmem<kCooSmallCap>];
   __shared__ CooBlockStats bs;
+  const int64_t a = coo_enter<PARTS>(sh, w, blockIdx.y);
+  if (a < 0 || (int)blockIdx.x >= sh.n_groups) return;  // uniform
+  coo_out(o, a);
   const uint32_t s = w.starts[blockIdx.x];
   const int n = (int)(w.starts[blockIdx.x + 1] - s);
   if (n > kCooSmallCap) {  // left to coo_sort_large
@@ -712,22 +835,27 @@ __global__ __launch_bounds__(kCooSmallCap / kCooItems) void coo_sort_small(CooSh
       if (n > kCooLargeCap)
         atomicOr(reinterpret_cast<unsigned long long*>(flags), (unsigned long long)kCooOverflow);
       else
-        w.large[1 + atomicAdd(w.large, 1u)] = blockIdx.x;
+        w.large[1 + atomicAdd(w.large, 1u)] = blockIdx.y << 16 | blockIdx.x;
     }
     return;
   }
   coo_sort_group<kCooSmallCap, O, VB>(sh, w, o, s, n, smem, bs);
 }
 
-template <typename O, int VB>
+template <typename O, int VB, bool PARTS>
 __global__ __launch_bounds__(kCooLargeCap / kCooItems) void coo_sort_large(CooShape sh, CooWork w,
                                                                            CooOut<O, VB> o) {
   __shared__ __align__(8) char smem[kCooSmem<kCooLargeCap>];
   __shared__ CooBlockStats bs;
   const uint32_t n_large = w.large[0];
   for (uint32_t i = blockIdx.x; i < n_large; i += gridDim.x) {
-    const uint32_t g = w.large[1 + i], s = w.starts[g];
-    coo_sort_group<kCooLargeCap, O, VB>(sh, w, o, s, (int)(w.starts[g + 1] - s), smem, bs);
+    const uint32_t id = w.large[1 + i], g = id & 0xffffu;
+    CooShape ps = sh;
+    CooWork pw = w;
+    CooOut<O, VB> po = o;
+    coo_out(po, coo_enter<PARTS>(ps, pw, (int)(id >> 16)));  // a listed part is not refused
+    const uint32_t s = pw.starts[g];
+    coo_sort_group<kCooLargeCap, O, VB>(ps, pw, po, s, (int)(pw.starts[g + 1] - s), smem, bs);
     __syncthreads();  // the next group reuses the LDS
   }
 }
@@ -747,22 +875,50 @@ __global__ __launch_bounds__(256) void coo_row_ptr(const int32_t* __restrict__ r
   ptr[r] = (P)lo;
 }
 
+// The passes over one input, or over all parts at once (grid y).
+template <typename In, typename O, int VB>
+int coo_passes(const In& in, const CooShape& s, const CooWork& w, const char* values,
+               const CooOut<O, VB>& o, int64_t* flags, hipStream_t st) {
+  constexpr bool kP = In::kParts;
+  const unsigned parts = (unsigned)s.parts;
+  // of one part at most
+  const int64_t most = kP ? kCooPart * 3 / 2 : s.nnz;
+  const int samples = kP ? kCooMaxSamples : s.n_samples, groups = kP ? kCooMaxGroups : s.n_groups;
+  const dim3 tiles((unsigned)((most + kCooTile - 1) / kCooTile), parts);
+  const int first = samples > s.n_buckets ? samples : s.n_buckets;
+  coo_sample<In><<<dim3((first + 255) / 256, parts), 256, 0, st>>>(in, s, w, flags);
+  if (kP || s.n_buckets > 1) {
+    // parts: few workgroups each, the binning of the sample is most of it
+    const dim3 grid(kP ? 32 : (samples + kCooRanked - 1) / kCooRanked, parts);
+    coo_splitters<kP><<<grid, kCooBlock, sizeof(uint64_t) * samples, st>>>(s, w);
+  }
+  coo_count<In><<<tiles, kCooBlock, 0, st>>>(in, s, w, flags);
+  coo_groups<kP><<<dim3(1, parts), kCooBlock, 0, st>>>(s, w);
+  coo_scatter<In, VB><<<tiles, kCooBlock, 0, st>>>(in, s, w, values, w.keys, o.out_values);
+  coo_sort_small<O, VB, kP><<<dim3(groups, parts), kCooSmallCap / kCooItems, 0, st>>>(s, w, o, flags);
+  if (s.nnz > kCooSmallCap) {
+    const int blocks = kP ? 256 : groups < 64 ? groups : 64;
+    coo_sort_large<O, VB, kP><<<blocks, kCooLargeCap / kCooItems, 0, st>>>(s, w, o);
+  }
+  return check_launch("fs_coo_sort");
+}
+
 template <typename I, typename O, int VB>
 int coo_run(const CooShape& s, const CooWork& w, const void* values, const I* row, const I* col,
             void* out_values, O* out_row, O* out_col, int64_t* flags, hipStream_t st) {
-  const unsigned tiles = (unsigned)((s.nnz + kCooTile - 1) / kCooTile);
-  const int first = s.n_samples > s.n_buckets ? s.n_samples : s.n_buckets;
-  coo_sample<I><<<(first + 255) / 256, 256, 0, st>>>(row, col, s, w, flags);
-  if (s.n_buckets > 1)
-    coo_splitters<<<(s.n_samples + kCooRanked - 1) / kCooRanked, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, w);
-  coo_count<I><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, flags);
-  coo_groups<<<1, kCooBlock, 0, st>>>(s, w);
+  const CooPairs<I> in{row, col};
   const CooOut<O, VB> o{static_cast<const char*>(values), static_cast<char*>(out_values), out_row, out_col};
-  coo_scatter<I, VB><<<tiles, kCooBlock, 0, st>>>(row, col, s, w, o.values, o.out_values);
-  coo_sort_small<O, VB><<<s.n_groups, kCooSmallCap / kCooItems, 0, st>>>(s, w, o, flags);
-  if (s.nnz > kCooSmallCap)
-    coo_sort_large<O, VB><<<s.n_groups < 64 ? s.n_groups : 64, kCooLargeCap / kCooItems, 0, st>>>(s, w, o);
-  return check_launch("fs_coo_sort");
+  if (s.parts == 1) return coo_passes<CooPairs<I>, O, VB>(in, s, w, o.values, o, flags, st);
+  // move the entries into the parts, with the same passes
+  CooWork pw = w;
+  coo_set(pw, s.parts);
+  const unsigned tiles = (unsigned)((s.nnz + kCooTile - 1) / kCooTile);
+  coo_sample<CooPairs<I>><<<(s.n_samples + 255) / 256, 256, 0, st>>>(in, s, pw, flags);
+  coo_splitters<false><<<(s.n_samples + kCooRanked - 1) / kCooRanked, kCooBlock, sizeof(uint64_t) * s.n_samples, st>>>(s, pw);
+  coo_count<CooPairs<I>><<<tiles, kCooBlock, 0, st>>>(in, s, pw, flags);
+  coo_parts<<<1, kWave, 0, st>>>(s, pw, flags);
+  coo_scatter<CooPairs<I>, VB><<<tiles, kCooBlock, 0, st>>>(in, s, pw, o.values, w.part_keys, w.part_values);
+  return coo_passes<CooKeys, O, VB>(CooKeys{}, s, w, w.part_values, o, flags, st);
 }
 
 template <typename I, typename O>
@@ -788,7 +944,7 @@ using namespace fs;
 extern "C" int64_t fs_coo_sort_workspace(int64_t nnz, int64_t n_rows, int64_t n_cols) {
   CooShape s;
   CooWork w;
-  return coo_shape(&s, nnz, n_rows, n_cols) ? coo_carve(&w, nullptr, nnz) : 0;
+  return coo_shape(&s, nnz, n_rows, n_cols) ? coo_carve(&w, nullptr, s) : 0;
 }
 
 extern "C" int fs_coo_sort(int32_t value_bytes, const void* values, int32_t index_type,
@@ -809,7 +965,7 @@ extern "C" int fs_coo_sort(int32_t value_bytes, const void* values, int32_t inde
   if (!values || !row || !col || !out_values || !out_col || !out_ptr || !workspace || !flags)
     return fail(FS_ERR_VALUE, "%s: null pointer", who);
   CooWork w;
-  if (workspace_bytes < coo_carve(&w, static_cast<char*>(workspace), nnz))
+  if (workspace_bytes < coo_carve(&w, static_cast<char*>(workspace), s))
     return fail(FS_ERR_VALUE, "%s: workspace too small", who);
   hipStream_t st = as_stream(stream);
   int rc;

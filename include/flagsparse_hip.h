@@ -401,10 +401,10 @@ int fs_csr_analyze_split(const fs_csr *A, int64_t *stats, int64_t short_max, int
  * outside [0, n_cols), 4: this sort's sample did not suit the entries; the
  * outputs mean something only if it is 0.  workspace: device memory of
  * fs_coo_sort_workspace(nnz, n_rows, n_cols) bytes, 256-byte aligned; that is
- * 0 where the sort does not apply: nnz of 0 or above 2^22, n_rows or n_cols
- * above 2^31 - 1, or bit widths of nnz, n_rows and n_cols above 64 together.  Replaces the
- * sort + unique + cumsum preparation of spmv_coo.py:297-327 and
- * spmv_csr.py:885-912.
+ * 0 where the sort does not apply: nnz of 0 or above 7 * 2^24, n_rows or n_cols
+ * above 2^31 - 1, or bit widths of nnz, n_rows and n_cols above 64 together.
+ * values and out_values must not overlap.  Replaces the sort + unique + cumsum
+ * preparation of spmv_coo.py:297-327 and spmv_csr.py:885-912.
  */
 int64_t fs_coo_sort_workspace(int64_t nnz, int64_t n_rows, int64_t n_cols);
 int fs_coo_sort(int32_t value_bytes, const void *values, int32_t index_type, const void *row,

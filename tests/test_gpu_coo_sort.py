@@ -62,7 +62,7 @@ def test_largest_size(kind):
 
 def test_sizes_that_do_not_apply():
     ok = _lib.coo_sort_applies
-    assert ok(1 << 22, 5, 5) and not ok((1 << 22) + 1, 5, 5) and not ok(0, 5, 5)
+    assert ok(7 << 24, 5, 5) and not ok((7 << 24) + 1, 5, 5) and not ok(0, 5, 5)
     assert ok(1 << 22, 1 << 21, 1 << 21) and not ok(1 << 22, 1 << 21, (1 << 21) + 1)
     assert ok(5, 2**31 - 1, 1 << 30) and not ok(5, 2**31, 5) and not ok(5, 5, 2**31)
 
