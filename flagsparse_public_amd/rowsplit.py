@@ -184,7 +184,10 @@ def tile_starts(row_lengths: torch.Tensor, short_max: int, tile_nnz: int,
 SPMM_FILL_LANES = 1 << 18  # lanes of 256 CUs with 16 wavefronts each
 
 
-def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int) -> Schedule:
+SPMM_CHUNK_BYTES = 1 << 27  # gathered bytes of a launch below which chunks shrink
+
+
+def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int = 0) -> Schedule:
     """Which SpMM rows one lane group walks alone and which whole wavefronts
     take in chunks.
 
@@ -199,7 +202,16 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int) -> Schedule:
     With long rows and too few of them to fill the chip with lane groups,
     every row gets a wavefront: 5,000 rows of about 300, N = 16: 45 -> 12 us;
     20,000 rows, N = 8: 77 -> 37 us; at 30,000 rows of 100 the two meet (N = 8,
-    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us)."""
+    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us).
+
+    The wider B (values of item_bytes each; 0 leaves this out), the fewer of a
+    chunk's entries its wavefront takes at once: 16 lanes a B row leave 64 round
+    trips for a chunk of 256, 64 lanes as many as it has entries.  Where a launch
+    gathers little, that chain is all of it and smaller chunks are faster, else
+    their partial sums cost more than they save.  Power-law rows, chunks of 64 /
+    128 / 256: 16,000 rows, N = 128 in fp32 (84 MB) 25 / 27 / 37 us, N = 160 in
+    bf16 (51 MB) 36 / 40 / 56; 4,000 rows, N = 160 in fp32 (23 MB) 19 / 25 / 40;
+    64,000 rows, N = 64 in fp32 (177 MB) 49 / 41 / 38."""
     mean = nnz / n_rows if n_rows > 0 else 0.0
     lanes = max(8, _pow2_ceil(n_dense / 4.0))
     if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
@@ -207,7 +219,10 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int) -> Schedule:
     short = 32
     while short < 2 * mean and short < 1024:
         short *= 2
-    return Schedule(group_lanes=1, short_max=short, chunk_nnz=256, unroll=4, col_tile=0)
+    chunk, row_bytes = 256, n_dense * item_bytes
+    if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:
+        chunk = 64 if row_bytes > 256 and nnz * row_bytes < SPMM_CHUNK_BYTES // 2 else 128
+    return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0)
 
 
 class RowSplitPlan:

@@ -127,7 +127,7 @@ def _native_spmm_coo_csr(data, row, col, B, shape):
     if not _lib.coo_sort_applies(nnz, n_rows, n_cols):
         return None
     index = torch.promote_types(row.dtype, col.dtype)
-    sch = default_spmm_schedule(n_rows, nnz, n_dense)
+    sch = default_spmm_schedule(n_rows, nnz, n_dense, data.element_size())
     lists = _lib.split_lists(nnz, n_rows, sch.short_max, sch.chunk_nnz, device)
     d, _, c, indptr = _lib.coo_sort(
         data.contiguous(), row.to(index).contiguous(), col.to(index).contiguous(), n_rows, n_cols,

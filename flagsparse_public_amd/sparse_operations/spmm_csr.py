@@ -208,7 +208,7 @@ def _spmm_call_inputs(data, indices, indptr, B, shape):
         return data, cols, indptr, B, n_rows, n_cols, n_dense, None, max_row_nnz
     data, cols, indptr, n_rows, n_cols = _check_spmm_csr_arrays(data, indices, indptr, shape)
     n_dense = int(B.shape[1])
-    sch = default_spmm_schedule(n_rows, data.numel(), n_dense)
+    sch = default_spmm_schedule(n_rows, data.numel(), n_dense, data.element_size())
     (stats, long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed,
      _) = _lib.analyze_split(
         _lib.make_csr(data, cols, indptr, n_rows, n_cols), data.device, sch.short_max,
@@ -322,7 +322,8 @@ def _hip_spmm_csr_impl(data, indices, indptr, B, n_rows, n_dense_cols, block_n, 
         return out.mul_(beta) if beta != 0.0 else out.zero_()
     n_cols = int(B.shape[0]) if n_cols is None else n_cols
     if plan is None:
-        sch = schedule or default_spmm_schedule(n_rows, data.numel(), n_dense_cols)
+        sch = schedule or default_spmm_schedule(n_rows, data.numel(), n_dense_cols,
+                                                data.element_size())
         plan = RowSplitPlan(indptr, n_rows, dtype, sch, _spmm_default_accumulate(dtype),
                             row_lengths=row_lengths)
     csr = _lib.make_csr(data, indices, indptr, n_rows, n_cols)
@@ -429,8 +430,8 @@ class PreparedCsrSpmmOpt:
         return self._csr
 
     def plan(self, accumulate, n_dense, schedule=None):
-        sch = schedule or self.schedule or default_spmm_schedule(self.n_rows, self.data.numel(),
-                                                                 n_dense)
+        sch = schedule or self.schedule or default_spmm_schedule(
+            self.n_rows, self.data.numel(), n_dense, self.data.element_size())
         return _plan_for(self._plans, self.kernel_indptr, self.n_rows, self.data.dtype,
                          accumulate, sch, self.row_lengths)
 
@@ -561,14 +562,15 @@ def spmm_launch_schedule(prepared, n_dense, schedule=None):
             return known[1]
         # the row split follows the mean row length whatever variant was
         # chosen (the variants' own bounds were picked with longer short rows)
-        split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense)
+        split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
+                                      prepared.data.element_size())
         sch = dataclasses.replace(prepared.schedule or split, short_max=split.short_max,
                                   chunk_nnz=split.chunk_nnz)
         launch = _library_spmm_launch(sch, prepared.data.dtype, n_dense)
         prepared._plans[("launch", n_dense)] = (prepared.schedule, launch)
         return launch
-    sch = schedule or prepared.schedule or default_spmm_schedule(prepared.n_rows,
-                                                                 prepared.data.numel(), n_dense)
+    sch = schedule or prepared.schedule or default_spmm_schedule(
+        prepared.n_rows, prepared.data.numel(), n_dense, prepared.data.element_size())
     return sch, sch.col_tile
 
 
