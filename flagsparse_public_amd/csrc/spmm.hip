@@ -759,10 +759,34 @@ static inline void spmm_tile_shape(int64_t n_dense, int64_t col_tile, int* vw, i
   *lanes = pow2_at_least((tile + v - 1) / v);
 }
 
+// Whether B rows are cut into tiles of one 128-byte line.  Tiles of one row go
+// to neighbouring blocks, which the XCDs take in turn, so with 2, 4 or 8 tiles
+// an XCD gathers only its part of every B row, and its L2 (4 MB) holds that many
+// times as many rows.  That pays where B does not fit one L2 and one tile of it
+// nearly does, rows have enough entries to pay for reading them once per tile,
+// and no long rows dominate (their chunks bring the wide launch its
+// parallelism).  Random rows of 20, fp32, N = 64 / 128 / 256: 32,000 rows 20.2 ->
+// 17.8 / 39.9 -> 31.2 / 85.8 -> 59.3 us, 64,000 rows 42.3 -> 38.1 / 86.6 -> 68.6 /
+// 181 -> 142 us, 96,000 rows 64.3 -> 59.4 / 134 -> 117 us; 160,000 rows 111 -> 109
+// / 230 -> 221 us (not taken: banded ones 118 -> 118).  Against it: rows of 5,
+// 64,000 rows, N = 128 29.6 -> 30.5 us; rows of 40 on a B of 8 MB, which the
+// lines' repeated use keeps in L2 anyway, fp64 25.3 -> 27.1 us; power-law rows,
+// 64,000, 66 -> 75 us.
+static inline bool spmm_line_tiles(const fs_csr* M, int64_t row_bytes, const fs_plan* pl) {
+  const int64_t lines = row_bytes / 128, panel = M->n_cols * 128, mb = 1 << 20;
+  return row_bytes % 128 == 0 && (lines == 2 || lines == 4 || lines == 8) &&
+         panel * lines > (M->nnz > 32 * M->n_rows ? 12 : 6) * mb &&
+         panel <= (lines == 8 ? 8 : 12) * mb && M->nnz >= 8 * M->n_rows &&
+         pl->n_long <= M->n_rows / 128;
+}
+
 template <typename V, typename A, typename I, typename P>
 int launch_spmm(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ldc, int64_t n_dense,
                 double alpha, double beta, const fs_plan* pl, int32_t col_tile, hipStream_t st) {
   constexpr int kMax = kMaxVw<V, I>;
+  if constexpr (std::is_same<I, int32_t>::value && kMax * sizeof(V) == 16 && kMax > 1)
+    if (col_tile == 0 && spmm_line_tiles(M, n_dense * (int64_t)sizeof(V), pl))
+      return launch_spmm_g<V, A, I, P, kMax>(8, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
   // fp64, B rows of 1 KB and more: tiles of 512 bytes unless the last would be
   // mostly idle.  Tiles of one row go to neighbouring blocks, so with two
   // tiles each XCD (round-robin by block) gathers only its half of every B
