@@ -207,6 +207,7 @@ _SIGNATURES = {
                                          ctypes.POINTER(FsPlan), ctypes.c_void_p]),
     "fs_batch_matrix_bytes": (ctypes.c_int64, []),
     "fs_batch_pack": (ctypes.c_int, [ctypes.POINTER(FsBatchEntry), ctypes.c_int64, ctypes.c_void_p]),
+    "fs_batch_rows": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int64]),
     "fs_batch_run": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64,
                                     ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32, ctypes.c_double,
                                     ctypes.c_double, ctypes.c_void_p]),

@@ -1,14 +1,14 @@
-"""Many uneven fp32 CSR SpMV / SpMM problems in one persistent launch.
+"""Many uneven fp32 CSR SpMV / SpMM problems in one launch.
 
 ``BatchedCsr`` takes a list of matrices (each with an optional SpMV operand x
 and an optional SpMM operand B), validates them, packs one device record per
-matrix, and builds a device work list whose items carry about the same
-number of bytes (entries weighted by the dense columns they gather for SpMM,
-rows cut at most every ``max_rows``).  ``run()`` launches the persistent
-kernel once; ``capture()`` records that launch into a HIP graph
-(``torch.cuda.CUDAGraph``) so a replay costs one graph launch.  The work
-queue resets itself at the end of every launch, so the graph needs no memset
-node.
+matrix, and builds a device work list of row ranges, one block each: the rows
+that a block's lane groups take in a few passes, at most ``max_rows``, cut again
+where they hold more than ``item_bytes`` (entries weighted by the dense columns
+they gather for SpMM).  ``run()`` launches the kernel once; ``capture()``
+records that launch into a HIP graph (``torch.cuda.CUDAGraph``) so a replay
+costs one graph launch.  ``blocks_per_cu`` is left over from persistent blocks
+and has no effect.
 
 Rows use the single-matrix kernels' per-row procedures: with the same lane
 group width a row's value is bit-identical to ``flagsparse_spmv_csr`` /
@@ -39,9 +39,10 @@ SPMV, SPMM = 0, 1
 
 
 def _cuts(indptr, weight_per_entry, target, max_rows, long_row=None):
-    """Row cut points of one matrix: a cut at the row holding every multiple
-    of `target` weighted entries, at least every `max_rows` rows, and around
-    every row longer than `long_row` (which then forms an item of its own)."""
+    """Row cut points of one matrix: a cut every `max_rows` rows, in ranges of
+    more than `target` weighted entries also at the row holding every multiple
+    of that, and around every row longer than `long_row` (which then forms an
+    item of its own)."""
     n = indptr.numel() - 1
     dev = indptr.device
     nnz = int(indptr[-1].item())
@@ -51,6 +52,11 @@ def _cuts(indptr, weight_per_entry, target, max_rows, long_row=None):
     by_nnz = torch.searchsorted(indptr[1:].to(torch.int64), marks, right=True)
     by_rows = (torch.arange(max_rows, n, max_rows, device=dev, dtype=torch.int64) if n > max_rows
                else torch.zeros(0, dtype=torch.int64, device=dev))
+    if by_nnz.numel():
+        # a range within the target stays whole: its rows fill the block's passes
+        first = torch.clamp(by_nnz, max=n - 1) // max_rows * max_rows
+        held = indptr[torch.clamp(first + max_rows, max=n)] - indptr[first]
+        by_nnz = by_nnz[held * weight_per_entry > target]
     parts = [torch.zeros(1, dtype=torch.int64, device=dev), by_nnz, by_rows,
              torch.full((1,), n, dtype=torch.int64, device=dev)]
     if long_row is not None and n > 0:
@@ -78,6 +84,7 @@ class BatchedCsr:
         self.keep = []  # tensors referenced by device records
         self.y, self.C = [], []
         self.group_lanes = []  # SpMV lanes per row of each matrix
+        lib = _lib_batch()
         items = []
         bytes_total = 0
         for i, m in enumerate(matrices):
@@ -118,14 +125,15 @@ class BatchedCsr:
             self.C.append(C)
             ip64 = indptr.to(torch.int64)
             if x is not None and n_rows:
-                cuts = _cuts(ip64, 12.0, item_bytes, max_rows, self.long_row)
+                rows = min(max_rows, lib.fs_batch_rows(int(s), 0))
+                cuts = _cuts(ip64, 12.0, item_bytes, rows, self.long_row)
                 items.append(self._items(i, SPMV, cuts))
                 bytes_total += 12 * nnz + 8 * n_rows
             if B is not None and n_rows and n_dense:
-                cuts = _cuts(ip64, 8.0 + 4.0 * n_dense, item_bytes, max_rows)
+                rows = min(max_rows, lib.fs_batch_rows(int(s), n_dense))
+                cuts = _cuts(ip64, 8.0 + 4.0 * n_dense, item_bytes, rows)
                 items.append(self._items(i, SPMM, cuts))
                 bytes_total += (8 + 4 * n_dense) * nnz + 4 * n_dense * n_rows
-        lib = _lib_batch()
         rec = int(lib.fs_batch_matrix_bytes())
         host = (ctypes.c_uint8 * (rec * len(matrices)))()
         _lib.check(lib.fs_batch_pack(self.entries, len(matrices), ctypes.addressof(host)),
@@ -163,7 +171,7 @@ class BatchedCsr:
         s = torch.cuda.Stream(device=self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(s):
-            self.run()  # warm (queue self-resets)
+            self.run()  # warm
         torch.cuda.current_stream(self.device).wait_stream(s)
         with torch.cuda.graph(g):
             self.run()

@@ -1,20 +1,24 @@
-// batched.hip -- many independent fp32 CSR SpMV / SpMM problems in one
-// persistent launch.
+// batched.hip -- many independent fp32 CSR SpMV / SpMM problems in one launch.
 //
 // The work list (device memory, built once per batch) holds items of
-// (matrix, kind, row range); ranges are cut so every item carries about the
-// same number of entries (weighted by dense columns for SpMM).  A persistent
-// grid of blocks pulls items from a device work queue (one atomic per item).
-// Rows are computed with the same per-row procedures (lane-group width,
-// unroll, reduction tree) as the single-matrix kernels' short-row role, so a
-// row's result is bit-identical to the single-matrix launch with the same
-// group width.  A single-row item longer than a lane group's bound is reduced
-// by the whole block instead.
+// (matrix, kind, row range), one block each: a few passes of the block's lane
+// groups over SpMV rows, one over SpMM rows.  Rows are computed with the
+// single-matrix kernels' short-row procedures (lane-group width, unroll,
+// reduction tree), so a row's result is bit-identical to the single-matrix
+// launch with the same group width.  A single-row SpMV item longer than a lane
+// group's bound is reduced by the whole block instead.
 //
-// The queue head and the finished-block counter reset themselves when the last
-// block leaves, so one launch can be replayed from a captured graph with no
-// memset node.  No counterpart in the reference (one launch per matrix and
-// bucket there).
+// The hardware hands the blocks out: there is no queue to wait for and no item
+// end at which a block's lane groups wait for the longest row of many, and
+// blocks of both kinds share a CU.  32 matrices of 1,000 to 200,000 rows of 34
+// (44M entries), one SpMV and one 8-column SpMM each: persistent blocks on a
+// queue of 96 KB items, two lanes per SpMM row, 744 us; this form 613 us (SpMV
+// alone 440 -> 271, SpMM alone 515 -> 386).  What bounds it: the requests of the
+// gathers to L2 and, for B beyond L2, the 128-byte lines behind them.  Small
+// batches no longer start and drain 2,048 blocks: 8 matrices of 15 to 3,000 rows
+// of 10 69.8 -> 6.2 us; 16 of 500 to 100,000 rows of 8, N = 12, 145 -> 69 us.
+// No counterpart in the reference (one launch per matrix and bucket there).
+#include "spmm_kernel.hpp"
 #include "spmv_kernel.hpp"
 
 namespace fs {
@@ -89,101 +93,31 @@ __device__ void bat_spmv_long_row(const BatchMatrix& m, int64_t row, double alph
   __syncthreads();
 }
 
-// --- SpMM rows: groups of G lanes, VW columns per lane (the single-matrix
-// short role's mm_accumulate<VW, 4>, restated here for the batch layout).
-constexpr int kBatMmU = 8;  // SpMM entries in flight per lane (4: 12.0 ms on the 512-matrix batch, 8: 11.0 ms)
+// --- SpMM rows: the single-matrix short role (G lanes a row, VW columns a
+// lane, entries loaded by the group through its LDS slots).
+constexpr int kBatMmU = 4;                // SpMM entries in flight per lane
+constexpr int kBatSlots = kBatBlock * 2;  // at most two fills per lane (kMmFill)
 
 template <int G, int VW>
-__device__ void bat_spmm_rows(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha, double beta) {
-  constexpr int kGroups = kBatBlock / G;
+__device__ void bat_spmm_rows(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha, double beta,
+                              int32_t* slot_col, float* slot_val) {
+  constexpr int kGroups = kBatBlock / G, F = kMmFill<G>;
+  static_assert(kBatBlock * F <= kBatSlots, "slots");
   const int grp = threadIdx.x / G, g = threadIdx.x % G;
+  const int first = grp * (G * F);
   const int64_t tiles = (m.n_dense + G * VW - 1) / (G * VW);
   for (int64_t t = 0; t < tiles; ++t) {
-    const int64_t n0 = t * (G * VW) + (int64_t)g * VW;
-    if (n0 >= m.n_dense) continue;
+    int64_t n0 = t * (G * VW) + (int64_t)g * VW;
+    const bool colok = n0 < m.n_dense;
+    const int skip = shift_tail<VW>(n0, m.n_dense);
     for (int64_t row = r0 + grp; row < r1; row += kGroups) {
       const int64_t rs = bm_ptr(m, row), re = bm_ptr(m, row + 1);
-      float acc[VW];
+      Plain<float> acc[VW];
 #pragma unroll
-      for (int k = 0; k < VW; ++k) acc[k] = 0.f;
-      int64_t j = rs;
-      for (; j + kBatMmU - 1 < re; j += kBatMmU) {
-        int64_t col[kBatMmU];
-        float a[kBatMmU];
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u) { col[u] = m.col[j + u]; a[u] = m.val[j + u]; }
-        float b[kBatMmU][VW];
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u) {
-          if constexpr (VW == 4) {
-            const float4 v = *reinterpret_cast<const float4*>(m.B + col[u] * m.ldb + n0);
-            b[u][0] = v.x; b[u][1] = v.y; b[u][2] = v.z; b[u][3] = v.w;
-          } else {
-#pragma unroll
-            for (int k = 0; k < VW; ++k) b[u][k] = m.B[col[u] * m.ldb + n0 + k];
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u)
-#pragma unroll
-          for (int k = 0; k < VW; ++k) acc[k] = __builtin_fmaf(a[u], b[u][k], acc[k]);
-      }
-      if (j < re) {  // the last, partial batch: its loads in flight together
-        int32_t ci[kBatMmU];
-        float a[kBatMmU];
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u) {
-          const bool ok = j + u < re;
-          ci[u] = ok ? m.col[j + u] : 0;
-          a[u] = ok ? m.val[j + u] : 0.f;
-        }
-        // the empty asm keeps each index's widening (and the wait for its
-        // load) out of the masked load's branch, so all four loads are issued
-        // before the first wait
-        int64_t col[kBatMmU];
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u) {
-          asm volatile("" : "+v"(ci[u]));
-          col[u] = ci[u];
-        }
-        float b[kBatMmU][VW];
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u) {
-#pragma unroll
-          for (int k = 0; k < VW; ++k) b[u][k] = 0.f;
-          if (j + u < re) {
-            if constexpr (VW == 4) {
-              const float4 v = *reinterpret_cast<const float4*>(m.B + col[u] * m.ldb + n0);
-              b[u][0] = v.x; b[u][1] = v.y; b[u][2] = v.z; b[u][3] = v.w;
-            } else {
-#pragma unroll
-              for (int k = 0; k < VW; ++k) b[u][k] = m.B[col[u] * m.ldb + n0 + k];
-            }
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kBatMmU; ++u)
-          if (j + u < re)
-#pragma unroll
-            for (int k = 0; k < VW; ++k) acc[k] = __builtin_fmaf(a[u], b[u][k], acc[k]);
-      }
-      if constexpr (VW == 4) {  // write_out's arithmetic, one 16-byte store
-        float* c = m.C + row * m.ldc + n0;
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = alpha == 1.0 ? acc[k] : scale(acc[k], alpha);
-        if (beta != 0.0) {
-          const float4 o = *reinterpret_cast<const float4*>(c);
-          v[0] = add(v[0], scale(o.x, beta));
-          v[1] = add(v[1], scale(o.y, beta));
-          v[2] = add(v[2], scale(o.z, beta));
-          v[3] = add(v[3], scale(o.w, beta));
-        }
-        *reinterpret_cast<float4*>(c) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < VW; ++k) write_out(m.C, row * m.ldc + n0 + k, acc[k], alpha, beta);
-      }
+      for (int k = 0; k < VW; ++k) acc[k].init();
+      mm_accumulate_group<VW, kBatMmU, G>(acc, slot_col + first, slot_val + first, m.col, m.val, m.B,
+                                          m.ldb, n0, colok, rs, re, g);
+      if (colok) write_vec<G, VW>(m.C, row * m.ldc + n0, acc, alpha, beta, skip);
     }
   }
 }
@@ -200,70 +134,42 @@ __device__ void bat_spmv_dispatch(const BatchMatrix& m, int64_t r0, int64_t r1, 
   }
 }
 
-__device__ void bat_spmm_dispatch(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha, double beta) {
+// The (VW, G) pairs that spmm_tile_shape<4> gives.
+__device__ void bat_spmm_dispatch(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha,
+                                  double beta, int32_t* sc, float* sv) {
   if (m.mm_vw == 4) {
     switch (m.mm_lanes) {
-      case 1: bat_spmm_rows<1, 4>(m, r0, r1, alpha, beta); break;
-      case 2: bat_spmm_rows<2, 4>(m, r0, r1, alpha, beta); break;
-      case 4: bat_spmm_rows<4, 4>(m, r0, r1, alpha, beta); break;
-      case 8: bat_spmm_rows<8, 4>(m, r0, r1, alpha, beta); break;
-      case 16: bat_spmm_rows<16, 4>(m, r0, r1, alpha, beta); break;
-      case 32: bat_spmm_rows<32, 4>(m, r0, r1, alpha, beta); break;
-      default: bat_spmm_rows<64, 4>(m, r0, r1, alpha, beta); break;
+      case 8: bat_spmm_rows<8, 4>(m, r0, r1, alpha, beta, sc, sv); break;
+      case 16: bat_spmm_rows<16, 4>(m, r0, r1, alpha, beta, sc, sv); break;
+      case 32: bat_spmm_rows<32, 4>(m, r0, r1, alpha, beta, sc, sv); break;
+      default: bat_spmm_rows<64, 4>(m, r0, r1, alpha, beta, sc, sv); break;
     }
+  } else if (m.mm_vw == 2) {
+    if (m.mm_lanes <= 8) bat_spmm_rows<8, 2>(m, r0, r1, alpha, beta, sc, sv);
+    else bat_spmm_rows<16, 2>(m, r0, r1, alpha, beta, sc, sv);
   } else {
-    switch (m.mm_lanes) {
-      case 1: bat_spmm_rows<1, 1>(m, r0, r1, alpha, beta); break;
-      case 2: bat_spmm_rows<2, 1>(m, r0, r1, alpha, beta); break;
-      case 4: bat_spmm_rows<4, 1>(m, r0, r1, alpha, beta); break;
-      case 8: bat_spmm_rows<8, 1>(m, r0, r1, alpha, beta); break;
-      case 16: bat_spmm_rows<16, 1>(m, r0, r1, alpha, beta); break;
-      case 32: bat_spmm_rows<32, 1>(m, r0, r1, alpha, beta); break;
-      default: bat_spmm_rows<64, 1>(m, r0, r1, alpha, beta); break;
-    }
+    if (m.mm_lanes <= 4) bat_spmm_rows<4, 1>(m, r0, r1, alpha, beta, sc, sv);
+    else if (m.mm_lanes <= 8) bat_spmm_rows<8, 1>(m, r0, r1, alpha, beta, sc, sv);
+    else bat_spmm_rows<16, 1>(m, r0, r1, alpha, beta, sc, sv);
   }
 }
 
 __global__ __launch_bounds__(kBatBlock) void batched_kernel(const BatchMatrix* __restrict__ mats,
                                                             const fs_batch_item* __restrict__ items,
-                                                            int64_t n_items, int64_t long_row,
-                                                            double alpha, double beta,
-                                                            int32_t* __restrict__ queue) {
-  __shared__ int64_t cur;
-  __shared__ float lds[2 * (kBatBlock / kWave)];
-  while (true) {
-    if (threadIdx.x == 0)
-      cur = __hip_atomic_fetch_add(queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int64_t it = cur;
-    __syncthreads();
-    if (it >= n_items) break;
-    const fs_batch_item w = items[it];
-    const BatchMatrix& m = mats[w.matrix];
-    if (w.kind == FS_BATCH_SPMV) {
-      if (w.row_end - w.row_begin == 1 &&
-          bm_ptr(m, w.row_begin + 1) - bm_ptr(m, w.row_begin) > long_row)
-        bat_spmv_long_row(m, w.row_begin, alpha, beta, lds);
-      else
-        bat_spmv_dispatch(m, w.row_begin, w.row_end, alpha, beta);
-    } else {
-      bat_spmm_dispatch(m, w.row_begin, w.row_end, alpha, beta);
-    }
+                                                            int64_t long_row, double alpha,
+                                                            double beta) {
+  __shared__ int32_t slot_col[kBatSlots];
+  __shared__ float slot_val[kBatSlots];
+  const fs_batch_item w = items[blockIdx.x];
+  const BatchMatrix& m = mats[w.matrix];
+  if (w.kind == FS_BATCH_SPMV) {
+    if (w.row_end - w.row_begin == 1 && bm_ptr(m, w.row_begin + 1) - bm_ptr(m, w.row_begin) > long_row)
+      bat_spmv_long_row(m, w.row_begin, alpha, beta, slot_val);
+    else
+      bat_spmv_dispatch(m, w.row_begin, w.row_end, alpha, beta);
+  } else {
+    bat_spmm_dispatch(m, w.row_begin, w.row_end, alpha, beta, slot_col, slot_val);
   }
-  // the last block out resets the queue for the next launch
-  if (threadIdx.x == 0) {
-    const int done = __hip_atomic_fetch_add(queue + 1, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    if (done == (int)gridDim.x - 1) {
-      __hip_atomic_store(queue, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(queue + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-}
-
-static int pow2_ceil_i(int64_t v) {
-  int g = 1;
-  while (g < v && g < 64) g <<= 1;
-  return g;
 }
 
 }  // namespace fs
@@ -304,15 +210,23 @@ extern "C" int fs_batch_pack(const fs_batch_entry* entries, int64_t n_entries, v
     m.ldc = e.ldc;
     m.group_lanes = s;
     m.ptr64 = A.ptr_type == FS_I64;
-    int vw = 1;
-    if (e.n_dense > 0 && e.n_dense % 4 == 0 && e.ldb % 4 == 0 && e.ldc % 4 == 0 &&
-        ((uintptr_t)e.B % 16) == 0 && ((uintptr_t)e.C % 16) == 0)
-      vw = 4;
+    int vw = 1, lanes = 1;
+    if (e.n_dense > 0) spmm_tile_shape<4>(e.n_dense, 0, &vw, &lanes);
     m.mm_vw = vw;
-    m.mm_lanes = pow2_ceil_i((e.n_dense + vw - 1) / vw);
+    m.mm_lanes = lanes;
     out[i] = m;
   }
   return FS_OK;
+}
+
+extern "C" int fs_batch_rows(int32_t group_lanes, int64_t n_dense) {
+  // SpMV: four rows per lane group (8 or 64 of 32 rows: 287 / 274 against 271 us
+  // on the batch above), enough to pay for a block's start; SpMM: one (two: 413
+  // against 382 us, the block waits for the longer of more rows)
+  if (n_dense <= 0) return group_lanes > 0 ? 4 * (kBatBlock / group_lanes) : kBatBlock;
+  int vw = 1, lanes = 1;
+  spmm_tile_shape<4>(n_dense, 0, &vw, &lanes);
+  return kBatBlock / (lanes < 4 ? 4 : lanes);
 }
 
 extern "C" int fs_batch_run(const void* packed_dev, int64_t n_matrices, const fs_batch_item* items,
@@ -323,11 +237,9 @@ extern "C" int fs_batch_run(const void* packed_dev, int64_t n_matrices, const fs
   if (!packed_dev || !items || !queue) return fail(FS_ERR_VALUE, "fs_batch_run: null pointer");
   if (grid <= 0) return fail(FS_ERR_VALUE, "fs_batch_run: grid must be positive");
   if (long_row < 1) return fail(FS_ERR_VALUE, "fs_batch_run: long_row must be >= 1");
-  // the work queue head is an int32 that every block advances once past the
-  // last item; it must not wrap
   if (n_items + (int64_t)grid > (int64_t)INT32_MAX)
     return fail(FS_ERR_UNSUPPORTED, "fs_batch_run: n_items + grid must stay below 2^31 - 1");
-  batched_kernel<<<grid, kBatBlock, 0, as_stream(stream)>>>(static_cast<const BatchMatrix*>(packed_dev),
-                                                           items, n_items, long_row, alpha, beta, queue);
+  batched_kernel<<<(unsigned)n_items, kBatBlock, 0, as_stream(stream)>>>(
+      static_cast<const BatchMatrix*>(packed_dev), items, long_row, alpha, beta);
   return check_launch("fs_batch_run");
 }

@@ -443,7 +443,7 @@ int fs_spmv_csr_split(const fs_csr *A, int32_t format, const void *hi, const voi
                       const float *row_scale, const void *x, void *y, double alpha, double beta,
                       const fs_plan *plan, void *stream);
 
-/* ------------------------------------------------- batched persistent path */
+/* ------------------------------------------------------------ batched path */
 /*
  * Many independent fp32 / int32-column CSR problems in one persistent launch
  * (replayable from a captured graph).  No counterpart in the reference, which
@@ -474,16 +474,18 @@ typedef struct fs_batch_item {
 /* Bytes of one packed matrix record; fs_batch_pack writes n_entries records
  * into host memory, which the caller copies to the device. */
 int64_t fs_batch_matrix_bytes(void);
+/* Rows of an item that suit its block: of SpMV items with group_lanes lanes a row
+ * (n_dense 0), or of SpMM items with n_dense columns. */
+int fs_batch_rows(int32_t group_lanes, int64_t n_dense);
 int fs_batch_pack(const fs_batch_entry *entries, int64_t n_entries, void *packed_host);
 
 /*
  * Run every item: y = alpha A x + beta y for SpMV items, C = alpha A B + beta C
- * for SpMM items.  packed_dev: the packed records in device memory; items:
- * device array; queue: two int32 in device memory, zero before the first call
- * and zero again after every call.  grid: persistent block count (e.g. a
- * small multiple of the CU count).  Single-row SpMV items longer than
- * long_row entries are reduced by a whole block.  Calls sharing a queue must
- * be ordered on one stream.
+ * for SpMM items, one block each.  packed_dev: the packed records in device
+ * memory; items: device array.  Single-row SpMV items longer than long_row
+ * entries are reduced by a whole block.  queue (two int32 in device memory) and
+ * grid (at least 1) are left over from blocks that pulled items from a queue:
+ * they are checked and not used.
  */
 int fs_batch_run(const void *packed_dev, int64_t n_matrices, const fs_batch_item *items,
                  int64_t n_items, int64_t long_row, int32_t *queue, int32_t grid, double alpha,
