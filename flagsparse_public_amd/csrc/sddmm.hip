@@ -3,64 +3,68 @@
 // fs_sddmm_csr).
 //
 // Replaces the reference's Triton kernel (sddmm_csr.py:108-151: a program per
-// 128 entries, K in BLOCK_K steps, tl.sum reduction).  Here a group of G
-// lanes takes kSdE<G> entries: each lane reads VW consecutive elements of the x
-// row and of the y row per step (16-byte loads when the rows are aligned),
-// keeps a running sum per entry, and the group reduces with DPP / swizzle
-// exchanges.  G is the smallest power of two covering K / VW (at most 64), so
-// short K does not leave lanes idle.
+// 128 entries, K in BLOCK_K steps, tl.sum reduction).  A row of x or y is cut
+// into parts of 16 bytes, loaded at any alignment; a group of at most 8 lanes
+// takes two entries, lane g parts g, g + 8, ..., and the group reduces with DPP /
+// swizzle exchanges.
+//
+// Why so few lanes: with a lane for every part (up to 64) the exchanges and the
+// address work of an entry, spread over many lanes with little to do, bound the
+// kernel; with 8 the 128-byte lines of the y rows do (about 7 TB/s) once y exceeds
+// L2.  3M entries of a banded pattern, where the lines stay in L2, fp32 K = 160 299
+// -> 197 us, fp64 K = 40 / 64 / 100: 171 -> 117 / 193 -> 157 / 393 -> 278 us; 1.6M
+// random entries, K = 160 in fp32 157 -> 151, in fp64 359 -> 298 us.  Adding beta *
+// data: banded fp32 K = 64 / 128 101 -> 85 / 200 -> 157 us.
+// Widths that 16 bytes do not divide took element loads: fp32 K = 33 / 97, random
+// 92 -> 47 / 122 -> 108 us, banded 172 -> 68 / 229 -> 156 us; fp64 K = 47 158 ->
+// 106 us.  16 lanes above 32 parts: 3-5% faster on random patterns, up to 18%
+// slower on banded ones.
 #include "fs_host.hpp"
 
 namespace fs {
 
 constexpr int kSdBlock = 256;
 
-template <typename T, int VW> struct VecOf;
-template <> struct VecOf<float, 4> { using type = float4; };
-template <> struct VecOf<float, 1> { using type = float; };
-template <> struct VecOf<double, 2> { using type = double2; };
-template <> struct VecOf<double, 1> { using type = double; };
-
-template <typename A, typename T, int VW>
-__device__ __forceinline__ void sd_fma(A& acc, const T* xr, const T* yr, int64_t k) {
-  using C = typename A::compute_t;
-  if constexpr (VW == 1) {
-    acc.add_prod((C)xr[k], (C)yr[k]);
-  } else {
-    using V = typename VecOf<T, VW>::type;
-    const V a = *reinterpret_cast<const V*>(xr + k);
-    const V b = *reinterpret_cast<const V*>(yr + k);
-    const T* pa = reinterpret_cast<const T*>(&a);
-    const T* pb = reinterpret_cast<const T*>(&b);
-#pragma unroll
-    for (int i = 0; i < VW; ++i) acc.add_prod((C)pa[i], (C)pb[i]);
-  }
+// VW consecutive elements of a row, at any address: one 16-byte load.
+template <typename T, int VW> struct SdVec {
+  typedef T type __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
+};
+template <typename T> struct SdVec<T, 1> { typedef T type; };
+template <int VW, typename V> __device__ __forceinline__ auto sd_elem(const V& v, int i) {
+  if constexpr (VW == 1) return v;
+  else return v[i];
 }
 
-// Entries per lane group: the group's kSdE entries (kSdBlock / G apart, so
-// consecutive groups still read consecutive row ids / columns) have their row
-// and column loads, and then their x / y row loads, in flight together.
-// Measured on a 1M x 1M Poisson(16) pattern, fp32: one entry per group
-// 418 / 880 / 1969 us at K = 32 / 64 / 128; two 333 / 649 / 1472; four
-// 334 / 625 / 1324; eight at K = 128 (32-lane groups) 1304 (K = 8: 288, 290,
-// 293 us for one, two, four).
-template <int G> constexpr int kSdE = G >= 32 ? 8 : (G >= 16 ? 4 : 2);
-
-template <typename A, typename T, typename O, int G, int VW>
+// A group takes E entries, kSdBlock / G apart, so that consecutive groups read
+// consecutive row ids / columns; their loads are in flight together.
+//
+// A lane takes the parts that NS lanes would take if there was one for every
+// part (up to 64): the sums of parts that would lie in different lanes stay
+// apart until the end and are added pairwise, so no sum has a longer chain of
+// additions than with that many lanes, and its error is the same (fp32 sums,
+// K = 64 / 160, relative to fp64: 6.80e-8 / 7.60e-8 with the lanes, 6.78e-8 /
+// 7.51e-8 here).  Sums in fp64 over fp32 values need no such care and keep one.
+// TAIL: the last part of a row is not whole; it is loaded VW elements from the
+// row's end, and those that the part before it holds are left out.
+template <typename A, typename T, typename O, int G, int VW, int NS, int E, bool TAIL>
 __global__ __launch_bounds__(kSdBlock) void sddmm_kernel(
     const int32_t* __restrict__ row_ids, const int32_t* __restrict__ cols,
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ data,
     O* __restrict__ out, int64_t nnz, int64_t k_dim, double alpha, double beta) {
   using C = typename A::compute_t;
+  using V = typename SdVec<T, VW>::type;
   constexpr int kGroups = kSdBlock / G;
-  constexpr int kE = kSdE<G>;
-  const int64_t p0 = (int64_t)blockIdx.x * kGroups * kE + threadIdx.x / G;
+  constexpr int kSums = sizeof(C) > sizeof(T) ? 1 : NS;
+  // parts in flight per lane and entry (fp32 K = 160, banded: 203 us with one,
+  // 200 with two, 247 with four, whose registers leave fewer wavefronts)
+  constexpr int kB = NS < 2 ? NS : 2;
+  const int64_t p0 = (int64_t)blockIdx.x * kGroups * E + threadIdx.x / G;
   const int g = threadIdx.x % G;
-  const T* xr[kE];
-  const T* yr[kE];
-  bool live[kE];  // the whole group agrees
+  const T* xr[E];
+  const T* yr[E];
+  bool live[E];  // the whole group agrees
 #pragma unroll
-  for (int e = 0; e < kE; ++e) {
+  for (int e = 0; e < E; ++e) {
     const int64_t p = p0 + (int64_t)e * kGroups;
     live[e] = p < nnz;
     // past nnz: the last entry again (nnz >= 1), computed and not written,
@@ -69,36 +73,83 @@ __global__ __launch_bounds__(kSdBlock) void sddmm_kernel(
     xr[e] = x + (int64_t)row_ids[q] * k_dim;
     yr[e] = y + (int64_t)cols[q] * k_dim;
   }
-  A acc[kE];
+  C d[E];  // loaded ahead of the rows, not behind the sums
 #pragma unroll
-  for (int e = 0; e < kE; ++e) acc[e].init();
-  for (int64_t k = (int64_t)g * VW; k < k_dim; k += (int64_t)G * VW)
+  for (int e = 0; e < E; ++e)
+    d[e] = data && live[e] ? (C)data[p0 + (int64_t)e * kGroups] * (C)beta : (C)0;
+  A acc[E][kSums];
 #pragma unroll
-    for (int e = 0; e < kE; ++e) sd_fma<A, T, VW>(acc[e], xr[e], yr[e], k);
+  for (int e = 0; e < E; ++e)
 #pragma unroll
-  for (int e = 0; e < kE; ++e) {
-    group_reduce<G>(acc[e]);
+    for (int i = 0; i < kSums; ++i) acc[e][i].init();
+  for (int64_t k0 = 0; k0 < k_dim; k0 += (int64_t)G * VW * NS)
+#pragma unroll
+    for (int s0 = 0; s0 < NS; s0 += kB) {
+      if (k0 + (int64_t)s0 * G * VW >= k_dim) break;  // uniform
+      V a[kB][E], b[kB][E];
+      bool ok[kB];
+      int skip[kB];
+#pragma unroll
+      for (int s = 0; s < kB; ++s) {
+        const int64_t k = k0 + (int64_t)((s0 + s) * G + g) * VW;
+        ok[s] = k < k_dim;
+        skip[s] = TAIL && ok[s] && k + VW > k_dim ? (int)(k + VW - k_dim) : 0;
+        const int64_t at = ok[s] ? k - skip[s] : 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          a[s][e] = *reinterpret_cast<const V*>(xr[e] + at);
+          b[s][e] = *reinterpret_cast<const V*>(yr[e] + at);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < kB; ++s) {
+        const int sum = kSums == 1 ? 0 : s0 + s;
+        if (ok[s] && !(TAIL && skip[s])) {
+#pragma unroll
+          for (int e = 0; e < E; ++e)
+#pragma unroll
+            for (int i = 0; i < VW; ++i)
+              acc[e][sum].add_prod((C)sd_elem<VW>(a[s][e], i), (C)sd_elem<VW>(b[s][e], i));
+        } else if (TAIL && skip[s]) {
+#pragma unroll
+          for (int i = 1; i < VW; ++i)
+            if (i >= skip[s])
+#pragma unroll
+              for (int e = 0; e < E; ++e)
+                acc[e][sum].add_prod((C)sd_elem<VW>(a[s][e], i), (C)sd_elem<VW>(b[s][e], i));
+        }
+      }
+    }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+#pragma unroll
+    for (int h = kSums / 2; h > 0; h /= 2)
+#pragma unroll
+      for (int i = 0; i < h; ++i) acc[e][i].merge(acc[e][i + h]);
+    group_reduce<G>(acc[e][0]);
     if (live[e] && g == 0) {
       const int64_t p = p0 + (int64_t)e * kGroups;
-      C v = acc[e].value() * (C)alpha;
-      if (data) v += (C)data[p] * (C)beta;
+      C v = acc[e][0].value() * (C)alpha;
+      if (data) v += d[e];
       out[p] = (O)v;
     }
   }
 }
 
-template <typename A, typename T, typename O, int G>
+template <typename A, typename T, typename O, int G, int VW, int NS, int E = 2>
 void sddmm_launch_g(const int32_t* rid, const int32_t* cols, const T* x, const T* y,
                     const T* data, O* out, int64_t nnz, int64_t k, double alpha, double beta,
-                    int vw, hipStream_t st) {
-  const int64_t per_block = (int64_t)(kSdBlock / G) * kSdE<G>;
+                    hipStream_t st) {
+  const int64_t per_block = (int64_t)(kSdBlock / G) * E;
   const int64_t blocks = (nnz + per_block - 1) / per_block;
   const dim3 grid((unsigned)blocks), block(kSdBlock);
-  constexpr int kVec = sizeof(T) == 4 ? 4 : 2;
-  if (vw == kVec)
-    sddmm_kernel<A, T, O, G, kVec><<<grid, block, 0, st>>>(rid, cols, x, y, data, out, nnz, k, alpha, beta);
-  else
-    sddmm_kernel<A, T, O, G, 1><<<grid, block, 0, st>>>(rid, cols, x, y, data, out, nnz, k, alpha, beta);
+  if constexpr (VW > 1) {
+    if (k % VW != 0) {
+      sddmm_kernel<A, T, O, G, VW, NS, E, true><<<grid, block, 0, st>>>(rid, cols, x, y, data, out, nnz, k, alpha, beta);
+      return;
+    }
+  }
+  sddmm_kernel<A, T, O, G, VW, NS, E, false><<<grid, block, 0, st>>>(rid, cols, x, y, data, out, nnz, k, alpha, beta);
 }
 
 template <typename A, typename T, typename O>
@@ -110,22 +161,37 @@ int sddmm_launch(const fs_csr* P, const int32_t* rid, const void* x, const void*
   const T* data = static_cast<const T*>(P->values);
   O* o = static_cast<O*>(out);
   constexpr int kVec = sizeof(T) == 4 ? 4 : 2;
-  // vector loads need every row start aligned: k a multiple of the width and
-  // 16-byte aligned bases
-  const bool vec = k % kVec == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)y % 16) == 0;
-  const int vw = vec ? kVec : 1;
-  int64_t per = (k + vw - 1) / vw;  // lane steps for one entry
-  int G = 1;
-  while (G < per && G < 64) G <<= 1;
-  const int64_t nnz = P->nnz;
-  switch (G) {
-    case 1: sddmm_launch_g<A, T, O, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    case 2: sddmm_launch_g<A, T, O, 2>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    case 4: sddmm_launch_g<A, T, O, 4>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    case 8: sddmm_launch_g<A, T, O, 8>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    case 16: sddmm_launch_g<A, T, O, 16>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    case 32: sddmm_launch_g<A, T, O, 32>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
-    default: sddmm_launch_g<A, T, O, 64>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, vw, st); break;
+  const int64_t nnz = P->nnz, per = (k + kVec - 1) / kVec;
+  if (k < kVec) {  // no whole vector in a row
+    if (k <= 1) sddmm_launch_g<A, T, O, 1, 1, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+    else if (k == 2) sddmm_launch_g<A, T, O, 2, 1, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+    else sddmm_launch_g<A, T, O, 4, 1, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+    return check_launch("fs_sddmm_csr");
+  }
+  int lanes = 1;  // the power of two that covers the row's parts, at most 64
+  while (lanes < per && lanes < 64) lanes <<= 1;
+  switch (lanes) {
+    case 1: sddmm_launch_g<A, T, O, 1, kVec, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st); break;
+    case 2: sddmm_launch_g<A, T, O, 2, kVec, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st); break;
+    case 4: sddmm_launch_g<A, T, O, 4, kVec, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st); break;
+    case 8: sddmm_launch_g<A, T, O, 8, kVec, 1>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st); break;
+    // fp32 without data keeps a lane for every part and more entries in flight.
+    // K = 128, 2M random entries of 400,000 rows 164 us against 177, 1.6M of
+    // 100,000 113 against 115; with data 181 against 177, banded 193 against 157.
+    // K = 64: 84.9 against 87.6, 56.0 against 55.4, banded 82 against 80 us.
+    case 16:
+      if (kVec == 4 && !data && k % kVec == 0)
+        sddmm_launch_g<A, T, O, 16, kVec, 1, 4>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+      else
+        sddmm_launch_g<A, T, O, 8, kVec, 2>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+      break;
+    case 32:
+      if (kVec == 4 && !data)
+        sddmm_launch_g<A, T, O, 32, kVec, 1, 8>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+      else
+        sddmm_launch_g<A, T, O, 8, kVec, 4>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st);
+      break;
+    default: sddmm_launch_g<A, T, O, 8, kVec, 8>(rid, cols, xs, ys, data, o, nnz, k, alpha, beta, st); break;
   }
   return check_launch("fs_sddmm_csr");
 }
