@@ -318,6 +318,13 @@ def make_csr(data, indices, indptr, n_rows, n_cols) -> FsCsr:
     )
 
 
+def make_rows(indptr, n_rows) -> FsCsr:
+    """The row pointers alone, for passes that read nothing else."""
+    return FsCsr(value_type=FS_F32, index_type=FS_I32, ptr_type=index_code(indptr.dtype),
+                 reserved=0, n_rows=int(n_rows), n_cols=0, nnz=0, row_ptr=ptr(indptr),
+                 col_idx=None, values=None)
+
+
 class _Nothing:
     def __enter__(self):
         return None
@@ -426,7 +433,7 @@ def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bo
     spare word of ``lists``).  Entries of the lists past n_long / n_chunks are
     unset.  ``lists``: from split_lists, where the caller uses the spare word."""
     lib = load()
-    nnz = int(csr.nnz)
+    nnz = int(csr.nnz)  # 0 for make_rows, which needs ``lists``
     if lists is None:
         lists = split_lists(nnz, int(csr.n_rows), short_max, chunk_nnz, device)
     buf, long_rows, long_chunk_ptr, chunk_long, cap_long, cap_chunks = lists

@@ -265,12 +265,12 @@ def _resolve_spmm_alg1_launch_config(n_dense_cols, max_row_nnz, block_n=None, bl
 
 # ---------------------------------------------------------------- launches
 
-def _plan_for(cache, kernel_indptr, n_rows, dtype, accumulate, schedule, row_lengths):
+def _plan_for(cache, kernel_indptr, n_rows, dtype, accumulate, schedule, row_lengths, nnz=None):
     key = (int(accumulate), schedule.key())
     p = cache.get(key)
     if p is None:
         p = RowSplitPlan(kernel_indptr, n_rows, dtype, schedule, accumulate,
-                         row_lengths=row_lengths)
+                         row_lengths=row_lengths, nnz=nnz)
         cache[key] = p
     return p
 
@@ -433,7 +433,7 @@ class PreparedCsrSpmmOpt:
         sch = schedule or self.schedule or default_spmm_schedule(
             self.n_rows, self.data.numel(), n_dense, self.data.element_size())
         return _plan_for(self._plans, self.kernel_indptr, self.n_rows, self.data.dtype,
-                         accumulate, sch, self.row_lengths)
+                         accumulate, sch, self.row_lengths, self.data.numel())
 
 
 _SPMM_OPT_BUCKET_SPECS = (

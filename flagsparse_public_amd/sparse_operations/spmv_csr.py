@@ -168,7 +168,8 @@ class PreparedCsrSpmv:
         if p is None:
             p = RowSplitPlan(self.kernel_indptr, self.n_rows, self.data.dtype, sch, accumulate,
                              row_lengths=self.row_lengths,
-                             max_row=None if self._stats is None else self.max_row_nnz)
+                             max_row=None if self._stats is None else self.max_row_nnz,
+                             nnz=self.data.numel())
             self._plans[key] = p
         return p
 
