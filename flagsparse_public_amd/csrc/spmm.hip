@@ -332,6 +332,22 @@ __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> 
   write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta, skip);
 }
 
+// Whether each XCD takes a contiguous range of rows (xcd_remap_block) although
+// the plan does not ask for it.  Neighbouring rows of matrices from meshes gather
+// the same B rows, which one L2 then holds once; dealt in turn, blocks bring them
+// into all eight.  fp32 / fp64, banded rows of 15: 1M rows N = 64 362 -> 351 us,
+// N = 100 705 -> 643; 300,000 rows N = 100 210 -> 194, fp64 405 -> 345 us.  Random
+// rows of 16: between -5% and +1%.  Not taken: B below 24 MB (20,000 rows N = 8 to
+// 64: up to 8% slower), rows of under 12 entries (1M banded rows of 9, N = 64 234
+// -> 241 us), 16-bit values (1M rows of 9, N = 100 303 -> 312 us), long rows, and
+// column tiles, whose neighbours belong on different XCDs.
+template <typename V>
+static inline bool spmm_xcd_rows(const fs_csr* M, int64_t n_dense, int64_t n_tiles, const fs_plan* pl) {
+  return (std::is_same<V, float>::value || std::is_same<V, double>::value) && n_tiles == 1 &&
+         M->n_cols * n_dense * (int64_t)sizeof(V) >= ((int64_t)24 << 20) &&
+         M->nnz >= 12 * M->n_rows && pl->n_long <= M->n_rows / 128;
+}
+
 template <typename V, typename A, typename I, typename P, int G, int VW>
 int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ldc,
                    int64_t n_dense, double alpha, double beta, const fs_plan* pl, hipStream_t st) {
@@ -356,7 +372,7 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
   p.long_chunk_ptr = pl->long_chunk_ptr;
   p.chunk_long = pl->chunk_long;
   p.partials = pl->partials;
-  p.xcd_remap = pl->xcd_remap;
+  p.xcd_remap = pl->xcd_remap || spmm_xcd_rows<V>(M, n_dense, p.n_tiles, pl);
   const int64_t rows_per_block = kMmBlock / G;
   const int64_t short_blocks = ((M->n_rows + rows_per_block - 1) / rows_per_block) * p.n_tiles;
   const int64_t grid = p.n_chunk_blocks + short_blocks;
