@@ -192,7 +192,7 @@ __device__ __forceinline__ void block_apply_all(const int64_t (&v)[FS_STATS_LEN]
 // of 16 entries 13.9 -> 8.6 us, 1M rows of 16 34.8 -> 22.8 us (67 MB), 4M rows
 // of 12 51.0 -> 42.9 us (208 MB, 4.8 TB/s); with 64-bit arrays, whose columns
 // took 8-byte loads, 15.6 -> 10.5, 41.3 -> 31.0, 82.0 -> 71.3 us (5.8 TB/s).
-template <typename I, typename P, bool SPLIT>
+template <typename I, typename P, bool SPLIT, bool NT>
 __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ ptr,
                                                           const I* __restrict__ idx,
                                                           int64_t n_rows, int64_t nnz,
@@ -241,10 +241,7 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
   // columns: only min and max are kept, so a lane past the end re-reads the
   // iteration's first column instead of branching.  16-byte loads (four 32-bit
   // or two 64-bit columns), eight in flight per thread, over the aligned body
-  // of the column array.  Non-temporal: the columns are read once here, and an
-  // unprepared call's SpMV follows at once, whose data they would otherwise
-  // push out of the caches (4M-row power-law matrix: this pass 51.5 -> 53.8 us,
-  // the whole repeated unprepared call 268 -> 254 us).
+  // of the column array.  NT (non-temporal): see kAnNtBytes.
   typedef I vec_t __attribute__((ext_vector_type(16 / sizeof(I))));
   constexpr int kPer = 16 / (int)sizeof(I);
   I mn = sizeof(I) == 4 ? (I)INT32_MAX : (I)INT64_MAX, mx = -1;
@@ -255,8 +252,11 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
   for (int64_t k = t0; k < nv; k += 8 * stride) {
     vec_t c[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      c[u] = __builtin_nontemporal_load(q + (k + u * stride < nv ? k + u * stride : k));
+    for (int u = 0; u < 8; ++u) {
+      const vec_t* at = q + (k + u * stride < nv ? k + u * stride : k);
+      if constexpr (NT) c[u] = __builtin_nontemporal_load(at);
+      else c[u] = *at;
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -296,6 +296,14 @@ __global__ __launch_bounds__(kAnBlock) void analyze_pass(const P* __restrict__ p
   block_apply_all(v, st);
 }
 
+// Columns of more bytes than this are read past the caches.  An unprepared
+// call's product follows at once and reads the columns again.  Smaller ones it
+// finds where this pass left them (whole calls, non-temporal -> cached: 4.5M
+// 32-bit columns in fp64 55.8 -> 53.7 us, 4.4M 64-bit ones in bf16 72.5 -> 65.0,
+// 20M 32-bit ones in fp32 116.6 -> 114.5); larger ones only push its other data
+// out (24M 32-bit columns 142 -> 149 us, 48M 243 -> 257, 36M 64-bit 288 -> 293).
+constexpr int64_t kAnNtBytes = (int64_t)80 << 20;
+
 template <typename I, typename P>
 int launch_analyze(const fs_csr* A, int64_t* st, const SplitOut* split, hipStream_t s) {
   const P* ptr = static_cast<const P*>(A->row_ptr);
@@ -311,10 +319,11 @@ int launch_analyze(const fs_csr* A, int64_t* st, const SplitOut* split, hipStrea
   // thread keeps eight 16-byte column loads in flight
   int64_t blocks = (work + kAnBlock * 32 - 1) / (kAnBlock * 32);
   if (blocks > 256) blocks = 256;
-  if (split)
-    analyze_pass<I, P, true><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st, *split);
-  else
-    analyze_pass<I, P, false><<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st, SplitOut{});
+  const bool nt = A->nnz * (int64_t)sizeof(I) > kAnNtBytes;
+  const SplitOut out = split ? *split : SplitOut{};
+  auto run = split ? (nt ? analyze_pass<I, P, true, true> : analyze_pass<I, P, true, false>)
+                   : (nt ? analyze_pass<I, P, false, true> : analyze_pass<I, P, false, false>);
+  run<<<(unsigned)blocks, kAnBlock, 0, s>>>(ptr, idx, A->n_rows, A->nnz, st, out);
   return check_launch("fs_csr_analyze");
 }
 
