@@ -27,7 +27,7 @@ reference (SciPy's CSR product in float64):
     random columns per row), N = 32 / 64 / 128 fp32 and N = 64 fp64, with a
     compulsory-bytes roofline (A once, B once, C once) and rocSPARSE beside it;
   * batched_512: 512 uneven matrices, one SpMV + one 8-column SpMM each, as one
-    graph-replayed persistent launch against the 1,024 separate launches;
+    graph-replayed launch against the 1,024 separate launches;
   * selection: on the 4M-row SpMV and the N = 64 SpMM, the learned choice
     against exhaustive autotuning (every variant timed) and the plain
     default-tile kernel;
@@ -370,7 +370,7 @@ def bench_sddmm(args):
 
 def bench_batched(args):
     """512 uneven CSR matrices, each with one SpMV and one 8-column SpMM, in
-    one persistent launch replayed from a HIP graph; beside it the 1,024
+    one launch replayed from a HIP graph; beside it the 1,024
     separate launches.  GB/s over the batch's algorithmic bytes."""
     import torch
     sys.path.insert(0, ROOT)
@@ -544,7 +544,7 @@ def sub_spmm_c3(steps, no_vendor=False):
 
 def sub_batched(steps):
     """512 uneven matrices (one SpMV, one 8-column SpMM each): graph replay of
-    the persistent launch, the same eagerly, and the 1,024 separate launches."""
+    the batched launch, the same eagerly, and the 1,024 separate launches."""
     import numpy as np
     import torch
     from flagsparse_public_amd.autotune import time_launches

@@ -445,7 +445,7 @@ int fs_spmv_csr_split(const fs_csr *A, int32_t format, const void *hi, const voi
 
 /* ------------------------------------------------------------ batched path */
 /*
- * Many independent fp32 / int32-column CSR problems in one persistent launch
+ * Many independent fp32 / int32-column CSR problems in one launch
  * (replayable from a captured graph).  No counterpart in the reference, which
  * launches per matrix and row bucket; used by callers with many small or
  * uneven matrices.
