@@ -12,8 +12,8 @@
 // end at which a block's lane groups wait for the longest row of many, and
 // blocks of both kinds share a CU.  32 matrices of 1,000 to 200,000 rows of 34
 // (44M entries), one SpMV and one 8-column SpMM each: persistent blocks on a
-// queue of 96 KB items, two lanes per SpMM row, 744 us; this form 613 us (SpMV
-// alone 440 -> 271, SpMM alone 515 -> 386).  What bounds it: the requests of the
+// queue of 96 KB items, two lanes per SpMM row, 744 us; this form 590 us (SpMV
+// alone 440 -> 248, SpMM alone 515 -> 376).  What bounds it: the requests of the
 // gathers to L2 and, for B beyond L2, the 128-byte lines behind them.  Small
 // batches no longer start and drain 2,048 blocks: 8 matrices of 15 to 3,000 rows
 // of 10 69.8 -> 6.2 us; 16 of 500 to 100,000 rows of 8, N = 12, 145 -> 69 us.
@@ -43,26 +43,101 @@ __device__ __forceinline__ int64_t bm_ptr(const BatchMatrix& m, int64_t r) {
                  : (int64_t) static_cast<const int32_t*>(m.row_ptr)[r];
 }
 
-// --- SpMV rows of an item with groups of S lanes (same procedure as the
-// single-matrix short role: accumulate_span<S, 4> then group_reduce<S>).
+// acc[r] += the products of row r's entries s[r] .. e[r] - 1 for lane g of S
+// (entries g, g + S, ...: accumulate_span's order), two entries of each of the
+// R rows in flight.
+template <int R, int S>
+__device__ __forceinline__ void bat_accumulate(Plain<float> (&acc)[R], const BatchMatrix& m,
+                                               const int64_t (&s)[R], const int64_t (&e)[R], int g) {
+  constexpr int U = 2;
+  int64_t j[R];
+  bool more = false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    j[r] = s[r] + g;
+    more |= j[r] < e[r];
+  }
+  while (more) {
+    int32_t ci[R][U];
+    float a[R][U], x[R][U];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool ok = j[r] + u * S < e[r];
+        ci[r][u] = ok ? m.col[j[r] + u * S] : 0;
+        a[r][u] = ok ? m.val[j[r] + u * S] : 0.f;
+      }
+    // the empty asm keeps each index's use (and the wait for its load) out of
+    // the masked load's branch, so all loads are issued before the first wait
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(ci[r][u]));
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[r][u] = j[r] + u * S < e[r] ? m.x[(int64_t)ci[r][u]] : 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(x[r][u]));
+    more = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j[r] + u * S < e[r]) acc[r].add_prod(a[r][u], x[r][u]);
+      j[r] += U * S;
+      more |= j[r] < e[r];
+    }
+  }
+}
+
+// --- SpMV rows of an item with groups of S lanes (the single-matrix short
+// role's lane order and group_reduce<S>).  A row of at most 2 S entries is one
+// round of loads for its group; wide groups take two rows at once, whose rounds
+// then overlap (32 matrices of rows of 34, SpMV alone: 268 -> 248 us, with the
+// SpMMs 610 -> 594; four rows: 315 and 796 us, their registers cost the whole
+// kernel wavefronts; 4-lane groups with two: 68.6 -> 69.5 us).  Rows over 8 S
+// entries take accumulate_span's deeper batches one by one.
 template <int S>
 __device__ void bat_spmv_rows(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha, double beta) {
-  constexpr int kGroups = kBatBlock / S;
+  constexpr int kGroups = kBatBlock / S, R = S >= 16 ? 2 : 1;
   const int grp = threadIdx.x / S, g = threadIdx.x % S;
   DirectVals<float> vs{m.val};
   // every group runs the same number of iterations so the S-lane exchange in
   // group_reduce always sees its whole group active
-  for (int64_t base = r0; base < r1; base += kGroups) {
-    const int64_t row = base + grp;
-    const bool live = row < r1;
-    Plain<float> acc;
-    acc.init();
-    if (live) {
-      const int64_t rs = bm_ptr(m, row), re = bm_ptr(m, row + 1);
-      accumulate_span<S, 4>(acc, m.col, vs, m.x, rs, re, g);
+  for (int64_t base = r0; base < r1; base += kGroups * R) {
+    int64_t s[R], e[R];
+    Plain<float> acc[R];
+    bool deep = R == 1;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t row = base + grp + r * kGroups;
+      const int64_t q = row < r1 ? row : r1 - 1;
+      s[r] = bm_ptr(m, q);
+      e[r] = bm_ptr(m, q + 1);
     }
-    group_reduce<S>(acc);
-    if (live && g == 0) write_out(m.y, row, acc.value(), alpha, beta);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (base + grp + r * kGroups >= r1) e[r] = s[r];
+      deep |= e[r] - s[r] > 8 * S;
+      acc[r].init();
+    }
+    if (deep) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) accumulate_span<S, 4>(acc[r], m.col, vs, m.x, s[r], e[r], g);
+    } else if constexpr (R > 1) {
+      bat_accumulate<R, S>(acc, m, s, e, g);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) group_reduce<S>(acc[r]);
+    if (g == 0)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (base + grp + r * kGroups < r1)
+          write_out(m.y, base + grp + r * kGroups, acc[r].value(), alpha, beta);
   }
 }
 
