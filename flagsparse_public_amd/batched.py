@@ -50,22 +50,18 @@ def _cuts(indptr, weight_per_entry, target, max_rows, long_row=None):
     marks = (torch.arange(step, nnz, step, device=dev, dtype=torch.int64) if nnz > step
              else torch.zeros(0, dtype=torch.int64, device=dev))
     by_nnz = torch.searchsorted(indptr[1:].to(torch.int64), marks, right=True)
-    by_rows = (torch.arange(max_rows, n, max_rows, device=dev, dtype=torch.int64) if n > max_rows
-               else torch.zeros(0, dtype=torch.int64, device=dev))
+    by_rows = torch.arange(0, n, max_rows, device=dev, dtype=torch.int64)
     if by_nnz.numel():
         # a range within the target stays whole: its rows fill the block's passes
         first = torch.clamp(by_nnz, max=n - 1) // max_rows * max_rows
         held = indptr[torch.clamp(first + max_rows, max=n)] - indptr[first]
         by_nnz = by_nnz[held * weight_per_entry > target]
-    parts = [torch.zeros(1, dtype=torch.int64, device=dev), by_nnz, by_rows,
-             torch.full((1,), n, dtype=torch.int64, device=dev)]
+    parts = [by_nnz, by_rows, torch.full((1,), n, dtype=torch.int64, device=dev)]
     if long_row is not None and n > 0:
         lens = indptr[1:] - indptr[:-1]
         long = torch.nonzero(lens > long_row, as_tuple=False).flatten().to(torch.int64)
         parts += [long, long + 1]
-    cuts = torch.cat(parts)
-    cuts = torch.unique(cuts)  # sorted
-    return cuts[(cuts >= 0) & (cuts <= n)]
+    return torch.unique(torch.cat(parts))  # sorted, all within 0 .. n
 
 
 class BatchedCsr:
@@ -150,9 +146,7 @@ class BatchedCsr:
 
     @staticmethod
     def _items(matrix, kind, cuts):
-        r0, r1 = cuts[:-1], cuts[1:]
-        keep = r1 > r0
-        r0, r1 = r0[keep], r1[keep]
+        r0, r1 = cuts[:-1], cuts[1:]  # each cut is there once: no empty range
         head = torch.full_like(r0, matrix | (kind << 32))
         return torch.stack([head, r0, r1], dim=1)
 
