@@ -12,7 +12,7 @@
 // end at which a block's lane groups wait for the longest row of many, and
 // blocks of both kinds share a CU.  32 matrices of 1,000 to 200,000 rows of 34
 // (44M entries), one SpMV and one 8-column SpMM each: persistent blocks on a
-// queue of 96 KB items, two lanes per SpMM row, 744 us; this form 590 us (SpMV
+// queue of 96 KB items, two lanes per SpMM row, 744 us; this form 587 us (SpMV
 // alone 440 -> 248, SpMM alone 515 -> 376).  What bounds it: the requests of the
 // gathers to L2 and, for B beyond L2, the 128-byte lines behind them.  Small
 // batches no longer start and drain 2,048 blocks: 8 matrices of 15 to 3,000 rows
@@ -98,7 +98,7 @@ __device__ __forceinline__ void bat_accumulate(Plain<float> (&acc)[R], const Bat
 // role's lane order and group_reduce<S>).  A row of at most 2 S entries is one
 // round of loads for its group; wide groups take two rows at once, whose rounds
 // then overlap (32 matrices of rows of 34, SpMV alone: 268 -> 248 us, with the
-// SpMMs 610 -> 594; four rows: 315 and 796 us, their registers cost the whole
+// SpMMs 605 -> 587; four rows: 315 and 796 us, their registers cost the whole
 // kernel wavefronts; 4-lane groups with two: 68.6 -> 69.5 us).  Rows over 8 S
 // entries take accumulate_span's deeper batches one by one.
 template <int S>
