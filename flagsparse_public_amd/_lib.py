@@ -392,8 +392,11 @@ def coo_sort(data, row, col, n_rows: int, n_cols: int, flags, index_dtype=None, 
     """Run fs_coo_sort on contiguous device arrays (row and col of one dtype);
     returns (values, rows or None, columns, row pointer) in CSR order, rows and
     columns as ``index_dtype`` (default: theirs).  ``flags`` (one int64 on the
-    device) receives the checks: read it before using the arrays."""
+    device) receives the checks: read it before using the arrays.  Values that
+    torch holds as a lazy conjugate or negative are written out first: the sort
+    moves what is in memory (``contiguous()`` leaves such a view as it is)."""
     lib = load()
+    data = data.resolve_conj().resolve_neg()
     device, nnz = data.device, data.numel()
     index_dtype = index_dtype or row.dtype
     out = torch.empty_like(data)
