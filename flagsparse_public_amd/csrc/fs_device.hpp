@@ -152,7 +152,8 @@ struct Comp {
     s = t;
     c += o.c + err;
   }
-  __device__ __forceinline__ float value() const { return s + c; }
+  // An infinite sum (or NaN) is the result itself: its correction is inf - inf.
+  __device__ __forceinline__ float value() const { return __builtin_isfinite(s) ? s + c : s; }
 };
 
 // f32c: a compensated fp32 sum held as a value pair (running sum s and the
