@@ -189,7 +189,8 @@ SPMM_CHUNK_BYTES = 1 << 27  # gathered bytes of a launch below which chunks shri
 
 def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int = 0) -> Schedule:
     """Which SpMM rows one lane group walks alone and which whole wavefronts
-    take in chunks.
+    take in chunks.  Every launch gives item_bytes, the bytes of a value; 0
+    leaves out what depends on them.
 
     A lane group walks its row serially (a round trip to the B rows per batch
     of entries), so the longest short row bounds the launch: rows over about
@@ -197,27 +198,37 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     us with rows up to 256 short, 96 us with 32; 60,000 fp64 rows, N = 16: 57
     against 22 us.  Below twice the mean, typical rows would leave the groups
     (100,000 rows of about 60, N = 64 in bf16: 90 us with 128, 119 with 64, 189
-    with 32); rows of 300, N = 64: 84 us with 1024 against 134 with 256.
+    with 32).  Rows over 256 entries are chunked whatever the mean: a group
+    sums a row in one chain per column, a chunk in several chains, which in
+    fp32 sums are compensated (fp32, N = 64, values of both signs, rms error of
+    20,000 rows of about 300 entries 7.7e-7 in chunks, 1.8e-6 in chains, of
+    40,000 rows of 600 3.0e-7 and 3.6e-6; the chains took 107 and 379 us, the
+    chunks take 154 and 484).
 
     With long rows and too few of them to fill the chip with lane groups,
     every row gets a wavefront: 5,000 rows of about 300, N = 16: 45 -> 12 us;
     20,000 rows, N = 8: 77 -> 37 us; at 30,000 rows of 100 the two meet (N = 8,
-    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us).
+    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us).  Its
+    chunks hold 512 entries where the chunk sums are compensated or in fp64
+    over fp32 values, 256 in fp64 and complex types, whose chains are then half
+    as long (2,000 fp64 rows of about 600, N = 130: rms error 4.2e-15 against
+    5.7e-15, 184 against 204 us).
 
-    The wider B (values of item_bytes each; 0 leaves this out), the fewer of a
-    chunk's entries its wavefront takes at once: 16 lanes a B row leave 64 round
-    trips for a chunk of 256, 64 lanes as many as it has entries.  Where a launch
-    gathers little, that chain is all of it and smaller chunks are faster, else
-    their partial sums cost more than they save.  Power-law rows, chunks of 64 /
-    128 / 256: 16,000 rows, N = 128 in fp32 (84 MB) 25 / 27 / 37 us, N = 160 in
-    bf16 (51 MB) 36 / 40 / 56; 4,000 rows, N = 160 in fp32 (23 MB) 19 / 25 / 40;
-    64,000 rows, N = 64 in fp32 (177 MB) 49 / 41 / 38."""
+    The wider B (values of item_bytes each), the fewer of a chunk's entries its
+    wavefront takes at once: 16 lanes a B row leave 64 round trips for a chunk
+    of 256, 64 lanes as many as it has entries.  Where a launch gathers little,
+    that chain is all of it and smaller chunks are faster, else their partial
+    sums cost more than they save.  Power-law rows, chunks of 64 / 128 / 256:
+    16,000 rows, N = 128 in fp32 (84 MB) 25 / 27 / 37 us, N = 160 in bf16 (51
+    MB) 36 / 40 / 56; 4,000 rows, N = 160 in fp32 (23 MB) 19 / 25 / 40; 64,000
+    rows, N = 64 in fp32 (177 MB) 49 / 41 / 38."""
     mean = nnz / n_rows if n_rows > 0 else 0.0
     lanes = max(8, _pow2_ceil(n_dense / 4.0))
     if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
-        return Schedule(group_lanes=1, short_max=32, chunk_nnz=512, unroll=4, col_tile=0)
-    short = 32
-    while short < 2 * mean and short < 1024:
+        chunk = 512 if item_bytes <= 4 else 256
+        return Schedule(group_lanes=1, short_max=32, chunk_nnz=chunk, unroll=4, col_tile=0)
+    short, most = 32, 256 if item_bytes else 1024
+    while short < 2 * mean and short < most:
         short *= 2
     chunk, row_bytes = 256, n_dense * item_bytes
     if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:

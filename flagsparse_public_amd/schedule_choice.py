@@ -61,7 +61,7 @@ def choose_schedule(op, request, data, n_rows, n_cols, stats_dev, indptr=None, i
     def fallback():
         if op == "spmv":
             return default_spmv_schedule(n_rows, nnz, data.dtype, n_cols, indptr, indices)
-        return default_spmm_schedule(n_rows, nnz, 64)
+        return default_spmm_schedule(n_rows, nnz, 64, data.element_size())
     if mode == "default" or n_rows == 0:
         return fallback(), "default"
     if mode == "exhaustive":
