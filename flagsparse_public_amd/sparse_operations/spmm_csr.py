@@ -19,6 +19,7 @@ import time
 import torch
 
 from .. import _lib
+from ..autotune import SPMM_VARIANTS
 from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule
 from ..schedule_choice import choose_schedule
 from ._common import (
@@ -561,11 +562,15 @@ def spmm_launch_schedule(prepared, n_dense, schedule=None):
         if known is not None and known[0] is prepared.schedule:
             return known[1]
         # the row split follows the mean row length whatever variant was
-        # chosen (the variants' own bounds were picked with longer short rows)
+        # chosen (the variants' own bounds were picked with longer short rows),
+        # but a variant that chunks shorter rows keeps doing so: their sums are
+        # compensated there
         split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
                                       prepared.data.element_size())
-        sch = dataclasses.replace(prepared.schedule or split, short_max=split.short_max,
-                                  chunk_nnz=split.chunk_nnz)
+        sch, short = prepared.schedule or split, split.short_max
+        if sch in SPMM_VARIANTS:
+            short = min(short, sch.short_max)
+        sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz)
         launch = _library_spmm_launch(sch, prepared.data.dtype, n_dense)
         prepared._plans[("launch", n_dense)] = (prepared.schedule, launch)
         return launch
