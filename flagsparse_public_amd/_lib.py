@@ -430,25 +430,36 @@ def split_lists(nnz: int, n_rows: int, short_max: int, chunk_nnz: int, device):
             buf[at + 2 * cap_long + 1:].view(torch.int32), cap_long, cap_chunks)
 
 
-def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bool, lists=None):
-    """Run fs_csr_analyze_split; returns (statistics on the host, long_rows,
-    long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed columns or None, the
-    spare word of ``lists``).  Entries of the lists past n_long / n_chunks are
-    unset.  ``lists``: from split_lists, where the caller uses the spare word."""
+def split_counts(word: int):
+    """(n_long, n_chunks) of analyze_split's packed count."""
+    return word >> SPLIT_CHUNK_BITS, word & ((1 << SPLIT_CHUNK_BITS) - 1)
+
+
+def enqueue_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, lists, cols32=None):
+    """Enqueue fs_csr_analyze_split into ``lists`` (split_lists): nothing is
+    read back."""
     lib = load()
-    nnz = int(csr.nnz)  # 0 for make_rows, which needs ``lists``
-    if lists is None:
-        lists = split_lists(nnz, int(csr.n_rows), short_max, chunk_nnz, device)
     buf, long_rows, long_chunk_ptr, chunk_long, cap_long, cap_chunks = lists
-    cols32 = torch.empty(nnz, dtype=torch.int32, device=device) if narrow else None
     with on_device(device):
         check(lib.fs_csr_analyze_split(ctypes.byref(csr), buf.data_ptr(), short_max, chunk_nnz,
                                        ptr(long_rows), long_chunk_ptr.data_ptr(), cap_long,
                                        ptr(chunk_long), cap_chunks, ptr(cols32),
                                        stream_handle(device)), "fs_csr_analyze_split")
+
+
+def analyze_split(csr: FsCsr, device, short_max: int, chunk_nnz: int, narrow: bool, lists=None):
+    """Run fs_csr_analyze_split; returns (statistics on the host, long_rows,
+    long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed columns or None, the
+    spare word of ``lists``).  Entries of the lists past n_long / n_chunks are
+    unset.  ``lists``: from split_lists, where the caller uses the spare word."""
+    nnz = int(csr.nnz)  # 0 for make_rows, which needs ``lists``
+    if lists is None:
+        lists = split_lists(nnz, int(csr.n_rows), short_max, chunk_nnz, device)
+    cols32 = torch.empty(nnz, dtype=torch.int32, device=device) if narrow else None
+    enqueue_split(csr, device, short_max, chunk_nnz, lists, cols32)
+    buf, long_rows, long_chunk_ptr, chunk_long = lists[:4]
     stats = buf[:FS_STATS_LEN + 2].cpu().tolist()
-    n_long = stats[FS_STATS_LEN] >> SPLIT_CHUNK_BITS
-    n_chunks = stats[FS_STATS_LEN] & ((1 << SPLIT_CHUNK_BITS) - 1)
+    n_long, n_chunks = split_counts(stats[FS_STATS_LEN])
     return (stats[:FS_STATS_LEN], long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, cols32,
             stats[FS_STATS_LEN + 1])
 

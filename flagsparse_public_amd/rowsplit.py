@@ -236,6 +236,16 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0)
 
 
+def spmm_split_widths(nnz: int, item_bytes: int) -> list[int]:
+    """Dense widths at which default_spmm_schedule may change, 1 first: every
+    split that it gives a matrix is that of one of these widths."""
+    widths = {1, 33, 65, 129, 128 // item_bytes + 1, 256 // item_bytes + 1}
+    if nnz > 0:
+        widths |= {-(-gathered // (nnz * item_bytes))
+                   for gathered in (SPMM_CHUNK_BYTES // 2, SPMM_CHUNK_BYTES)}
+    return sorted(widths)
+
+
 class RowSplitPlan:
     """Device metadata of one schedule for one matrix (see module docstring).
 
@@ -269,22 +279,16 @@ class RowSplitPlan:
             self.n_long, self.n_chunks = 0, 0
             self.tile_start, self.n_tiles = None, 0
             return
-        if (nnz is not None and nnz < 1 << 31 and n_rows > 0 and schedule.tile_nnz == 0
-                and schedule.short_max >= 1 and schedule.chunk_nnz > 0
-                and schedule.chunk_nnz % 64 == 0 and indptr.is_cuda):
+        if self._listed_natively(indptr, n_rows, nnz, schedule):
             # row groups of a matrix whose size the caller knows: one native pass
             # and one host read list the long rows (in any order) instead of a
             # dozen torch operators with three reads.  COO SpMV of 170,000
             # power-law rows, a new plan a call: 383 -> 264 us.
             lists = _lib.split_lists(nnz, n_rows, schedule.short_max, schedule.chunk_nnz, device)
-            _, rows, chunk_ptr, chunk_long, n_long, n_chunks, _, _ = _lib.analyze_split(
+            _, _, _, _, n_long, n_chunks, _, _ = _lib.analyze_split(
                 _lib.make_rows(indptr, n_rows), device, schedule.short_max, schedule.chunk_nnz,
                 False, lists)
-            if n_long <= lists[4] and n_chunks <= lists[5]:  # row pointers that match nnz
-                self.n_long, self.n_chunks = n_long, n_chunks
-                self.long_rows, self.long_chunk_ptr = rows[:n_long], chunk_ptr[:n_long + 1]
-                self.chunk_long = chunk_long[:n_chunks]
-                self.tile_start, self.n_tiles = None, 0
+            if self._take_lists(lists, n_long, n_chunks):
                 return
         if row_lengths is None:
             row_lengths = (indptr[1:].to(torch.int64) - indptr[:-1].to(torch.int64)) if n_rows > 0 \
@@ -312,6 +316,46 @@ class RowSplitPlan:
         else:
             self.tile_start = None
             self.n_tiles = 0
+
+    @staticmethod
+    def _listed_natively(indptr, n_rows, nnz, schedule):
+        """Whether fs_csr_analyze_split lists this plan's rows."""
+        return (nnz is not None and nnz < 1 << 31 and n_rows > 0 and schedule.tile_nnz == 0
+                and schedule.short_max >= 1 and schedule.chunk_nnz > 0
+                and schedule.chunk_nnz % 64 == 0 and indptr.is_cuda)
+
+    def _take_lists(self, lists, n_long, n_chunks):
+        """Takes the lists of one native pass; False (nothing taken) where they
+        do not hold the counts: row pointers that do not match nnz."""
+        _, rows, chunk_ptr, chunk_long, cap_long, cap_chunks = lists
+        if n_long > cap_long or n_chunks > cap_chunks:
+            return False
+        self.n_long, self.n_chunks = n_long, n_chunks
+        self.long_rows, self.long_chunk_ptr = rows[:n_long], chunk_ptr[:n_long + 1]
+        self.chunk_long = chunk_long[:n_chunks]
+        self.tile_start, self.n_tiles = None, 0
+        return True
+
+    @classmethod
+    def several(cls, indptr, n_rows, value_dtype, schedules, accumulate, nnz, row_lengths=None):
+        """Plans of several row-group schedules for one matrix: a native pass
+        each, one host read together."""
+        csr, lists = _lib.make_rows(indptr, n_rows), {}
+        for s in schedules:
+            if cls._listed_natively(indptr, n_rows, nnz, s):
+                lists[s] = _lib.split_lists(nnz, n_rows, s.short_max, s.chunk_nnz, indptr.device)
+                _lib.enqueue_split(csr, indptr.device, s.short_max, s.chunk_nnz, lists[s])
+        words = torch.cat([li[0][_lib.FS_STATS_LEN:_lib.FS_STATS_LEN + 1]
+                           for li in lists.values()]).cpu().tolist() if lists else []
+        counts = {s: _lib.split_counts(word) for s, word in zip(lists, words)}
+        plans = []
+        for s in schedules:
+            p = None
+            if s in lists:
+                p = cls.listed(s, accumulate, value_dtype, indptr.device, None, None, None, 0, 0)
+                p = p if p._take_lists(lists[s], *counts[s]) else None
+            plans.append(p or cls(indptr, n_rows, value_dtype, s, accumulate, row_lengths))
+        return plans
 
     @classmethod
     def listed(cls, schedule: Schedule, accumulate: int, value_dtype, device, long_rows,

@@ -20,7 +20,7 @@ import torch
 
 from .. import _lib
 from ..autotune import SPMM_VARIANTS
-from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule
+from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule, spmm_split_widths
 from ..schedule_choice import choose_schedule
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
@@ -266,13 +266,25 @@ def _resolve_spmm_alg1_launch_config(n_dense_cols, max_row_nnz, block_n=None, bl
 
 # ---------------------------------------------------------------- launches
 
-def _plan_for(cache, kernel_indptr, n_rows, dtype, accumulate, schedule, row_lengths, nnz=None):
-    key = (int(accumulate), schedule.key())
-    p = cache.get(key)
+def _spmm_plan(prepared, accumulate, schedule):
+    """The plan of one schedule of a prepared matrix.  The row split follows
+    the dense width, so with the first of the library's schedules those of all
+    widths get their plans: later calls list nothing and read nothing back,
+    whatever their width, and can be captured."""
+    acc, plans = int(accumulate), prepared._plans
+    p = plans.get((acc, schedule.key()))
     if p is None:
-        p = RowSplitPlan(kernel_indptr, n_rows, dtype, schedule, accumulate,
-                         row_lengths=row_lengths, nnz=nnz)
-        cache[key] = p
+        schedules = [schedule]
+        if prepared.library_schedule:
+            widths = spmm_split_widths(prepared.data.numel(), prepared.data.element_size())
+            of_widths = dict.fromkeys(_library_schedule(prepared, n)[0] for n in widths)
+            if schedule in of_widths:
+                schedules = [s for s in of_widths if (acc, s.key()) not in plans]
+        for s, q in zip(schedules, RowSplitPlan.several(
+                prepared.kernel_indptr, prepared.n_rows, prepared.data.dtype, schedules, acc,
+                prepared.data.numel(), prepared.row_lengths)):
+            plans[acc, s.key()] = q
+        p = plans[acc, schedule.key()]
     return p
 
 
@@ -433,8 +445,7 @@ class PreparedCsrSpmmOpt:
     def plan(self, accumulate, n_dense, schedule=None):
         sch = schedule or self.schedule or default_spmm_schedule(
             self.n_rows, self.data.numel(), n_dense, self.data.element_size())
-        return _plan_for(self._plans, self.kernel_indptr, self.n_rows, self.data.dtype,
-                         accumulate, sch, self.row_lengths, self.data.numel())
+        return _spmm_plan(self, accumulate, sch)
 
 
 _SPMM_OPT_BUCKET_SPECS = (
@@ -554,6 +565,20 @@ def _library_spmm_launch(sch, dtype, n_dense):
     return sch, col_tile
 
 
+def _library_schedule(prepared, n_dense):
+    """(schedule, column tile) for n_dense columns where the library chooses.
+    The row split follows the mean row length whatever variant was chosen (the
+    variants' own bounds were picked with longer short rows), but a variant
+    that chunks shorter rows keeps doing so: their sums are compensated there."""
+    split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
+                                  prepared.data.element_size())
+    sch, short = prepared.schedule or split, split.short_max
+    if sch in SPMM_VARIANTS:
+        short = min(short, sch.short_max)
+    sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz)
+    return _library_spmm_launch(sch, prepared.data.dtype, n_dense)
+
+
 def spmm_launch_schedule(prepared, n_dense, schedule=None):
     """The (schedule, column tile) an opt / alg2 SpMM call with n_dense
     columns launches."""
@@ -561,17 +586,7 @@ def spmm_launch_schedule(prepared, n_dense, schedule=None):
         known = prepared._plans.get(("launch", n_dense))
         if known is not None and known[0] is prepared.schedule:
             return known[1]
-        # the row split follows the mean row length whatever variant was
-        # chosen (the variants' own bounds were picked with longer short rows),
-        # but a variant that chunks shorter rows keeps doing so: their sums are
-        # compensated there
-        split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
-                                      prepared.data.element_size())
-        sch, short = prepared.schedule or split, split.short_max
-        if sch in SPMM_VARIANTS:
-            short = min(short, sch.short_max)
-        sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz)
-        launch = _library_spmm_launch(sch, prepared.data.dtype, n_dense)
+        launch = _library_schedule(prepared, n_dense)
         prepared._plans[("launch", n_dense)] = (prepared.schedule, launch)
         return launch
     sch = schedule or prepared.schedule or default_spmm_schedule(

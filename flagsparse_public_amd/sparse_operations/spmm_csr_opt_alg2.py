@@ -20,9 +20,9 @@ from ..schedule_choice import choose_schedule
 from ._common import _INDEX_LIMIT_INT32
 from .spmm_csr import (  # noqa: F401  (re-exported like the reference)
     _launch_spmm,
-    _plan_for,
     _prepare_spmm_csr_matrix,
     _spmm_coo_reference_tolerance,
+    _spmm_plan,
     _spmm_target,
     _spmm_validation_metrics,
     flagsparse_spmm_csr,
@@ -253,8 +253,7 @@ def _hip_spmm_csr_impl_opt_alg2_prepared(prepared, B, return_meta=False, out=Non
     device_props = _normalize_spmm_opt_alg2_device_props(prepared.data.device)
     n_dense = int(B.shape[1])
     sch, col_tile = spmm_launch_schedule(prepared, n_dense, schedule)
-    plan = _plan_for(prepared._plans, prepared.kernel_indptr, prepared.n_rows,
-                     prepared.data.dtype, _lib.FS_ACC_NATIVE, sch, prepared.row_lengths)
+    plan = _spmm_plan(prepared, _lib.FS_ACC_NATIVE, sch)
     C = _launch_spmm(prepared.csr_struct(), plan, B, prepared.n_rows, n_dense, B.dtype, B.device,
                      out, alpha, beta, col_tile)
     meta = None
