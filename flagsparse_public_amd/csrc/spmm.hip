@@ -332,8 +332,8 @@ __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> 
   write_vec<G, VW>(p.C, row * p.ldc + n0, acc, p.alpha, p.beta, skip);
 }
 
-// Whether each XCD takes a contiguous range of rows (xcd_remap_block) although
-// the plan does not ask for it.  Neighbouring rows of matrices from meshes gather
+// Whether each XCD takes a contiguous range of rows (xcd_remap_block) where the
+// plan leaves it to the launch.  Neighbouring rows of matrices from meshes gather
 // the same B rows, which one L2 then holds once; dealt in turn, blocks bring them
 // into all eight.  fp32 / fp64, banded rows of 15: 1M rows N = 64 362 -> 351 us,
 // N = 100 705 -> 643; 300,000 rows N = 100 210 -> 194, fp64 405 -> 345 us.  Random
@@ -372,7 +372,8 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
   p.long_chunk_ptr = pl->long_chunk_ptr;
   p.chunk_long = pl->chunk_long;
   p.partials = pl->partials;
-  p.xcd_remap = pl->xcd_remap || spmm_xcd_rows<V>(M, n_dense, p.n_tiles, pl);
+  p.xcd_remap = pl->xcd_remap == FS_XCD_AUTO ? spmm_xcd_rows<V>(M, n_dense, p.n_tiles, pl)
+                                             : pl->xcd_remap != 0;
   const int64_t rows_per_block = kMmBlock / G;
   const int64_t short_blocks = ((M->n_rows + rows_per_block - 1) / rows_per_block) * p.n_tiles;
   const int64_t grid = p.n_chunk_blocks + short_blocks;
@@ -427,7 +428,8 @@ int launch_spmm_g(int G, const fs_csr* M, const void* B, int64_t ldb, void* C, i
   }
 }
 
-// Whether B rows are cut into tiles of one 128-byte line.  Tiles of one row go
+// Whether B rows are cut into tiles of one 128-byte line, where plan and column
+// tile leave it to the launch.  Tiles of one row go
 // to neighbouring blocks, which the XCDs take in turn, so with 2, 4 or 8 tiles
 // an XCD gathers only its part of every B row, and its L2 (4 MB) holds that many
 // times as many rows.  That pays where B does not fit one L2 and one tile of it
@@ -453,7 +455,8 @@ int launch_spmm(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t ld
                 double alpha, double beta, const fs_plan* pl, int32_t col_tile, hipStream_t st) {
   constexpr int kMax = kMaxVw<V, I>;
   if constexpr (std::is_same<I, int32_t>::value && kMax * sizeof(V) == 16 && kMax > 1)
-    if (col_tile == 0 && spmm_line_tiles(M, n_dense * (int64_t)sizeof(V), pl))
+    if (col_tile == 0 && pl->xcd_remap == FS_XCD_AUTO &&
+        spmm_line_tiles(M, n_dense * (int64_t)sizeof(V), pl))
       return launch_spmm_g<V, A, I, P, kMax>(8, M, B, ldb, C, ldc, n_dense, alpha, beta, pl, st);
   // fp64, B rows of 1 KB and more: tiles of 512 bytes unless the last would be
   // mostly idle.  Tiles of one row go to neighbouring blocks, so with two

@@ -28,7 +28,8 @@ class Schedule:
     short_max: int = 128      # longest row of the short role
     chunk_nnz: int = 512      # entries per long-row chunk (multiple of 64)
     unroll: int = 4           # entries in flight per lane
-    xcd_remap: int = 0        # 1: contiguous row ranges per XCD
+    xcd_remap: int = 0        # 1: contiguous row ranges per XCD (FS_XCD_AUTO: SpMM's
+                              # launch rules choose; the library's own schedules)
     col_tile: int = 0         # SpMM dense columns per lane group (0: all)
     tile_nnz: int = 0         # SpMV: > 0 selects the tile role for short rows
     x_slice_cols: int = 0     # SpMV native path: > 0 cuts the columns into slices of
@@ -226,14 +227,16 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     lanes = max(8, _pow2_ceil(n_dense / 4.0))
     if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
         chunk = 512 if item_bytes <= 4 else 256
-        return Schedule(group_lanes=1, short_max=32, chunk_nnz=chunk, unroll=4, col_tile=0)
+        return Schedule(group_lanes=1, short_max=32, chunk_nnz=chunk, unroll=4, col_tile=0,
+                        xcd_remap=_lib.FS_XCD_AUTO)
     short, most = 32, 256 if item_bytes else 1024
     while short < 2 * mean and short < most:
         short *= 2
     chunk, row_bytes = 256, n_dense * item_bytes
     if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:
         chunk = 64 if row_bytes > 256 and nnz * row_bytes < SPMM_CHUNK_BYTES // 2 else 128
-    return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0)
+    return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0,
+                    xcd_remap=_lib.FS_XCD_AUTO)
 
 
 def spmm_split_widths(nnz: int, item_bytes: int) -> list[int]:

@@ -575,7 +575,8 @@ def _library_schedule(prepared, n_dense):
     sch, short = prepared.schedule or split, split.short_max
     if sch in SPMM_VARIANTS:
         short = min(short, sch.short_max)
-    sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz)
+    sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz,
+                              xcd_remap=sch.xcd_remap or _lib.FS_XCD_AUTO)
     return _library_spmm_launch(sch, prepared.data.dtype, n_dense)
 
 

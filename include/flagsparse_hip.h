@@ -101,10 +101,13 @@ typedef struct fs_csr {
  * at most 2 * tile_nnz entries and either only rows of length <= short_max
  * or exactly one longer row (left to the chunk role); short_max <= tile_nnz.
  */
+#define FS_XCD_AUTO 2
 typedef struct fs_plan {
   int32_t accumulate;      /* FS_ACC_*                                     */
   int32_t group_lanes;     /* SpMV lanes per short row: 1,2,4,8,16,32,64   */
-  int32_t xcd_remap;       /* 1: give each XCD a contiguous range of rows  */
+  int32_t xcd_remap;       /* 1: give each XCD a contiguous range of rows;
+                              FS_XCD_AUTO (SpMM): by the launch's own rules,
+                              column tiles of B among them if col_tile is 0  */
   int32_t unroll;          /* entries in flight per lane: 1, 2, 4 or 8     */
   int64_t short_max;       /* longest row handled by the short-row role    */
   int64_t chunk_nnz;       /* entries per long-row chunk (multiple of 64)  */
