@@ -71,15 +71,17 @@ def _normalize_spmv_coo_index_fallback_policy(index_fallback_policy):
     return policy
 
 
-_SEGS_ON_READ = object()
+_STATS_EMPTY_ROWS = 8  # place in the statistics of fs_csr_analyze
 
 
 class PreparedCoo:
     """Sorted COO + row-run bounds ``seg_starts`` (spmv_coo.py:77-129), plus
     the row pointer of the sorted entries for the CSR kernels."""
 
-    __slots__ = ("data", "row", "col", "shape", "n_rows", "n_cols", "nnz", "_seg_starts", "use_seg_kernel", "op", "transpose", "index_fallback_policy",
-                 "index_fallback_applied", "index_fallback_reason", "_csr", "_ordered")
+    __slots__ = ("data", "row", "col", "shape", "n_rows", "n_cols", "nnz", "_seg_starts",
+                 "_segs_on_read", "n_segs", "use_seg_kernel", "op", "transpose",
+                 "index_fallback_policy", "index_fallback_applied", "index_fallback_reason",
+                 "_csr", "_ordered")
 
     def __init__(self, data, row, col, shape, seg_starts=None, transpose=False, op=None,
                  index_fallback_policy="auto", index_fallback_applied=False,
@@ -91,12 +93,9 @@ class PreparedCoo:
         self.n_rows, self.n_cols = self.shape
         self.nnz = int(data.numel())
         self._seg_starts = seg_starts
-        if seg_starts is None:
-            self.use_seg_kernel = False
-        elif seg_starts is _SEGS_ON_READ:
-            self.use_seg_kernel = self.nnz > 0
-        else:
-            self.use_seg_kernel = int(seg_starts.numel()) > 1
+        self._segs_on_read = False  # whether seg_starts is still to be built
+        self.n_segs = 0 if seg_starts is None else int(seg_starts.numel()) - 1
+        self.use_seg_kernel = self.n_segs > 0
         self.op = _normalize_spmv_coo_op(op, transpose=transpose)
         self.transpose = _spmv_coo_op_transposes(self.op)
         self.index_fallback_policy = str(index_fallback_policy).lower()
@@ -109,19 +108,17 @@ class PreparedCoo:
 
     @property
     def seg_starts(self):
-        """Bounds of the constant-row runs; built on first read where the
-        constructor was told so (no kernel here reads them)."""
-        if self._seg_starts is _SEGS_ON_READ:
+        """Bounds of the constant-row runs; built on first read after the
+        native sort (no kernel here reads them)."""
+        if self._segs_on_read:
             self._seg_starts = _seg_starts_from_sorted_rows(self.row, self.nnz, self.data.device)
+            self._segs_on_read = False
         return self._seg_starts
 
     @seg_starts.setter
     def seg_starts(self, value):
         self._seg_starts = value
-
-    @property
-    def n_segs(self):
-        return 0 if self.seg_starts is None else int(self.seg_starts.numel()) - 1
+        self._segs_on_read = False
 
 
 def _sort_coo_lex(data, row, col, n_cols):
@@ -164,7 +161,6 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
     if col.dtype not in SUPPORTED_INDEX_DTYPES:
         raise TypeError("col dtype must be torch.int32 or torch.int64")
     # both orders are sorted here (deterministic sums); seg_starts only when asked
-    seg = _SEGS_ON_READ if sort_by_row and data.numel() > 0 else None
     if (_lib.coo_sort_applies(data.numel(), n_rows, n_cols) and row.device == data.device
             and col.device == data.device):
         # one native sort that also checks the index ranges, the analysis of
@@ -190,8 +186,9 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
         if bad & _lib.COO_BAD_COL:
             raise IndexError("col indices out of range")
         if bad == 0:
-            return d, kr, kc, seg, (indptr, stats_dev, stats[:_lib.FS_STATS_LEN], chosen)
+            return d, kr, kc, None, (indptr, stats_dev, stats[:_lib.FS_STATS_LEN], chosen)
     data, kr, kc = _sort_coo_lex(data, row, col, n_cols)
+    seg = _seg_starts_from_sorted_rows(kr, data.numel(), data.device) if sort_by_row else None
     if data.numel() > 0:
         r64, c64 = kr.to(torch.int64), kc.to(torch.int64)
         if int(r64.min().item()) < 0 or int(r64.max().item()) >= n_rows:
@@ -220,6 +217,9 @@ def prepare_spmv_coo(data, row, col, shape, sort_by_row=True, transpose=False, o
     prepared = PreparedCoo(d, kr, kc, shape, seg_starts=seg, transpose=transpose, op=op_code,
                            index_fallback_policy=index_fallback_policy)
     prepared._ordered = ordered
+    if ordered is not None and sort_by_row:
+        prepared.n_segs = prepared.n_rows - ordered[2][_STATS_EMPTY_ROWS]
+        prepared.use_seg_kernel = prepared._segs_on_read = True  # nnz > 0
     return prepared
 
 
