@@ -102,8 +102,7 @@ class PreparedCoo:
         self.index_fallback_applied = bool(index_fallback_applied)
         self.index_fallback_reason = index_fallback_reason
         self._csr = None
-        # (row pointer, device and host statistics, chosen variant) of the
-        # native sort, until _csr_of
+        # _sorted_order of the native sort, until _csr_of
         self._ordered = None
 
     @property
@@ -186,7 +185,8 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
         if bad & _lib.COO_BAD_COL:
             raise IndexError("col indices out of range")
         if bad == 0:
-            return d, kr, kc, None, (indptr, stats_dev, stats[:_lib.FS_STATS_LEN], chosen)
+            return d, kr, kc, None, _sorted_order((d, kr, kc), indptr, stats_dev,
+                                                  stats[:_lib.FS_STATS_LEN], chosen)
     data, kr, kc = _sort_coo_lex(data, row, col, n_cols)
     seg = _seg_starts_from_sorted_rows(kr, data.numel(), data.device) if sort_by_row else None
     if data.numel() > 0:
@@ -218,7 +218,7 @@ def prepare_spmv_coo(data, row, col, shape, sort_by_row=True, transpose=False, o
                            index_fallback_policy=index_fallback_policy)
     prepared._ordered = ordered
     if ordered is not None and sort_by_row:
-        prepared.n_segs = prepared.n_rows - ordered[2][_STATS_EMPTY_ROWS]
+        prepared.n_segs = prepared.n_rows - ordered[4][_STATS_EMPTY_ROWS]
         prepared.use_seg_kernel = prepared._segs_on_read = True  # nnz > 0
     return prepared
 
@@ -240,16 +240,31 @@ def _validate_x_coo(x, prepared):
     return x.contiguous()
 
 
+def _versions(arrays):
+    """Counts of in-place writes (tensors made in inference mode have none)."""
+    return [None if t.is_inference() else t._version for t in arrays]
+
+
+def _sorted_order(arrays, indptr, stats_dev, stats, chosen):
+    """What the native sort found for its sorted (data, row, col): their row
+    pointer, the device and host statistics, the chosen variant."""
+    return arrays, _versions(arrays[1:]), indptr, stats_dev, stats, chosen
+
+
 def _csr_of(prepared):
-    """PreparedCsrSpmv over the sorted entries (row pointer from the rows)."""
+    """PreparedCsrSpmv over the sorted entries (row pointer from the rows).
+    Arrays that were set or written to since the sort are looked at anew."""
     if prepared._csr is None:
         from .spmv_csr import prepare_spmv_csr
-        if prepared._ordered is not None:
-            indptr, *analyzed = prepared._ordered
-            prepared._csr = prepare_spmv_csr(prepared.data, prepared.col, indptr, prepared.shape,
-                                             _analyzed=analyzed)
-            prepared._ordered = None
-            return prepared._csr
+        ordered = prepared._ordered  # read once: other threads may be here
+        held = (prepared.data, prepared.row, prepared.col)
+        if (ordered is not None and all(a is b for a, b in zip(ordered[0], held))
+                and ordered[1] == _versions(held[1:])):
+            _, _, indptr, *analyzed = ordered
+            csr = prepare_spmv_csr(prepared.data, prepared.col, indptr, prepared.shape,
+                                   _analyzed=analyzed)
+            prepared._csr, prepared._ordered = csr, None
+            return csr
         counts = torch.bincount(prepared.row.to(torch.int64), minlength=prepared.n_rows)
         ptr_dtype = torch.int32 if prepared.nnz <= _INDEX_LIMIT_INT32 else torch.int64
         indptr = torch.zeros(prepared.n_rows + 1, dtype=torch.int64, device=prepared.data.device)

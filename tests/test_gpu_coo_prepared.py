@@ -1,4 +1,5 @@
-"""PreparedCoo as an object: copies, saved files, its run bounds and counts."""
+"""PreparedCoo as an object: copies, saved files, its run bounds and counts, arrays
+set before the first product."""
 
 import copy
 import io
@@ -50,3 +51,30 @@ def test_n_segs_is_a_plain_number(monkeypatch):
     p.n_segs = 5
     assert p.n_segs == 5
     assert prepare_spmv_coo(*args, (N, M), sort_by_row=False).n_segs == 0
+
+
+def test_arrays_set_before_the_first_product():
+    """A product takes the arrays that the object holds at that time."""
+    args, dense, _ = _entries()
+    x = torch.arange(M, device=DEV, dtype=torch.float64)
+    other = torch.sort(torch.randint(0, N, (NNZ,), device=DEV)).values
+    p = prepare_spmv_coo(*args, (N, M))
+    p.row = other
+    want = torch.zeros((N, M), dtype=torch.float64, device=DEV)
+    want.index_put_((other, p.col), p.data, accumulate=True)
+    assert torch.equal(flagsparse_spmv_coo(x=x, prepared=p), want @ x)
+    p = prepare_spmv_coo(*args, (N, M))
+    p.row.copy_(other)
+    assert torch.equal(flagsparse_spmv_coo(x=x, prepared=p), want @ x)
+    p = prepare_spmv_coo(*args, (N, M))
+    p.data.mul_(2)  # values alone may change
+    assert torch.equal(flagsparse_spmv_coo(x=x, prepared=p), 2 * (dense @ x))
+
+
+def test_columns_set_before_the_first_product_are_checked():
+    args, _, _ = _entries()
+    x = torch.ones(M, device=DEV, dtype=torch.float64)
+    p = prepare_spmv_coo(*args, (N, M))
+    p.col[7] = M
+    with pytest.raises(IndexError):
+        flagsparse_spmv_coo(x=x, prepared=p)
