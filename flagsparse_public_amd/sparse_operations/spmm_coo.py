@@ -115,14 +115,13 @@ def _sorted_csr(data, row, col, n_rows):
     return data[order].contiguous(), col[order].contiguous(), indptr
 
 
-def _native_spmm_coo_csr(data, row, col, B, shape):
-    """The entries in CSR order with their row-split plan, by fs_coo_sort and
-    fs_csr_analyze_split with one host read for the index checks and the
-    lists: (values, columns, row pointer, plan), or None where the sort does not
-    apply.  The sort orders equal (row, col) pairs by input position, as
-    _sorted_csr does."""
+def _native_spmm_coo_csr(data, row, col, B, n_rows, n_cols):
+    """The entries (arrays of _check_spmm_coo_arrays) in CSR order with their
+    row-split plan, by fs_coo_sort and fs_csr_analyze_split with one host read
+    for the index checks and the lists: (values, columns, row pointer, plan),
+    or None where the sort does not apply.  The sort orders equal (row, col)
+    pairs by input position, as _sorted_csr does."""
     from .spmm_csr import _spmm_default_accumulate
-    n_rows, n_cols = _check_spmm_coo_arrays(data, row, col, B, shape)
     nnz, n_dense, device = data.numel(), int(B.shape[1]), data.device
     if not _lib.coo_sort_applies(nnz, n_rows, n_cols):
         return None
@@ -155,16 +154,20 @@ def _run_spmm_coo_route(data, row, col, B, shape, block_n=None, block_nnz=256, o
         raise ValueError("block_n must be positive when provided")
     if block_nnz is not None and block_nnz <= 0:
         raise ValueError("block_nnz must be positive when provided")
-    t0 = None
-    if return_time and torch.cuda.is_available():
+    n_rows, n_cols = _check_spmm_coo_arrays(data, row, col, B, shape)
+    n_dense = int(B.shape[1])
+
+    def start_clock():
+        if not return_time:
+            return None
         torch.cuda.synchronize()
-        t0 = time.perf_counter()
-    native = _native_spmm_coo_csr(data, row, col, B, shape)
+        return time.perf_counter()
+    # a timed call times the sort (whose passes check the indices) and the product
+    t0 = start_clock()
+    native = _native_spmm_coo_csr(data, row, col, B, n_rows, n_cols)
     if native is None:
-        data, krow, kcol, B, n_rows, n_cols, n_dense = _prepare_spmm_coo_inputs(data, row, col, B,
-                                                                               shape)
-    else:
-        n_rows, n_cols, n_dense = int(shape[0]), int(shape[1]), int(B.shape[1])
+        data, krow, kcol, B, *_ = _prepare_spmm_coo_inputs(data, row, col, B, shape)
+        t0 = start_clock()
     _resolve_spmm_coo_launch_config(n_dense, data.numel(), block_n=block_n, block_nnz=block_nnz)
     if out is not None:
         if not out.is_cuda:
