@@ -314,7 +314,14 @@ extern "C" int fs_batch_run(const void* packed_dev, int64_t n_matrices, const fs
   if (long_row < 1) return fail(FS_ERR_VALUE, "fs_batch_run: long_row must be >= 1");
   if (n_items + (int64_t)grid > (int64_t)INT32_MAX)
     return fail(FS_ERR_UNSUPPORTED, "fs_batch_run: n_items + grid must stay below 2^31 - 1");
-  batched_kernel<<<(unsigned)n_items, kBatBlock, 0, as_stream(stream)>>>(
-      static_cast<const BatchMatrix*>(packed_dev), items, long_row, alpha, beta);
-  return check_launch("fs_batch_run");
+  // a launch holds fewer than 2^32 work-items: long lists go in several
+  constexpr int64_t kMost = (int64_t)1 << 23;
+  for (int64_t i = 0; i < n_items; i += kMost) {
+    const int64_t n = n_items - i < kMost ? n_items - i : kMost;
+    batched_kernel<<<(unsigned)n, kBatBlock, 0, as_stream(stream)>>>(
+        static_cast<const BatchMatrix*>(packed_dev), items + i, long_row, alpha, beta);
+    const int rc = check_launch("fs_batch_run");
+    if (rc) return rc;
+  }
+  return FS_OK;
 }
