@@ -298,7 +298,9 @@ extern "C" int fs_batch_rows(int32_t group_lanes, int64_t n_dense) {
   // SpMV: four rows per lane group (8 or 64 of 32 rows: 287 / 274 against 271 us
   // on the batch above), enough to pay for a block's start; SpMM: one (two: 413
   // against 382 us, the block waits for the longer of more rows)
-  if (n_dense <= 0) return group_lanes > 0 ? 4 * (kBatBlock / group_lanes) : kBatBlock;
+  // (lanes that fs_batch_pack refuses get some positive count here)
+  if (n_dense <= 0)
+    return group_lanes > 0 && group_lanes <= kWave ? 4 * (kBatBlock / group_lanes) : kBatBlock;
   int vw = 1, lanes = 1;
   spmm_tile_shape<4>(n_dense, 0, &vw, &lanes);
   return kBatBlock / (lanes < 4 ? 4 : lanes);
