@@ -45,8 +45,13 @@ struct SpmmParams {
   const int64_t* long_chunk_ptr;
   const int32_t* chunk_long;
   void* partials;     // [n_chunks * n_dense] accumulators
+  int64_t n_blocks;   // of all launches of the kernel
+  int64_t block0;     // first block of this one
   int xcd_remap;
 };
+
+// A launch holds fewer than 2^32 work-items: larger grids go in several.
+constexpr int64_t kMmMostBlocks = ((int64_t)1 << 32) / kMmBlock - 1;
 
 template <typename V, typename A, typename I, typename P, int G, int VW, int U>
 __device__ __forceinline__ void spmm_chunk_role(const SpmmParams<V, I, P>& p, int64_t bid) {
@@ -293,13 +298,13 @@ __device__ __forceinline__ void spmm_staged_rows(const SpmmParams<V, I, P>& p, i
 
 template <typename V, typename A, typename I, typename P, int G, int VW, int U>
 __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> p) {
-  const int64_t bid = blockIdx.x;
+  const int64_t bid = p.block0 + blockIdx.x;
   if (bid < p.n_chunk_blocks) {
     spmm_chunk_role<V, A, I, P, G, VW, U>(p, bid);
     return;
   }
   int64_t sb = bid - p.n_chunk_blocks;
-  if (p.xcd_remap) sb = xcd_remap_block(sb, (int64_t)gridDim.x - p.n_chunk_blocks);
+  if (p.xcd_remap) sb = xcd_remap_block(sb, p.n_blocks - p.n_chunk_blocks);
   const int64_t tile = sb % p.n_tiles, rb = sb / p.n_tiles;
   const int64_t row = rb * (kMmBlock / G) + threadIdx.x / G;
   const int g = threadIdx.x % G;
@@ -382,17 +387,17 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
     return fail(FS_ERR_UNSUPPORTED, "fs_spmm_csr: grid of %lld blocks too large", (long long)grid);
   // entries in flight per lane: 8 on request for fp32 / fp64 with int32
   // columns (short rows then finish in one or two batches), else 4
-  bool launched = false;
-  if constexpr (kHotSpmm<V, I>) {
-    if (pl->unroll >= 8) {
-      spmm_csr_kernel<V, A, I, P, G, VW, 8><<<dim3((unsigned)grid), dim3(kMmBlock), 0, st>>>(p);
-      launched = true;
-    }
+  auto kernel = spmm_csr_kernel<V, A, I, P, G, VW, 4>;
+  if constexpr (kHotSpmm<V, I>)
+    if (pl->unroll >= 8) kernel = spmm_csr_kernel<V, A, I, P, G, VW, 8>;
+  p.n_blocks = grid;
+  for (p.block0 = 0; p.block0 < grid; p.block0 += kMmMostBlocks) {
+    const int64_t n = grid - p.block0 < kMmMostBlocks ? grid - p.block0 : kMmMostBlocks;
+    kernel<<<dim3((unsigned)n), dim3(kMmBlock), 0, st>>>(p);
+    const int rc = check_launch("fs_spmm_csr");
+    if (rc) return rc;
   }
-  if (!launched)
-    spmm_csr_kernel<V, A, I, P, G, VW, 4><<<dim3((unsigned)grid), dim3(kMmBlock), 0, st>>>(p);
-  int rc = check_launch("fs_spmm_csr");
-  if (rc || pl->n_chunks <= pl->n_long) return rc;  // no row spans several chunks
+  if (pl->n_chunks <= pl->n_long) return FS_OK;  // no row spans several chunks
   const int64_t blocks = (pl->n_long + kMmWaves - 1) / kMmWaves;
   int col_shift = 0;
   while (col_shift < 6 && ((int64_t)1 << col_shift) < n_dense) ++col_shift;
