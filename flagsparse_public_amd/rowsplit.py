@@ -223,30 +223,34 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     16,000 rows, N = 128 in fp32 (84 MB) 25 / 27 / 37 us, N = 160 in bf16 (51
     MB) 36 / 40 / 56; 4,000 rows, N = 160 in fp32 (23 MB) 19 / 25 / 40; 64,000
     rows, N = 64 in fp32 (177 MB) 49 / 41 / 38."""
+    short, chunk = _spmm_split(n_rows, nnz, n_dense, item_bytes)
+    return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0,
+                    xcd_remap=_lib.FS_XCD_AUTO)
+
+
+def _spmm_split(n_rows: int, nnz: int, n_dense: int, item_bytes: int) -> tuple[int, int]:
+    """(short_max, chunk_nnz) of default_spmm_schedule."""
     mean = nnz / n_rows if n_rows > 0 else 0.0
     lanes = max(8, _pow2_ceil(n_dense / 4.0))
     if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
-        chunk = 512 if item_bytes <= 4 else 256
-        return Schedule(group_lanes=1, short_max=32, chunk_nnz=chunk, unroll=4, col_tile=0,
-                        xcd_remap=_lib.FS_XCD_AUTO)
+        return 32, 512 if item_bytes <= 4 else 256
     short, most = 32, 256 if item_bytes else 1024
     while short < 2 * mean and short < most:
         short *= 2
     chunk, row_bytes = 256, n_dense * item_bytes
     if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:
         chunk = 64 if row_bytes > 256 and nnz * row_bytes < SPMM_CHUNK_BYTES // 2 else 128
-    return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0,
-                    xcd_remap=_lib.FS_XCD_AUTO)
+    return short, chunk
 
 
-def spmm_split_widths(nnz: int, item_bytes: int) -> list[int]:
-    """Dense widths at which default_spmm_schedule may change, 1 first: every
-    split that it gives a matrix is that of one of these widths."""
+def spmm_splits(n_rows: int, nnz: int, item_bytes: int) -> list[tuple[int, int]]:
+    """Every (short_max, chunk_nnz) that default_spmm_schedule gives a matrix:
+    those of the widths at which the rule may change."""
     widths = {1, 33, 65, 129, 128 // item_bytes + 1, 256 // item_bytes + 1}
     if nnz > 0:
         widths |= {-(-gathered // (nnz * item_bytes))
                    for gathered in (SPMM_CHUNK_BYTES // 2, SPMM_CHUNK_BYTES)}
-    return sorted(widths)
+    return sorted({_spmm_split(n_rows, nnz, n, item_bytes) for n in widths})
 
 
 class RowSplitPlan:
@@ -348,8 +352,9 @@ class RowSplitPlan:
             if cls._listed_natively(indptr, n_rows, nnz, s):
                 lists[s] = _lib.split_lists(nnz, n_rows, s.short_max, s.chunk_nnz, indptr.device)
                 _lib.enqueue_split(csr, indptr.device, s.short_max, s.chunk_nnz, lists[s])
-        words = torch.cat([li[0][_lib.FS_STATS_LEN:_lib.FS_STATS_LEN + 1]
-                           for li in lists.values()]).cpu().tolist() if lists else []
+        words = [li[0][_lib.FS_STATS_LEN:_lib.FS_STATS_LEN + 1] for li in lists.values()]
+        if words:
+            words = (torch.cat(words) if len(words) > 1 else words[0]).cpu().tolist()
         counts = {s: _lib.split_counts(word) for s, word in zip(lists, words)}
         plans = []
         for s in schedules:

@@ -20,7 +20,7 @@ import torch
 
 from .. import _lib
 from ..autotune import SPMM_VARIANTS
-from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule, spmm_split_widths
+from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule, spmm_splits
 from ..schedule_choice import choose_schedule
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
@@ -276,10 +276,12 @@ def _spmm_plan(prepared, accumulate, schedule):
     if p is None:
         schedules = [schedule]
         if prepared.library_schedule:
-            widths = spmm_split_widths(prepared.data.numel(), prepared.data.element_size())
-            of_widths = dict.fromkeys(_library_schedule(prepared, n)[0] for n in widths)
-            if schedule in of_widths:
-                schedules = [s for s in of_widths if (acc, s.key()) not in plans]
+            splits = spmm_splits(prepared.n_rows, prepared.data.numel(),
+                                 prepared.data.element_size())
+            if len(splits) > 1:
+                of_widths = dict.fromkeys(_library_schedule(prepared, 1, s)[0] for s in splits)
+                if schedule in of_widths:
+                    schedules = [s for s in of_widths if (acc, s.key()) not in plans]
         for s, q in zip(schedules, RowSplitPlan.several(
                 prepared.kernel_indptr, prepared.n_rows, prepared.data.dtype, schedules, acc,
                 prepared.data.numel(), prepared.row_lengths)):
@@ -565,17 +567,19 @@ def _library_spmm_launch(sch, dtype, n_dense):
     return sch, col_tile
 
 
-def _library_schedule(prepared, n_dense):
-    """(schedule, column tile) for n_dense columns where the library chooses.
+def _library_schedule(prepared, n_dense, split=None):
+    """(schedule, column tile) for n_dense columns where the library chooses
+    (the schedule of another row split than that of n_dense: ``split``).
     The row split follows the mean row length whatever variant was chosen (the
     variants' own bounds were picked with longer short rows), but a variant
     that chunks shorter rows keeps doing so: their sums are compensated there."""
-    split = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
-                                  prepared.data.element_size())
-    sch, short = prepared.schedule or split, split.short_max
+    rule = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
+                                 prepared.data.element_size())
+    sch = prepared.schedule or rule
+    short, chunk = split or (rule.short_max, rule.chunk_nnz)
     if sch in SPMM_VARIANTS:
         short = min(short, sch.short_max)
-    sch = dataclasses.replace(sch, short_max=short, chunk_nnz=split.chunk_nnz,
+    sch = dataclasses.replace(sch, short_max=short, chunk_nnz=chunk,
                               xcd_remap=sch.xcd_remap or _lib.FS_XCD_AUTO)
     return _library_spmm_launch(sch, prepared.data.dtype, n_dense)
 
