@@ -417,12 +417,22 @@ def coo_sort(data, row, col, n_rows: int, n_cols: int, flags, index_dtype=None, 
 SPLIT_CHUNK_BITS = 36  # stats[FS_STATS_LEN] of analyze_split: n_long << 36 | n_chunks
 
 
+def most_long_rows(nnz: int, n_rows: int, short_max: int) -> int:
+    """Rows of more than short_max entries that a valid matrix has at most."""
+    return min(n_rows, nnz // (short_max + 1))
+
+
+def splits_natively(nnz: int, n_rows: int, short_max: int) -> bool:
+    """Whether fs_csr_analyze_split takes a matrix of this size."""
+    return nnz < 1 << 31 and most_long_rows(nnz, n_rows, short_max) < 1 << (63 - SPLIT_CHUNK_BITS)
+
+
 def split_lists(nnz: int, n_rows: int, short_max: int, chunk_nnz: int, device):
     """One allocation for analyze_split: the statistics, their packed counts,
     one spare word that its host copy also reads (element FS_STATS_LEN + 1 of
     the first tensor returned), and the lists at their largest sizes for a
     valid matrix."""
-    cap_long = min(n_rows, nnz // (short_max + 1))
+    cap_long = most_long_rows(nnz, n_rows, short_max)
     cap_chunks = min(nnz // chunk_nnz + cap_long, nnz)
     at = FS_STATS_LEN + 2
     buf = torch.empty(at + 2 * cap_long + 1 + (cap_chunks + 1) // 2, dtype=torch.int64,

@@ -22,7 +22,8 @@ static_assert(ST_LONGNNZ + 1 == FS_STATS_LEN, "statistics layout");
 // Row-split outputs of fs_csr_analyze_split (see the header).  st[ST_SPLIT]
 // counts long rows and chunks together, chunks in the low kSplitBits bits, so
 // that one atomic gives a group of rows consecutive long-row ordinals and
-// consecutive chunks at once.
+// consecutive chunks at once.  That leaves the count 27 bits below the sign,
+// which the entry point checks.
 constexpr int ST_SPLIT = FS_STATS_LEN;
 constexpr int kSplitBits = 36;
 
@@ -361,6 +362,8 @@ extern "C" int fs_csr_analyze_split(const fs_csr* A, int64_t* stats, int64_t sho
   if (short_max < 1) return fail(FS_ERR_VALUE, "%s: short_max must be >= 1", who);
   if (chunk_nnz <= 0 || chunk_nnz % kWave != 0)
     return fail(FS_ERR_VALUE, "%s: chunk_nnz must be a positive multiple of 64", who);
+  if (A && (A->n_rows < cap_long ? A->n_rows : cap_long) >= (int64_t)1 << (63 - kSplitBits))
+    return fail(FS_ERR_UNSUPPORTED, "%s: room for 2^27 long rows or more", who);
   if (cap_long < 0 || cap_chunks < 0 || cap_long > INT32_MAX || cap_chunks > INT32_MAX)
     return fail(FS_ERR_VALUE, "%s: capacities must be in [0, 2^31)", who);
   if (!long_chunk_ptr || (cap_long > 0 && !long_rows) || (cap_chunks > 0 && !chunk_long))

@@ -327,15 +327,16 @@ class RowSplitPlan:
     @staticmethod
     def _listed_natively(indptr, n_rows, nnz, schedule):
         """Whether fs_csr_analyze_split lists this plan's rows."""
-        return (nnz is not None and nnz < 1 << 31 and n_rows > 0 and schedule.tile_nnz == 0
+        return (nnz is not None and n_rows > 0 and schedule.tile_nnz == 0
                 and schedule.short_max >= 1 and schedule.chunk_nnz > 0
-                and schedule.chunk_nnz % 64 == 0 and indptr.is_cuda)
+                and schedule.chunk_nnz % 64 == 0 and indptr.is_cuda
+                and _lib.splits_natively(nnz, n_rows, schedule.short_max))
 
     def _take_lists(self, lists, n_long, n_chunks):
         """Takes the lists of one native pass; False (nothing taken) where they
         do not hold the counts: row pointers that do not match nnz."""
         _, rows, chunk_ptr, chunk_long, cap_long, cap_chunks = lists
-        if n_long > cap_long or n_chunks > cap_chunks:
+        if not 0 <= n_long <= cap_long or n_chunks > cap_chunks:
             return False
         self.n_long, self.n_chunks = n_long, n_chunks
         self.long_rows, self.long_chunk_ptr = rows[:n_long], chunk_ptr[:n_long + 1]

@@ -112,7 +112,7 @@ typedef struct fs_plan {
   int64_t short_max;       /* longest row handled by the short-row role    */
   int64_t chunk_nnz;       /* entries per long-row chunk (multiple of 64)  */
   int64_t n_long;          /* number of listed long rows                   */
-  const int64_t *long_rows;      /* [n_long] row ids, ascending            */
+  const int64_t *long_rows;      /* [n_long] row ids, in any order         */
   const int64_t *long_chunk_ptr; /* [n_long + 1] first chunk of each row   */
   int64_t n_chunks;
   const int32_t *chunk_long;     /* [n_chunks] long-row ordinal of a chunk */
@@ -387,7 +387,8 @@ int fs_csr_analyze(const fs_csr *A, int64_t *stats, void *stream);
  * chunks, and nothing is written past the capacities for any other.  cols32
  * (or null): the columns of a matrix with 64-bit indices, narrowed; they mean
  * something only if the statistics say that every column fits.  At most
- * 2^31 - 1 entries.
+ * 2^31 - 1 entries, and fewer than 2^27 long rows: FS_ERR_UNSUPPORTED where
+ * cap_long and n_rows leave room for more.
  */
 int fs_csr_analyze_split(const fs_csr *A, int64_t *stats, int64_t short_max, int64_t chunk_nnz,
                          int64_t *long_rows, int64_t *long_chunk_ptr, int64_t cap_long,
