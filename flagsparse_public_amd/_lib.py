@@ -399,6 +399,8 @@ def coo_sort(data, row, col, n_rows: int, n_cols: int, flags, index_dtype=None, 
     lib = load()
     data = data.resolve_conj().resolve_neg()
     device, nnz = data.device, data.numel()
+    if not nnz == row.numel() == col.numel():
+        raise ValueError("coo_sort: data, row and col must have the same length")
     index_dtype = index_dtype or row.dtype
     out = torch.empty_like(data)
     out_row = torch.empty(nnz, dtype=index_dtype, device=device) if want_rows else None
