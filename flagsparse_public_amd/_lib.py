@@ -380,6 +380,7 @@ def analyze(csr: FsCsr, device) -> list[int]:
     return analyze_device(csr, device).cpu().tolist()
 
 
+COO_SORT_VALUE_BYTES = (2, 4, 8, 16)  # that fs_coo_sort moves
 COO_BAD_ROW, COO_BAD_COL, COO_OVERFLOW = 1, 2, 4  # *flags of fs_coo_sort
 
 

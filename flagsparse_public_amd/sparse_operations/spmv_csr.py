@@ -702,6 +702,7 @@ def coo_to_csr_for_spmv(data, row, col, shape, assume_sorted=False):
     else:
         if (_lib.coo_sort_applies(row.numel(), n_rows, n_cols) and row.is_cuda
                 and data.ndim == 1 and data.shape == row.shape == col.shape
+                and data.element_size() in _lib.COO_SORT_VALUE_BYTES
                 and row.dtype in SUPPORTED_INDEX_DTYPES and col.dtype in SUPPORTED_INDEX_DTYPES
                 and row.device == data.device and col.device == data.device):
             flags = torch.empty(1, dtype=torch.int64, device=data.device)

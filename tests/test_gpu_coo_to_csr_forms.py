@@ -19,6 +19,16 @@ def _pairs():
     return torch.from_numpy(r).to(DEV), torch.from_numpy(c).to(DEV), order
 
 
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int8, torch.int16, torch.float16,
+                                   torch.bfloat16, torch.float32, torch.int64, torch.complex128],
+                         ids=str)
+def test_value_types(dtype):
+    r, c, order = _pairs()
+    data = (torch.arange(NNZ, device=DEV) % 101).to(dtype)
+    d, cols, _ = coo_to_csr_for_spmv(data, r, c, (N, M))
+    assert torch.equal(d, data[order]) and torch.equal(cols, c[order].to(torch.int32))
+
+
 @pytest.mark.parametrize("shape", [(NNZ + 300,), (NNZ, 3), (NNZ + 5, 2)], ids=str)
 def test_more_values_than_pairs(shape):
     """The values are indexed by the pairs' order whatever else they hold."""
