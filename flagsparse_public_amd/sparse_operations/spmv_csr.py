@@ -700,7 +700,7 @@ def coo_to_csr_for_spmv(data, row, col, shape, assume_sorted=False):
     if assume_sorted or _coo_is_sorted_lex(row64, col64, n_cols):
         row_s, col_s, data_s = row64, col64, data
     else:
-        if (_lib.coo_sort_applies(row.numel(), n_rows, n_cols) and row.is_cuda
+        if (row.is_cuda and _lib.coo_sort_applies(row.numel(), n_rows, n_cols)
                 and data.ndim == 1 and data.shape == row.shape == col.shape
                 and data.element_size() in _lib.COO_SORT_VALUE_BYTES
                 and row.dtype in SUPPORTED_INDEX_DTYPES and col.dtype in SUPPORTED_INDEX_DTYPES
