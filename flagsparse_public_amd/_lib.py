@@ -389,6 +389,16 @@ def coo_sort_applies(nnz: int, n_rows: int, n_cols: int) -> bool:
     return nnz > 0 and int(load().fs_coo_sort_workspace(nnz, n_rows, n_cols)) > 0
 
 
+def torch_follows(data) -> bool:
+    """Whether torch follows what is done to these values (gradients, tangents,
+    function transforms, subclasses), which a native pass over their memory would
+    cut off."""
+    return ((data.requires_grad and torch.is_grad_enabled())
+            or type(data) not in (torch.Tensor, torch.nn.Parameter)
+            or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad.unpack_dual(data).tangent is not None)
+
+
 def coo_sort(data, row, col, n_rows: int, n_cols: int, flags, index_dtype=None, want_rows=True,
              ptr_dtype=torch.int64):
     """Run fs_coo_sort on contiguous device arrays (row and col of one dtype);

@@ -161,7 +161,7 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
         raise TypeError("col dtype must be torch.int32 or torch.int64")
     # both orders are sorted here (deterministic sums); seg_starts only when asked
     if (_lib.coo_sort_applies(data.numel(), n_rows, n_cols) and row.device == data.device
-            and col.device == data.device):
+            and col.device == data.device and not _lib.torch_follows(data)):
         # one native sort that also checks the index ranges, the analysis of
         # the result and the schedule selection behind it, one host read for
         # the three
@@ -348,6 +348,8 @@ def flagsparse_spmv_coo(data=None, row=None, col=None, x=None, shape=None, out=N
     if prepared is None:
         if any(a is None for a in (data, row, col, x, shape)):
             raise ValueError("data, row, col, x, shape required when prepared is None")
+        if torch.is_tensor(data):  # the product is not differentiable
+            data = data.detach()
         prepared = prepare_spmv_coo(data, row, col, shape, sort_by_row=sort_by_row, op=op_code,
                                     index_fallback_policy=index_fallback_policy)
     else:

@@ -704,7 +704,8 @@ def coo_to_csr_for_spmv(data, row, col, shape, assume_sorted=False):
                 and data.ndim == 1 and data.shape == row.shape == col.shape
                 and data.element_size() in _lib.COO_SORT_VALUE_BYTES
                 and row.dtype in SUPPORTED_INDEX_DTYPES and col.dtype in SUPPORTED_INDEX_DTYPES
-                and row.device == data.device and col.device == data.device):
+                and row.device == data.device and col.device == data.device
+                and not _lib.torch_follows(data)):
             flags = torch.empty(1, dtype=torch.int64, device=data.device)
             dtype = torch.promote_types(row.dtype, col.dtype)
             data_s, _, col_s, indptr = _lib.coo_sort(
@@ -712,7 +713,8 @@ def coo_to_csr_for_spmv(data, row, col, shape, assume_sorted=False):
                 n_cols, flags, index_dtype=torch.int32, want_rows=False)
             if int(flags.item()) == 0:
                 return data_s, col_s, indptr
-        # larger, or out-of-range indices (reported by what follows)
+        # what the native sort does not take, or out-of-range indices (reported
+        # by what follows)
         order = torch.argsort(row64 * max(1, n_cols) + col64, stable=True)
         row_s, col_s, data_s = row64[order], col64[order], data[order]
     indptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=data.device)
@@ -764,7 +766,8 @@ def flagsparse_spmv_coo_tocsr(data=None, row=None, col=None, x=None, shape=None,
         raise TypeError(_spmv_dtype_error_message())
     if x.dtype != data.dtype:
         raise TypeError("x dtype must match data dtype")
-    data_s, indices, indptr = coo_to_csr_for_spmv(data, row, col, shape,
+    # the product is not differentiable: nothing need follow its values
+    data_s, indices, indptr = coo_to_csr_for_spmv(data.detach(), row, col, shape,
                                                   assume_sorted=assume_sorted)
     return flagsparse_spmv_csr(data_s, indices, indptr, x, shape, block_nnz=block_nnz,
                                max_segments=max_segments, out=out, return_time=return_time,
