@@ -347,10 +347,17 @@ __global__ __launch_bounds__(kMmBlock) void spmm_csr_kernel(SpmmParams<V, I, P> 
 // rows of 16: between -5% and +1%.  Not taken: B below 24 MB (20,000 rows N = 8 to
 // 64: up to 8% slower), rows of under 12 entries (1M banded rows of 9, N = 64 234
 // -> 241 us), 16-bit values (1M rows of 9, N = 100 303 -> 312 us), long rows, and
-// column tiles, whose neighbours belong on different XCDs.
+// column tiles, whose neighbours belong on different XCDs, unless the last tile
+// holds a few columns only: it reads the lines where the tile before it ends, and
+// finds them in the L2 of its own XCD.  Random rows of 15, fp64 N = 129 / 131: 344 ->
+// 250 / 339 -> 242 us, fp32 N = 257 338 -> 235 us, bf16 N = 513 347 -> 300; rows of 5,
+// power-law and banded rows, B of 2 to 400 MB: from -30% to +2%.  Tiles a quarter
+// full: +8% on banded fp64 N = 158.
 template <typename V>
-static inline bool spmm_xcd_rows(const fs_csr* M, int64_t n_dense, int64_t n_tiles, const fs_plan* pl) {
-  return (std::is_same<V, float>::value || std::is_same<V, double>::value) && n_tiles == 1 &&
+static inline bool spmm_xcd_rows(const fs_csr* M, int64_t n_dense, int64_t tile, int64_t n_tiles,
+                                 const fs_plan* pl) {
+  if (n_tiles > 1) return n_dense % tile != 0 && n_dense % tile <= tile / 8;
+  return (std::is_same<V, float>::value || std::is_same<V, double>::value) &&
          M->n_cols * n_dense * (int64_t)sizeof(V) >= ((int64_t)24 << 20) &&
          M->nnz >= 12 * M->n_rows && pl->n_long <= M->n_rows / 128;
 }
@@ -379,7 +386,7 @@ int launch_spmm_gv(const fs_csr* M, const void* B, int64_t ldb, void* C, int64_t
   p.long_chunk_ptr = pl->long_chunk_ptr;
   p.chunk_long = pl->chunk_long;
   p.partials = pl->partials;
-  p.xcd_remap = pl->xcd_remap == FS_XCD_AUTO ? spmm_xcd_rows<V>(M, n_dense, p.n_tiles, pl)
+  p.xcd_remap = pl->xcd_remap == FS_XCD_AUTO ? spmm_xcd_rows<V>(M, n_dense, G * VW, p.n_tiles, pl)
                                              : pl->xcd_remap != 0;
   const int64_t rows_per_block = kMmBlock / G;
   const int64_t short_blocks = ((M->n_rows + rows_per_block - 1) / rows_per_block) * p.n_tiles;
