@@ -188,10 +188,12 @@ SPMM_FILL_LANES = 1 << 18  # lanes of 256 CUs with 16 wavefronts each
 SPMM_CHUNK_BYTES = 1 << 27  # gathered bytes of a launch below which chunks shrink
 
 
-def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int = 0) -> Schedule:
+def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int = 0,
+                          wide: bool = False, max_row: int | None = None) -> Schedule:
     """Which SpMM rows one lane group walks alone and which whole wavefronts
     take in chunks.  Every launch gives item_bytes, the bytes of a value; 0
-    leaves out what depends on them.
+    leaves out what depends on them.  wide: sums in a wider type than the
+    values (fp32 in fp64).  max_row: the longest row, where it is known.
 
     A lane group walks its row serially (a round trip to the B rows per batch
     of entries), so the longest short row bounds the launch: rows over about
@@ -204,16 +206,25 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     fp32 sums are compensated (fp32, N = 64, values of both signs, rms error of
     20,000 rows of about 300 entries 7.7e-7 in chunks, 1.8e-6 in chains, of
     40,000 rows of 600 3.0e-7 and 3.6e-6; the chains took 107 and 379 us, the
-    chunks take 154 and 484).
+    chunks take 154 and 484).  Wide sums lose nothing in a chain, and where the
+    groups fill the chip they take rows up to 1024 (30,000 rows of 200, N = 256
+    in fp32: 518 us, in chunks 795).
 
     With long rows and too few of them to fill the chip with lane groups,
-    every row gets a wavefront: 5,000 rows of about 300, N = 16: 45 -> 12 us;
-    20,000 rows, N = 8: 77 -> 37 us; at 30,000 rows of 100 the two meet (N = 8,
-    240,000 lanes: 26.6 -> 24.7 us; N = 64, 480,000 lanes: 57 -> 61 us).  Its
-    chunks hold 512 entries where the chunk sums are compensated or in fp64
-    over fp32 values, 256 in fp64 and complex types, whose chains are then half
-    as long (2,000 fp64 rows of about 600, N = 130: rms error 4.2e-15 against
-    5.7e-15, 184 against 204 us).
+    every row gets a wavefront: 5,000 rows of about 200, N = 8: 28 -> 10 us;
+    30,000 power-law rows of mean 70, N = 8: 42 -> 24 us.  Where no row is far
+    longer than the mean, the lanes added to a row pay only as long as they
+    are few against its entries: 30,000 rows, N = 8 (240,000 lanes), of 70
+    entries 16.6 -> 20.2 us, of 100 23.4 -> 24.2 (fp64 29 -> 35), of 200 54.9 ->
+    38.8; 15,000 rows of 70 11.0 -> 11.3; 8,000 fp64 rows of 200, N = 36, 56 -> 72;
+    and a group that is a wavefront already has none to add (1,500 rows of
+    100, N = 256: 17.9 -> 25.5 us).  Chunks of 512 there hold most rows whole;
+    rows of about 400 need two, and then 256 are faster (300 rows, N = 64: 20.3
+    against 14.0 us), as they are where one group takes the whole wavefront
+    (300 power-law rows of mean 70, N = 256: 68 against 38 us).  fp64 and complex
+    types, whose sums are as wide as the values, keep 256, for chains half as
+    long (2,000 fp64 rows of about 600, N = 130: rms error 4.2e-15 against
+    5.7e-15).
 
     The wider B (values of item_bytes each), the fewer of a chunk's entries its
     wavefront takes at once: 16 lanes a B row leave 64 round trips for a chunk
@@ -223,34 +234,59 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     16,000 rows, N = 128 in fp32 (84 MB) 25 / 27 / 37 us, N = 160 in bf16 (51
     MB) 36 / 40 / 56; 4,000 rows, N = 160 in fp32 (23 MB) 19 / 25 / 40; 64,000
     rows, N = 64 in fp32 (177 MB) 49 / 41 / 38."""
-    short, chunk = _spmm_split(n_rows, nnz, n_dense, item_bytes)
+    mean = nnz / n_rows if n_rows > 0 else 0.0
+    lanes = max(8, _pow2_ceil(n_dense / 4.0))
+    row_bytes = n_dense * item_bytes
+    filled = n_rows * lanes >= SPMM_FILL_LANES
+    few = not filled
+    if few and item_bytes and max_row is not None and max_row <= SPMM_EVEN_ROWS * mean:
+        lanes = spmm_row_lanes(n_dense, item_bytes)
+        few = (n_rows * lanes < min(SPMM_FILL_LANES, (1300 if item_bytes <= 4 else 1000) * mean)
+               and (lanes < 64 or n_rows < 1024))
+    if mean >= 64 and few:
+        short, chunk = 32, 512 if item_bytes == 0 or _long_chunks(mean, item_bytes, row_bytes) else 256
+    else:
+        short, chunk = _short_rows(mean, 1024 if item_bytes == 0 or (wide and filled) else 256), 256
+        if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:
+            chunk = 64 if row_bytes > 256 and nnz * row_bytes < SPMM_CHUNK_BYTES // 2 else 128
     return Schedule(group_lanes=1, short_max=short, chunk_nnz=chunk, unroll=4, col_tile=0,
                     xcd_remap=_lib.FS_XCD_AUTO)
 
 
-def _spmm_split(n_rows: int, nnz: int, n_dense: int, item_bytes: int) -> tuple[int, int]:
-    """(short_max, chunk_nnz) of default_spmm_schedule."""
-    mean = nnz / n_rows if n_rows > 0 else 0.0
-    lanes = max(8, _pow2_ceil(n_dense / 4.0))
-    if mean >= 64 and n_rows * lanes < SPMM_FILL_LANES:
-        return 32, 512 if item_bytes <= 4 else 256
-    short, most = 32, 256 if item_bytes else 1024
+SPMM_EVEN_ROWS = 8  # rows up to this many times the mean length count as alike
+
+
+def spmm_row_lanes(n_dense: int, item_bytes: int) -> int:
+    """Lanes that an SpMM row takes over all its columns (the launch's shape:
+    16 bytes a lane where that leaves eight lanes)."""
+    width = max(1, 16 // item_bytes)
+    while width > 1 and n_dense // width < 8:
+        width //= 2
+    return 1 << (-(-n_dense // width) - 1).bit_length() if n_dense > 0 else 1
+
+
+def _short_rows(mean: float, most: int) -> int:
+    short = 32
     while short < 2 * mean and short < most:
         short *= 2
-    chunk, row_bytes = 256, n_dense * item_bytes
-    if row_bytes > 128 and nnz * row_bytes < SPMM_CHUNK_BYTES:
-        chunk = 64 if row_bytes > 256 and nnz * row_bytes < SPMM_CHUNK_BYTES // 2 else 128
-    return short, chunk
+    return short
+
+
+def _long_chunks(mean: float, item_bytes: int, row_bytes: int) -> bool:
+    return item_bytes <= 4 and row_bytes <= 256 and (mean <= 320 or row_bytes <= 16)
 
 
 def spmm_splits(n_rows: int, nnz: int, item_bytes: int) -> list[tuple[int, int]]:
-    """Every (short_max, chunk_nnz) that default_spmm_schedule gives a matrix:
-    those of the widths at which the rule may change."""
-    widths = {1, 33, 65, 129, 128 // item_bytes + 1, 256 // item_bytes + 1}
-    if nnz > 0:
-        widths |= {-(-gathered // (nnz * item_bytes))
-                   for gathered in (SPMM_CHUNK_BYTES // 2, SPMM_CHUNK_BYTES)}
-    return sorted({_spmm_split(n_rows, nnz, n, item_bytes) for n in widths})
+    """Every (short_max, chunk_nnz) that default_spmm_schedule may give a
+    matrix over the dense widths, for sums in the type of the values."""
+    mean = nnz / n_rows if n_rows > 0 else 0.0
+    first = 128 + item_bytes  # bytes of the narrowest B row past the smaller chunks' bound
+    chunks = [256] + [128] * (nnz * (first - first % item_bytes) < SPMM_CHUNK_BYTES) \
+        + [64] * (nnz * 256 < SPMM_CHUNK_BYTES // 2)
+    splits = [(_short_rows(mean, 256), chunk) for chunk in chunks]
+    if mean >= 64 and n_rows * 1 < SPMM_FILL_LANES:
+        splits += [(32, 256)] + [(32, 512)] * (item_bytes <= 4)
+    return splits
 
 
 class RowSplitPlan:

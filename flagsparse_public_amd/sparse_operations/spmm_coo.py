@@ -19,7 +19,7 @@ import time
 import torch
 
 from .. import _lib
-from ..rowsplit import RowSplitPlan, default_spmm_schedule
+from ..rowsplit import RowSplitPlan
 from ..sortkey import stable_order
 from ._common import SUPPORTED_INDEX_DTYPES, _INDEX_LIMIT_INT32
 from .spmm_csr import SUPPORTED_SPMM_VALUE_DTYPES, _select_spmm_alg1_warp_and_factor
@@ -121,12 +121,12 @@ def _native_spmm_coo_csr(data, row, col, B, n_rows, n_cols):
     for the index checks and the lists: (values, columns, row pointer, plan),
     or None where the sort does not apply.  The sort orders equal (row, col)
     pairs by input position, as _sorted_csr does."""
-    from .spmm_csr import _spmm_default_accumulate
+    from .spmm_csr import _spmm_call_schedule, _spmm_default_accumulate
     nnz, n_dense, device = data.numel(), int(B.shape[1]), data.device
     if not _lib.coo_sort_applies(nnz, n_rows, n_cols):
         return None
     index = torch.promote_types(row.dtype, col.dtype)
-    sch = default_spmm_schedule(n_rows, nnz, n_dense, data.element_size())
+    sch = _spmm_call_schedule(n_rows, data, n_dense)
     lists = _lib.split_lists(nnz, n_rows, sch.short_max, sch.chunk_nnz, device)
     d, _, c, indptr = _lib.coo_sort(
         data.contiguous(), row.to(index).contiguous(), col.to(index).contiguous(), n_rows, n_cols,

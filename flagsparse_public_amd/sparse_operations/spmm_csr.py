@@ -209,7 +209,7 @@ def _spmm_call_inputs(data, indices, indptr, B, shape):
         return data, cols, indptr, B, n_rows, n_cols, n_dense, None, max_row_nnz
     data, cols, indptr, n_rows, n_cols = _check_spmm_csr_arrays(data, indices, indptr, shape)
     n_dense = int(B.shape[1])
-    sch = default_spmm_schedule(n_rows, data.numel(), n_dense, data.element_size())
+    sch = _spmm_call_schedule(n_rows, data, n_dense)
     (stats, long_rows, long_chunk_ptr, chunk_long, n_long, n_chunks, narrowed,
      _) = _lib.analyze_split(
         _lib.make_csr(data, cols, indptr, n_rows, n_cols), data.device, sch.short_max,
@@ -325,6 +325,12 @@ def _spmm_default_accumulate(dtype):
     return _lib.FS_ACC_WIDE if dtype == torch.float32 else _lib.FS_ACC_NATIVE
 
 
+def _spmm_call_schedule(n_rows, data, n_dense):
+    """The schedule of a product with _spmm_default_accumulate."""
+    return default_spmm_schedule(n_rows, data.numel(), n_dense, data.element_size(),
+                                 wide=data.dtype == torch.float32)
+
+
 def _hip_spmm_csr_impl(data, indices, indptr, B, n_rows, n_dense_cols, block_n, block_nnz,
                        schedule=None, row_lengths=None, n_cols=None, out=None, alpha=1.0,
                        beta=0.0, plan=None):
@@ -337,8 +343,7 @@ def _hip_spmm_csr_impl(data, indices, indptr, B, n_rows, n_dense_cols, block_n, 
         return out.mul_(beta) if beta != 0.0 else out.zero_()
     n_cols = int(B.shape[0]) if n_cols is None else n_cols
     if plan is None:
-        sch = schedule or default_spmm_schedule(n_rows, data.numel(), n_dense_cols,
-                                                data.element_size())
+        sch = schedule or _spmm_call_schedule(n_rows, data, n_dense_cols)
         plan = RowSplitPlan(indptr, n_rows, dtype, sch, _spmm_default_accumulate(dtype),
                             row_lengths=row_lengths)
     csr = _lib.make_csr(data, indices, indptr, n_rows, n_cols)
@@ -574,11 +579,11 @@ def _library_schedule(prepared, n_dense, split=None):
     variants' own bounds were picked with longer short rows), but a variant
     that chunks shorter rows keeps doing so: their sums are compensated there."""
     rule = default_spmm_schedule(prepared.n_rows, prepared.data.numel(), n_dense,
-                                 prepared.data.element_size())
+                                 prepared.data.element_size(), max_row=prepared.max_row_nnz)
     sch = prepared.schedule or rule
     short, chunk = split or (rule.short_max, rule.chunk_nnz)
-    if sch in SPMM_VARIANTS:
-        short = min(short, sch.short_max)
+    if sch in SPMM_VARIANTS and sch.short_max < short:
+        short, chunk = sch.short_max, max(chunk, sch.chunk_nnz)
     sch = dataclasses.replace(sch, short_max=short, chunk_nnz=chunk,
                               xcd_remap=sch.xcd_remap or _lib.FS_XCD_AUTO)
     return _library_spmm_launch(sch, prepared.data.dtype, n_dense)

@@ -18,6 +18,6 @@ def test_chosen_variants_keep_their_chunked_rows(variant, mean, n_dense):
     data = types.SimpleNamespace(numel=lambda: n_rows * mean, element_size=lambda: 4,
                                  dtype=torch.float32)
     p = types.SimpleNamespace(schedule=variant, library_schedule=True, n_rows=n_rows, data=data,
-                              _plans={})
+                              max_row_nnz=4 * mean, _plans={})
     sch, _ = spmm_launch_schedule(p, n_dense)
     assert sch.short_max <= min(256, variant.short_max)
