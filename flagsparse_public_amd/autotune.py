@@ -169,7 +169,7 @@ def tune_spmm(prepared, B, variants=SPMM_VARIANTS, reps=5, warmup=1, inner=1):
     n_dense = int(B.shape[1])
     times = []
     for sch in variants:
-        run, col_tile = _library_spmm_launch(sch, B.dtype, n_dense)
+        run, col_tile = _library_spmm_launch(sch, B.dtype, n_dense, prepared.n_rows)
         run = dataclasses.replace(run, col_tile=col_tile)
         times.append(time_launches(
             lambda s=run: _hip_spmm_csr_impl_opt_prepared(prepared, B, out=C, schedule=s),

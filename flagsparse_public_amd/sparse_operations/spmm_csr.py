@@ -20,7 +20,8 @@ import torch
 
 from .. import _lib
 from ..autotune import SPMM_VARIANTS
-from ..rowsplit import RowSplitPlan, Schedule, default_spmm_schedule, spmm_splits
+from ..rowsplit import (RowSplitPlan, SPMM_FILL_LANES, Schedule, default_spmm_schedule,
+                        spmm_row_lanes, spmm_splits)
 from ..schedule_choice import choose_schedule
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
@@ -555,20 +556,26 @@ def _check_opt_B(prepared, B):
         raise ValueError("B must be a 2D dense tensor")
 
 
-def _library_spmm_launch(sch, dtype, n_dense):
+def _library_spmm_launch(sch, dtype, n_dense, n_rows=0):
     """(schedule, column tile) to launch for a schedule the library chose
     itself (selector, fixed rule or exhaustive search).  Those are picked for
     B with 64 columns at 4 entries in flight per lane; measured on MI355X
     (1M-row banded matrix, N = 32 / 64 / 128), fp32 runs faster with 8 in
     flight (418 vs 437 us at N = 64), and a wider B keeps the chosen lanes per
     64 columns (N = 128 with one 128-column tile: 883 vs 926 us).  fp64 keeps
-    4 in flight (851 vs 929 us).  Schedules passed in by the caller run as
-    given."""
+    4 in flight (851 vs 929 us).  Widths that 16 bytes do not divide are taken
+    in one tile where the rows fill the chip (fp32, 120,000 rows of 40, N = 66 /
+    99 / 129: 288 / 383 / 485 us in the tiles chosen for 64 columns, 223 / 313 /
+    414 in one; 300 rows of 200, N = 130, need the tiles: 14 against 38 us).
+    Schedules passed in by the caller run as given."""
     if dtype == torch.float32 and sch.unroll == 4:
         sch = dataclasses.replace(sch, unroll=8)
     col_tile = sch.col_tile
     if col_tile > 0 and n_dense > 64:
         col_tile *= n_dense // 64
+    if (n_dense % 4 and dtype == torch.float32
+            and n_rows * spmm_row_lanes(n_dense, 4) >= SPMM_FILL_LANES):
+        col_tile = 0
     return sch, col_tile
 
 
@@ -586,7 +593,7 @@ def _library_schedule(prepared, n_dense, split=None):
         short, chunk = sch.short_max, max(chunk, sch.chunk_nnz)
     sch = dataclasses.replace(sch, short_max=short, chunk_nnz=chunk,
                               xcd_remap=sch.xcd_remap or _lib.FS_XCD_AUTO)
-    return _library_spmm_launch(sch, prepared.data.dtype, n_dense)
+    return _library_spmm_launch(sch, prepared.data.dtype, n_dense, prepared.n_rows)
 
 
 def spmm_launch_schedule(prepared, n_dense, schedule=None):
