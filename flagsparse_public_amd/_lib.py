@@ -28,6 +28,7 @@ FS_ACC_NATIVE, FS_ACC_WIDE = 0, 1
 FS_STORE_BF16X2, FS_STORE_BF16, FS_STORE_F16_ROWSCALE = 1, 2, 3
 FS_STATS_LEN = 16
 FS_TILE_ROWS, FS_TILE_ENTRIES = 0, 1
+FS_BATCH_LONG_MM = 512  # batched SpMM rows above take a block of their own
 FS_XCD_AUTO = 2  # fs_plan.xcd_remap: the SpMM launch decides
 FS_XG_TILE_MAJOR, FS_XG_WINDOW_MAJOR = 0, 1
 FS_NOALLOC_SCRATCH_BYTES = 4 << 20  # fs_spmv_csr_noalloc's per-GPU partials scratch

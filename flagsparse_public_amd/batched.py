@@ -13,7 +13,8 @@ and has no effect.
 Rows use the single-matrix kernels' per-row procedures: with the same lane
 group width a row's value is bit-identical to ``flagsparse_spmv_csr`` /
 ``flagsparse_spmm_csr_opt`` on that matrix (rows short enough for the
-short-row role).
+short-row role).  SpMV rows over ``long_row`` entries and SpMM rows over
+``_lib.FS_BATCH_LONG_MM`` are items of their own, summed by a whole block.
 """
 
 from __future__ import annotations
@@ -89,10 +90,10 @@ class BatchedCsr:
             if data.dtype != torch.float32:
                 raise TypeError("batched path takes float32 matrices")
             if validate:
-                data, indices, indptr, n_rows, n_cols, _, _ = _prepare_spmv_csr_matrix(
+                data, indices, indptr, n_rows, n_cols, _, longest = _prepare_spmv_csr_matrix(
                     data, indices, indptr, shape)
             else:
-                n_rows, n_cols = shape
+                (n_rows, n_cols), longest = shape, None
             if indices.dtype != torch.int32:
                 indices = indices.to(torch.int32)
             x, B = m.get("x"), m.get("B")
@@ -127,7 +128,9 @@ class BatchedCsr:
                 bytes_total += 12 * nnz + 8 * n_rows
             if B is not None and n_rows and n_dense:
                 rows = min(max_rows, lib.fs_batch_rows(int(s), n_dense))
-                cuts = _cuts(ip64, 8.0 + 4.0 * n_dense, item_bytes, rows)
+                some_long = longest is None or longest > _lib.FS_BATCH_LONG_MM
+                cuts = _cuts(ip64, 8.0 + 4.0 * n_dense, item_bytes, rows,
+                             _lib.FS_BATCH_LONG_MM if some_long else None)
                 items.append(self._items(i, SPMM, cuts))
                 bytes_total += (8 + 4 * n_dense) * nnz + 4 * n_dense * n_rows
         rec = int(lib.fs_batch_matrix_bytes())

@@ -5,7 +5,7 @@
 // groups over SpMV rows, one over SpMM rows.  Rows are computed with the
 // single-matrix kernels' short-row procedures (lane-group width, unroll,
 // reduction tree), so a row's result is bit-identical to the single-matrix
-// launch with the same group width.  A single-row SpMV item longer than a lane
+// launch with the same group width.  A single-row item longer than a lane
 // group's bound is reduced by the whole block instead.
 //
 // The hardware hands the blocks out: there is no queue to wait for and no item
@@ -169,30 +169,68 @@ __device__ void bat_spmv_long_row(const BatchMatrix& m, int64_t row, double alph
 }
 
 // --- SpMM rows: the single-matrix short role (G lanes a row, VW columns a
-// lane, entries loaded by the group through its LDS slots).
+// lane, entries loaded by the group through its LDS slots).  A row of its own
+// that is longer than FS_BATCH_LONG_MM belongs to the whole block: its groups
+// take equal ranges of the entries, and their sums are added in order,
+// compensated.  One group would walk it alone while the rest of the launch is
+// done: six power-law matrices of 30,000 rows (up to 20,000 entries), N = 3 / 8 /
+// 40 / 260, by one group 2137 / 2137 / 3099 / 5276 us (by the former two lanes with
+// eight entries in flight 1050 / 1567 / 1749 / 3016), here 102 / 119 / 272 / 1530.
 constexpr int kBatMmU = 4;                // SpMM entries in flight per lane
 constexpr int kBatSlots = kBatBlock * 2;  // at most two fills per lane (kMmFill)
+union BatLds {
+  struct {
+    int32_t col[kBatSlots];
+    float val[kBatSlots];
+  } slot;
+  float part[kBatBlock * 4];  // sums of a long row's groups
+};
 
 template <int G, int VW>
 __device__ void bat_spmm_rows(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha, double beta,
-                              int32_t* slot_col, float* slot_val) {
+                              BatLds& lds) {
   constexpr int kGroups = kBatBlock / G, F = kMmFill<G>;
   static_assert(kBatBlock * F <= kBatSlots, "slots");
   const int grp = threadIdx.x / G, g = threadIdx.x % G;
   const int first = grp * (G * F);
+  // uniform over the block
+  const bool whole = r1 - r0 == 1 && bm_ptr(m, r1) - bm_ptr(m, r0) > FS_BATCH_LONG_MM;
   const int64_t tiles = (m.n_dense + G * VW - 1) / (G * VW);
   for (int64_t t = 0; t < tiles; ++t) {
     int64_t n0 = t * (G * VW) + (int64_t)g * VW;
     const bool colok = n0 < m.n_dense;
     const int skip = shift_tail<VW>(n0, m.n_dense);
-    for (int64_t row = r0 + grp; row < r1; row += kGroups) {
-      const int64_t rs = bm_ptr(m, row), re = bm_ptr(m, row + 1);
+    for (int64_t row = whole ? r0 : r0 + grp; row < r1; row += kGroups) {
+      int64_t rs = bm_ptr(m, row), re = bm_ptr(m, row + 1);
+      if (whole) {
+        const int64_t per = (re - rs + kGroups - 1) / kGroups;
+        rs = rs + grp * per < re ? rs + grp * per : re;
+        re = rs + per < re ? rs + per : re;
+      }
       Plain<float> acc[VW];
 #pragma unroll
       for (int k = 0; k < VW; ++k) acc[k].init();
-      mm_accumulate_group<VW, kBatMmU, G>(acc, slot_col + first, slot_val + first, m.col, m.val, m.B,
-                                          m.ldb, n0, colok, rs, re, g);
-      if (colok) write_vec<G, VW>(m.C, row * m.ldc + n0, acc, alpha, beta, skip);
+      mm_accumulate_group<VW, kBatMmU, G>(acc, lds.slot.col + first, lds.slot.val + first, m.col,
+                                          m.val, m.B, m.ldb, n0, colok, rs, re, g);
+      if (whole) {
+        __syncthreads();  // the slots' memory is the sums'
+#pragma unroll
+        for (int k = 0; k < VW; ++k) lds.part[threadIdx.x * VW + k] = acc[k].value();
+        __syncthreads();
+        if (grp == 0 && colok) {
+          Comp sum[VW];
+#pragma unroll
+          for (int k = 0; k < VW; ++k) sum[k].init();
+#pragma unroll 1
+          for (int i = 0; i < kGroups; ++i)
+#pragma unroll
+            for (int k = 0; k < VW; ++k) sum[k].add_value(lds.part[(i * G + g) * VW + k]);
+          write_vec<G, VW>(m.C, row * m.ldc + n0, sum, alpha, beta, skip);
+        }
+        __syncthreads();  // the next tile's slots
+      } else if (colok) {
+        write_vec<G, VW>(m.C, row * m.ldc + n0, acc, alpha, beta, skip);
+      }
     }
   }
 }
@@ -211,21 +249,21 @@ __device__ void bat_spmv_dispatch(const BatchMatrix& m, int64_t r0, int64_t r1, 
 
 // The (VW, G) pairs that spmm_tile_shape<4> gives.
 __device__ void bat_spmm_dispatch(const BatchMatrix& m, int64_t r0, int64_t r1, double alpha,
-                                  double beta, int32_t* sc, float* sv) {
+                                  double beta, BatLds& lds) {
   if (m.mm_vw == 4) {
     switch (m.mm_lanes) {
-      case 8: bat_spmm_rows<8, 4>(m, r0, r1, alpha, beta, sc, sv); break;
-      case 16: bat_spmm_rows<16, 4>(m, r0, r1, alpha, beta, sc, sv); break;
-      case 32: bat_spmm_rows<32, 4>(m, r0, r1, alpha, beta, sc, sv); break;
-      default: bat_spmm_rows<64, 4>(m, r0, r1, alpha, beta, sc, sv); break;
+      case 8: bat_spmm_rows<8, 4>(m, r0, r1, alpha, beta, lds); break;
+      case 16: bat_spmm_rows<16, 4>(m, r0, r1, alpha, beta, lds); break;
+      case 32: bat_spmm_rows<32, 4>(m, r0, r1, alpha, beta, lds); break;
+      default: bat_spmm_rows<64, 4>(m, r0, r1, alpha, beta, lds); break;
     }
   } else if (m.mm_vw == 2) {
-    if (m.mm_lanes <= 8) bat_spmm_rows<8, 2>(m, r0, r1, alpha, beta, sc, sv);
-    else bat_spmm_rows<16, 2>(m, r0, r1, alpha, beta, sc, sv);
+    if (m.mm_lanes <= 8) bat_spmm_rows<8, 2>(m, r0, r1, alpha, beta, lds);
+    else bat_spmm_rows<16, 2>(m, r0, r1, alpha, beta, lds);
   } else {
-    if (m.mm_lanes <= 4) bat_spmm_rows<4, 1>(m, r0, r1, alpha, beta, sc, sv);
-    else if (m.mm_lanes <= 8) bat_spmm_rows<8, 1>(m, r0, r1, alpha, beta, sc, sv);
-    else bat_spmm_rows<16, 1>(m, r0, r1, alpha, beta, sc, sv);
+    if (m.mm_lanes <= 4) bat_spmm_rows<4, 1>(m, r0, r1, alpha, beta, lds);
+    else if (m.mm_lanes <= 8) bat_spmm_rows<8, 1>(m, r0, r1, alpha, beta, lds);
+    else bat_spmm_rows<16, 1>(m, r0, r1, alpha, beta, lds);
   }
 }
 
@@ -233,17 +271,16 @@ __global__ __launch_bounds__(kBatBlock) void batched_kernel(const BatchMatrix* _
                                                             const fs_batch_item* __restrict__ items,
                                                             int64_t long_row, double alpha,
                                                             double beta) {
-  __shared__ int32_t slot_col[kBatSlots];
-  __shared__ float slot_val[kBatSlots];
+  __shared__ BatLds lds;
   const fs_batch_item w = items[blockIdx.x];
   const BatchMatrix& m = mats[w.matrix];
   if (w.kind == FS_BATCH_SPMV) {
     if (w.row_end - w.row_begin == 1 && bm_ptr(m, w.row_begin + 1) - bm_ptr(m, w.row_begin) > long_row)
-      bat_spmv_long_row(m, w.row_begin, alpha, beta, slot_val);
+      bat_spmv_long_row(m, w.row_begin, alpha, beta, lds.part);
     else
       bat_spmv_dispatch(m, w.row_begin, w.row_end, alpha, beta);
   } else {
-    bat_spmm_dispatch(m, w.row_begin, w.row_end, alpha, beta, slot_col, slot_val);
+    bat_spmm_dispatch(m, w.row_begin, w.row_end, alpha, beta, lds);
   }
 }
 

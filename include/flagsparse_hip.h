@@ -477,6 +477,7 @@ typedef struct fs_batch_item {
 
 /* Bytes of one packed matrix record; fs_batch_pack writes n_entries records
  * into host memory, which the caller copies to the device. */
+#define FS_BATCH_LONG_MM 512
 int64_t fs_batch_matrix_bytes(void);
 /* Rows of an item that suit its block: of SpMV items with group_lanes lanes a row
  * (n_dense 0), or of SpMM items with n_dense columns. */
@@ -487,7 +488,8 @@ int fs_batch_pack(const fs_batch_entry *entries, int64_t n_entries, void *packed
  * Run every item: y = alpha A x + beta y for SpMV items, C = alpha A B + beta C
  * for SpMM items, one block each.  packed_dev: the packed records in device
  * memory; items: device array.  Single-row SpMV items longer than long_row
- * entries are reduced by a whole block.  queue (two int32 in device memory) and
+ * entries, and single-row SpMM items longer than FS_BATCH_LONG_MM, are reduced
+ * by a whole block.  queue (two int32 in device memory) and
  * grid (at least 1) are left over from blocks that pulled items from a queue:
  * they are checked and not used.
  */
