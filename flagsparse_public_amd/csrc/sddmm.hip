@@ -6,7 +6,8 @@
 // 128 entries, K in BLOCK_K steps, tl.sum reduction).  A row of x or y is cut
 // into parts of 16 bytes, loaded at any alignment; a group of at most 8 lanes
 // takes two entries, lane g parts g, g + 8, ..., and the group reduces with DPP /
-// swizzle exchanges.
+// swizzle exchanges.  fp32 without data keeps a lane for every part up to 32
+// parts: 16 lanes take four entries, 32 lanes eight (sddmm_launch).
 //
 // Why so few lanes: with a lane for every part (up to 64) the exchanges and the
 // address work of an entry, spread over many lanes with little to do, bound the
@@ -18,7 +19,8 @@
 // Widths that 16 bytes do not divide took element loads: fp32 K = 33 / 97, random
 // 92 -> 47 / 122 -> 108 us, banded 172 -> 68 / 229 -> 156 us; fp64 K = 47 158 ->
 // 106 us.  16 lanes above 32 parts: 3-5% faster on random patterns, up to 18%
-// slower on banded ones.
+// slower on banded ones; a lane for every part there: 5-7% faster on 600,000
+// random entries (fp32 K = 200 / 512: 74 / 171 us against 78 / 182).
 #include "fs_host.hpp"
 
 namespace fs {
@@ -82,44 +84,61 @@ __global__ __launch_bounds__(kSdBlock) void sddmm_kernel(
   for (int e = 0; e < E; ++e)
 #pragma unroll
     for (int i = 0; i < kSums; ++i) acc[e][i].init();
-  for (int64_t k0 = 0; k0 < k_dim; k0 += (int64_t)G * VW * NS)
+  if constexpr (NS == 1 && !TAIL && G <= 16) {
+    // a lane for every part: the parts' loads sit under the lane's own bound,
+    // which takes 40 instead of 72 registers in the 16-lane kernel with four
+    // entries (K = 40 / 64, 600,000 random entries: 17.6 -> 16.4 / 20.9 -> 19.9
+    // us); 32 lanes with eight entries are faster below (K = 80 / 96: 29.7 / 31.3
+    // against 32.4 / 33.5)
+    for (int64_t k = (int64_t)g * VW; k < k_dim; k += (int64_t)G * VW)
 #pragma unroll
-    for (int s0 = 0; s0 < NS; s0 += kB) {
-      if (k0 + (int64_t)s0 * G * VW >= k_dim) break;  // uniform
-      V a[kB][E], b[kB][E];
-      bool ok[kB];
-      int skip[kB];
+      for (int e = 0; e < E; ++e) {
+        const V a = *reinterpret_cast<const V*>(xr[e] + k);
+        const V b = *reinterpret_cast<const V*>(yr[e] + k);
 #pragma unroll
-      for (int s = 0; s < kB; ++s) {
-        const int64_t k = k0 + (int64_t)((s0 + s) * G + g) * VW;
-        ok[s] = k < k_dim;
-        skip[s] = TAIL && ok[s] && k + VW > k_dim ? (int)(k + VW - k_dim) : 0;
-        const int64_t at = ok[s] ? k - skip[s] : 0;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          a[s][e] = *reinterpret_cast<const V*>(xr[e] + at);
-          b[s][e] = *reinterpret_cast<const V*>(yr[e] + at);
-        }
+        for (int i = 0; i < VW; ++i)
+          acc[e][0].add_prod((C)sd_elem<VW>(a, i), (C)sd_elem<VW>(b, i));
       }
+  } else {
+    for (int64_t k0 = 0; k0 < k_dim; k0 += (int64_t)G * VW * NS)
 #pragma unroll
-      for (int s = 0; s < kB; ++s) {
-        const int sum = kSums == 1 ? 0 : s0 + s;
-        if (ok[s] && !(TAIL && skip[s])) {
+      for (int s0 = 0; s0 < NS; s0 += kB) {
+        if (k0 + (int64_t)s0 * G * VW >= k_dim) break;  // uniform
+        V a[kB][E], b[kB][E];
+        bool ok[kB];
+        int skip[kB];
 #pragma unroll
-          for (int e = 0; e < E; ++e)
+        for (int s = 0; s < kB; ++s) {
+          const int64_t k = k0 + (int64_t)((s0 + s) * G + g) * VW;
+          ok[s] = k < k_dim;
+          skip[s] = TAIL && ok[s] && k + VW > k_dim ? (int)(k + VW - k_dim) : 0;
+          const int64_t at = ok[s] ? k - skip[s] : 0;
 #pragma unroll
-            for (int i = 0; i < VW; ++i)
-              acc[e][sum].add_prod((C)sd_elem<VW>(a[s][e], i), (C)sd_elem<VW>(b[s][e], i));
-        } else if (TAIL && skip[s]) {
+          for (int e = 0; e < E; ++e) {
+            a[s][e] = *reinterpret_cast<const V*>(xr[e] + at);
+            b[s][e] = *reinterpret_cast<const V*>(yr[e] + at);
+          }
+        }
 #pragma unroll
-          for (int i = 1; i < VW; ++i)
-            if (i >= skip[s])
+        for (int s = 0; s < kB; ++s) {
+          const int sum = kSums == 1 ? 0 : s0 + s;
+          if (ok[s] && !(TAIL && skip[s])) {
 #pragma unroll
-              for (int e = 0; e < E; ++e)
+            for (int e = 0; e < E; ++e)
+#pragma unroll
+              for (int i = 0; i < VW; ++i)
                 acc[e][sum].add_prod((C)sd_elem<VW>(a[s][e], i), (C)sd_elem<VW>(b[s][e], i));
+          } else if (TAIL && skip[s]) {
+#pragma unroll
+            for (int i = 1; i < VW; ++i)
+              if (i >= skip[s])
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+                  acc[e][sum].add_prod((C)sd_elem<VW>(a[s][e], i), (C)sd_elem<VW>(b[s][e], i));
+          }
         }
       }
-    }
+  }
 #pragma unroll
   for (int e = 0; e < E; ++e) {
 #pragma unroll
