@@ -240,15 +240,17 @@ def _validate_x_coo(x, prepared):
     return x.contiguous()
 
 
-def _versions(arrays):
+def _versions(row, col):
     """Counts of in-place writes (tensors made in inference mode have none)."""
-    return [None if t.is_inference() else t._version for t in arrays]
+    if row.is_inference() or col.is_inference():
+        return None
+    return row._version, col._version
 
 
 def _sorted_order(arrays, indptr, stats_dev, stats, chosen):
     """What the native sort found for its sorted (data, row, col): their row
     pointer, the device and host statistics, the chosen variant."""
-    return arrays, _versions(arrays[1:]), indptr, stats_dev, stats, chosen
+    return arrays, _versions(*arrays[1:]), indptr, stats_dev, stats, chosen
 
 
 def _csr_of(prepared):
@@ -257,9 +259,9 @@ def _csr_of(prepared):
     if prepared._csr is None:
         from .spmv_csr import prepare_spmv_csr
         ordered = prepared._ordered  # read once: other threads may be here
-        held = (prepared.data, prepared.row, prepared.col)
-        if (ordered is not None and all(a is b for a, b in zip(ordered[0], held))
-                and ordered[1] == _versions(held[1:])):
+        if (ordered is not None and ordered[0][0] is prepared.data
+                and ordered[0][1] is prepared.row and ordered[0][2] is prepared.col
+                and ordered[1] == _versions(prepared.row, prepared.col)):
             _, _, indptr, *analyzed = ordered
             csr = prepare_spmv_csr(prepared.data, prepared.col, indptr, prepared.shape,
                                    _analyzed=analyzed)
@@ -348,7 +350,7 @@ def flagsparse_spmv_coo(data=None, row=None, col=None, x=None, shape=None, out=N
     if prepared is None:
         if any(a is None for a in (data, row, col, x, shape)):
             raise ValueError("data, row, col, x, shape required when prepared is None")
-        if torch.is_tensor(data):  # the product is not differentiable
+        if torch.is_tensor(data) and data.requires_grad:  # the product is not differentiable
             data = data.detach()
         prepared = prepare_spmv_coo(data, row, col, shape, sort_by_row=sort_by_row, op=op_code,
                                     index_fallback_policy=index_fallback_policy)
