@@ -27,8 +27,9 @@
 // 532 us (with the 64-bit radix sort and its follow-up passes about 2.9 ms).
 //
 // Bucket sizes vary with the sample (gamma distributed, four samples each).
-// A group beyond kCooLargeCap entries, 8 times the mean at the size limit, is
-// reported in *flags, and the caller sorts by other means.
+// A group beyond kCooLargeCap entries, 4 times the mean group (8 times the mean
+// bucket) at the size limit, is reported in *flags, and the caller sorts by
+// other means.
 #include "fs_host.hpp"
 
 namespace fs {
