@@ -204,9 +204,9 @@ def default_spmm_schedule(n_rows: int, nnz: int, n_dense: int, item_bytes: int =
     with 32).  Rows over 256 entries are chunked whatever the mean: a group
     sums a row in one chain per column, a chunk in several chains, which in
     fp32 sums are compensated (fp32, N = 64, values of both signs, rms error of
-    20,000 rows of about 300 entries 7.7e-7 in chunks, 1.8e-6 in chains, of
-    40,000 rows of 600 3.0e-7 and 3.6e-6; the chains took 107 and 379 us, the
-    chunks take 154 and 484).  Wide sums lose nothing in a chain, and where the
+    20,000 rows of about 300 entries 7.6e-7 in chunks, 1.8e-6 in chains, of
+    40,000 rows of 600 2.0e-7 and 3.6e-6; the chains took 107 and 379 us, the
+    chunks take 150 and 464).  Wide sums lose nothing in a chain, and where the
     groups fill the chip they take rows up to 1024 (30,000 rows of 200, N = 256
     in fp32: 518 us, in chunks 795).
 
