@@ -180,8 +180,11 @@ __device__ __forceinline__ f32c add(f32c a, f32c b) {
 }
 // scaling by a power of two (the fp16 row scales) is exact on both parts
 __device__ __forceinline__ f32c scale(f32c a, double s) { return {a.s * (float)s, a.c * (float)s}; }
-// the value a finished sum stands for (other sum types are their own value)
-__device__ __forceinline__ float final_value(f32c a) { return a.s + a.c; }
+// the value a finished sum stands for, an infinite one itself as in Comp (other
+// sum types are their own value)
+__device__ __forceinline__ float final_value(f32c a) {
+  return __builtin_isfinite(a.s) ? a.s + a.c : a.s;
+}
 template <typename T> __device__ __forceinline__ T final_value(T a) { return a; }
 
 // -------------------------------------------------------- lane exchanges
